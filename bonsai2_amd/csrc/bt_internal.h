@@ -12,10 +12,6 @@ namespace bt {
 
 constexpr int kSortErr = 8;   // DevCounters::err bit: a sort pass's look-back wait timed out
 constexpr int kLevels = 32;   // level table slots (reference int2[32], code/Treecode.h:171)
-#ifndef BT_LEVEL_BLOCKS
-#define BT_LEVEL_BLOCKS 2048
-#endif
-constexpr int kLevelBlocks = BT_LEVEL_BLOCKS;  // fixed grid of the per-level tree kernels
 constexpr int kFp64Levels = 4;     // cells at levels <= this combine moments in FP64
 
 struct MlpDev;   // matrix-core operands of the opening-angle network (bt_learn.h)
@@ -48,6 +44,7 @@ constexpr int kLdsStack = 1024;
 struct DevCounters {
   int lvl_start[kLevels + 2];
   int lvl_count[kLevels + 2];
+  int lvl_total[kLevels];   // cells per level as counted ([0]: leaves), before the capacity check
   int nnodes, nleaves, nlevels, ncells;
   int ngroups;
   int flags;   // BT_FLAG_*
@@ -135,8 +132,9 @@ struct Ctx {
   float2 *cq1 = nullptr, *cls = nullptr;
   float4 *cscr = nullptr;      // 6 float4 per cell (bottom-up moments)
   float4 *cwalk = nullptr;     // 3 float4 per cell: walk record (com,M) (3Q) (3Qxz,3Qyz,trQ/2,1.5trQ)
-  int *child_bnd = nullptr;    // 8 ints per parent of the current level
-  int *lvl_blk = nullptr;      // block sums / offsets of the level scan
+  uint4 *cell_raw = nullptr;   // the cells in octant order, before [nodes][leaves] of each parent
+  int *cell_fin = nullptr, *cell_nch = nullptr;  // their final slots and child counts
+  int *cell_cnt = nullptr;     // cells per level and tile of particles, then their prefixes
   int2 *level_beg = nullptr;   // int2[32] (reference d_level_begIdx)
   int2 *root_cells = nullptr;  // per system (first level-1 cell, count)
 
@@ -249,6 +247,8 @@ void launch_bbox(Ctx &c);
 void launch_geo_keys(Ctx &c);
 void launch_gather_tree(Ctx &c);
 void launch_levels(Ctx &c);
+int cell_tiles(int n);   // c.cell_cnt holds kCellCntRows ints per tile
+constexpr int kCellCntRows = 22;
 void launch_multipoles(Ctx &c);
 
 void radix_sort_pairs(Ctx &c, uint64_t *keys, int *vals, uint64_t *keys_tmp, int *vals_tmp,

@@ -77,12 +77,13 @@ void free_particle_arrays(Ctx &c) {
   dev_free(&c.acc); dev_free(&c.groups); dev_free(&c.group_sys); dev_free(&c.gtmp0);
   dev_free(&c.gtmp1); dev_free(&c.gcounts); dev_free(&c.gpot);
   dev_free(&c.box); dev_free(&c.bbox_part); dev_free(&c.root_cells); dev_free(&c.d_off);
-  dev_free(&c.d_energy); dev_free(&c.sys_scale);
+  dev_free(&c.d_energy); dev_free(&c.sys_scale); dev_free(&c.cell_cnt);
 }
 
 void free_cell_arrays(Ctx &c) {
   dev_free(&c.cells); dev_free(&c.csize); dev_free(&c.cmono); dev_free(&c.cq0);
-  dev_free(&c.cq1); dev_free(&c.cls); dev_free(&c.cscr); dev_free(&c.child_bnd);
+  dev_free(&c.cq1); dev_free(&c.cls); dev_free(&c.cscr);
+  dev_free(&c.cell_raw); dev_free(&c.cell_fin); dev_free(&c.cell_nch);
   dev_free(&c.cwalk);
 }
 
@@ -102,7 +103,9 @@ int alloc_cells(Ctx &c, int cap) {
   rc |= dev_alloc(c, &c.cls, n * w);
   rc |= dev_alloc(c, &c.cscr, n * 6 * w);
   rc |= dev_alloc(c, &c.cwalk, n * 3 * w);
-  rc |= dev_alloc(c, &c.child_bnd, (size_t)cap * 8 + 8 * (size_t)c.nsys);
+  rc |= dev_alloc(c, &c.cell_raw, n);
+  rc |= dev_alloc(c, &c.cell_fin, n);
+  rc |= dev_alloc(c, &c.cell_nch, n);
   return rc ? BT_ERR_HIP : 0;
 }
 
@@ -509,7 +512,7 @@ int create_ctx(bt_ctx **out, double eps, double theta, int ncrit, bool fp64) {
   for (int k = 0; k < 12; k++) (void)hipEventCreate(&c.ev[k]);
   if (dev_alloc(c, &c.dc, 1) || dev_alloc(c, &c.level_beg, kLevels) ||
       dev_alloc(c, &c.d_wstats, 4 + 4 * (size_t)kWalkStatBlocks) || dev_alloc(c, &c.d_wpot, 1) ||
-      dev_alloc(c, &c.lvl_blk, kLevelBlocks) || dev_alloc(c, &c.mlp_params, kMlpParams) ||
+      dev_alloc(c, &c.mlp_params, kMlpParams) ||
       dev_alloc(c, &c.mlp_m, kMlpParams) || dev_alloc(c, &c.mlp_v, kMlpParams) ||
       dev_alloc(c, &c.mlp_dev, 1)) {
     delete h;
@@ -564,7 +567,6 @@ int bt_destroy(bt_ctx *h) {
   dev_free(&c.sort_hpart); dev_free(&c.sort_gcount); dev_free(&c.sort_status);
   dev_free(&c.sort_ctr);
   dev_free(&c.scan_blk);
-  dev_free(&c.lvl_blk);
   dev_free(&c.d_direct);
   dev_free(&c.mlp_params); dev_free(&c.mlp_m); dev_free(&c.mlp_v); dev_free(&c.mlp_dev);
   dev_free(&c.d_check); dev_free(&c.d_check_idx);
@@ -712,6 +714,7 @@ int bt_alloc(bt_ctx *h, int n, int nsys, const int *offsets) {
     rc |= dev_alloc(c, &c.gcounts, n); rc |= dev_alloc(c, &c.gpot, n);
     rc |= dev_alloc(c, &c.box, (size_t)nsys * w); rc |= dev_alloc(c, &c.root_cells, nsys);
     rc |= dev_alloc(c, &c.sys_scale, nsys);
+    rc |= dev_alloc(c, &c.cell_cnt, (size_t)kCellCntRows * cell_tiles(n));
     rc |= dev_alloc(c, &c.d_off, nsys + 1);
     rc |= dev_alloc(c, &c.d_energy, 2 * (size_t)nsys * 65);
     if (rc) return BT_ERR_HIP;

@@ -3,7 +3,7 @@
 // The reference builds the octree by recursive dynamic parallelism
 // (code/buildTree.cu:170-584: every split cell's last block launches the
 // children's grid from the device).  HIP has no device-side launch, so the
-// build here is level-synchronous and key-based:
+// build here is key-based:
 //
 //   1. root box per system (code/buildTree.cu:80-166), bit-exact float ops;
 //   2. per particle, its geometric key: the 21 octant digits it takes down the
@@ -11,13 +11,13 @@
 //      (code/Particle4.h:129-148, code/buildTree.cu:233-247);
 //   3. a stable radix sort of the keys = the reference's scatter into child
 //      ranges in octant order (:444-471), within-leaf order canonical;
-//   4. cells, level by level: the children of a level-(L-1) cell are the runs
-//      of equal digit L inside its particle range; count > NLEAF -> node,
-//      0 < count <= NLEAF -> leaf (:394-395); children of one parent are
-//      [nodes in octant order][leaves in octant order] (:393-400, :549) and
-//      levels are contiguous, parents in order (the level sort, :932-951).
-//      Each level is three fixed-size launches (count, scan, emit) whose work
-//      sizes are read on the device, so the whole build can be graph-captured.
+//   4. cells: the children of a level-(L-1) cell are the runs of equal digit L
+//      inside its particle range; count > NLEAF -> node, 0 < count <= NLEAF ->
+//      leaf (:394-395); children of one parent are [nodes in octant order]
+//      [leaves in octant order] (:393-400, :549) and levels are contiguous,
+//      parents in order (the level sort, :932-951).  All levels are found at
+//      once from the sorted keys, in launches whose sizes the host knows, so
+//      the whole build can be graph-captured.
 //
 // Multipoles (code/computeMultipoles.cu:81-190) are computed bottom-up, one
 // launch per level from the deepest: a leaf sums its particles, a node
@@ -27,6 +27,8 @@
 // most the particle extent l and the FP32 sums keep their digits for small
 // cells far from the origin and for sparse cells; levels <= kFp64Levels
 // combine in FP64.  Outputs keep the reference layout (:180-188).
+#include <algorithm>
+
 #include "bt_device.h"
 #include "bt_internal.h"
 
@@ -182,239 +184,339 @@ __global__ __launch_bounds__(kBlock) void k_gather3(int n, const int *__restrict
   }
 }
 
-// ---- level-synchronous cell emission ------------------------------------
+// ---- cell emission: every level from the sorted keys at once ---------------
 //
-// Parents of level L are the cells of level L-1 (the roots for L = 1).  Eight
-// lanes serve one parent; lane o finds the end of child octant o (first index
-// in the parent's range whose digit L exceeds o) by binary search on the
-// sorted keys.  Parents are split into kLevelBlocks contiguous chunks so the
-// block sums give each parent's first child slot in parent order.
+// Which cells exist, and where they begin and end, follows from each particle's
+// neighbours in key order alone, so no level has to wait for the one above it:
+//   * c(i): the octant digits particle i shares with particle i - 1 (0 at a
+//     system's first particle);
+//   * D(i): the deepest node that holds particle i.  A cell holds more than
+//     NLEAF particles iff some window of NLEAF + 1 consecutive particles lies in
+//     it, so D(i) is the maximum of the shared digits of keys[k], keys[k + NLEAF]
+//     over the windows k in [i - NLEAF, i], at most kMaxLevel - 1 (a level-21
+//     cell does not split) and at least 0 (the root always splits,
+//     code/buildTree.cu:702).
+// Particle i begins the cells of levels c(i) + 1 .. D(i) + 1, the last of them a
+// leaf, and ends those of levels c(i) + 1 .. D(i - 1) + 1.  A cell's place in its
+// level is the number of beginnings of that level before it, which is the parent
+// order with the children of a parent in octant order; only [nodes][leaves]
+// within one parent (code/buildTree.cu:393-400, :549) has to be put right after.
+// Five launches for any tree: count the beginnings per tile and level, scan them
+// over the tiles, write the cells in octant order ("raw" slots), order each
+// parent's children, write the cells.  Bound by latency below 2^20 particles and
+// by the traffic on keys (8 B per particle, twice) and cells above.
+// A launch triple per level with binary searches for the children (64 launches)
+// took 0.26 ms at 2^16 and 0.83 ms at 2^24 particles.
+
+constexpr int kCellTile = 1024;                      // particles per block
+constexpr int kCellRounds = kCellTile / kBlock;      // per wave: rounds of 64 in a row
+constexpr int kCellRows = kCellCntRows;                // row 0: leaves; row L: cells of level L
+static_assert(kCellRows == kMaxLevel + 1, "a row per level and one for the leaves");
+constexpr int kMaxLeaf = 64;
+constexpr int kScanBlock = 1024, kScanPer = 4;       // the scan of one row over the tiles
 
 struct LevelArgs {
-  int L, nsys, nleaf, cap_cells, n;
+  int nsys, nleaf, cap_cells, n, ntiles;
   const int *off;
   const uint64_t *keys;
   uint4 *cells;
-  int *bnd;          // 8 ints per parent: end of each child octant
-  int *blk;          // kLevelBlocks block sums -> offsets
+  uint4 *raw;        // octant-order slots: (raw parent | L << 27, first raw child or ~0, begin, end)
+  int *fin;          // final slot of each raw slot
+  int *nch;          // children of each raw node
+  int *cnt;          // kCellRows x ntiles: counts, then their prefixes over the tiles
   int2 *root_cells;
+  int2 *level_beg;
   DevCounters *dc;
 };
 
-__device__ __forceinline__ int level_parent_count(const LevelArgs &a) {
-  return a.L == 1 ? a.nsys : a.dc->lvl_count[a.L - 1];
+// Octant digits two 63-bit keys share.
+__device__ __forceinline__ int shared_digits(uint64_t a, uint64_t b) {
+  const uint64_t x = a ^ b;
+  return x == 0 ? kMaxLevel : (__clzll((long long)x) - 1) / 3;
 }
 
-__device__ __forceinline__ void parent_range(const LevelArgs &a, int p, int &b, int &e,
-                                             bool &splits) {
-  if (a.L == 1) {
-    b = a.off[p];
-    e = a.off[p + 1];
-    splits = e > b;  // the root always splits (code/buildTree.cu:702)
-  } else {
-    const uint4 c = a.cells[a.dc->lvl_start[a.L - 1] + p];
-    b = (int)c.z;
-    e = (int)c.w;
-    splits = !cell_leaf(c);
+// One tile's keys and depths.  Entry j of a window array belongs to particle
+// t0 - 1 - NLEAF + j, entry j of depth to particle t0 - 1 + j.
+struct CellTile {
+  uint64_t key[kCellTile + 2 * kMaxLeaf + 2];
+  int sys[kCellTile + 2 * kMaxLeaf + 2];   // forest: the particle's system
+  unsigned char win[2][kCellTile + kMaxLeaf + 2];
+  unsigned char depth[kCellTile + 2];
+};
+
+// Fills the tile and returns whether one of its windows shares all digits (a
+// level-21 cell of more than NLEAF particles).
+template <bool FOREST>
+__device__ __forceinline__ bool load_cell_tile(const LevelArgs &a, int t0, CellTile &T) {
+  const int nl = a.nleaf;
+  const int k0 = t0 - 1 - nl;   // particle of entry 0
+  for (int j = threadIdx.x; j < kCellTile + 2 * nl + 1; j += kBlock) {
+    const int i = min(max(k0 + j, 0), a.n - 1);
+    T.key[j] = a.keys[i];
+    if (FOREST) T.sys[j] = system_of(i, a.nsys, a.off);
   }
-}
-
-// Per-lane child boundaries of one parent; returns the child count of octant o.
-__device__ __forceinline__ int child_count(const LevelArgs &a, int p, bool active, int o,
-                                           int *end_out) {
-  int b = 0, e = 0;
-  bool splits = false;
-  if (active) parent_range(a, p, b, e, splits);
-  int end = b;
-  if (active && splits) {
-    const int shift = 63 - 3 * a.L;
-    // first index in [b, e) with digit > o
-    int lo = b, hi = e;
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      const int d = (int)((a.keys[mid] >> shift) & 7ull);
-      if (d <= o) lo = mid + 1; else hi = mid;
+  __syncthreads();
+  bool full = false;
+  const int nw = kCellTile + nl + 1;
+  for (int j = threadIdx.x; j < nw; j += kBlock) {
+    const int k = k0 + j;
+    int w = 0;
+    if (k >= 0 && k + nl < a.n && (!FOREST || T.sys[j] == T.sys[j + nl])) {
+      w = shared_digits(T.key[j], T.key[j + nl]);
+      full |= w == kMaxLevel;
+      w = min(w, kMaxLevel - 1);
     }
-    end = lo;
+    T.win[0][j] = (unsigned char)w;
   }
-  const int beg_lane = __shfl_up(end, 1, 8);
-  const int beg = (o == 0) ? b : beg_lane;
-  *end_out = end;
-  return (active && splits) ? end - beg : 0;
-}
-
-__global__ __launch_bounds__(kBlock) void k_level_count(LevelArgs a) {
-  BT_BUILD_PRIO();
-  __shared__ int shw[4];
-  const int np = level_parent_count(a);
-  const int chunk = (np + kLevelBlocks - 1) / kLevelBlocks;
-  const int p0 = blockIdx.x * chunk, p1 = min(np, p0 + chunk);
-  const int o = threadIdx.x & 7;
-  int sum = 0;
-  for (int pb = p0; pb < p1; pb += kBlock / 8) {
-    const int p = pb + (threadIdx.x >> 3);
-    const bool active = p < p1;
-    int end;
-    const int cnt = child_count(a, p, active, o, &end);
-    if (active) a.bnd[8 * p + o] = end;
-    sum += cnt > 0 ? 1 : 0;
-  }
-  sum = wave_sum(sum);
-  if (lane_id() == 0) shw[threadIdx.x >> 6] = sum;
   __syncthreads();
-  if (threadIdx.x == 0) a.blk[blockIdx.x] = shw[0] + shw[1] + shw[2] + shw[3];
+  // maxima over 2, 4, ... consecutive windows; the last power of two within
+  // NLEAF + 1 covers them as two overlapping runs
+  int cur = 0, len = 1;
+  for (; 2 * len <= nl + 1; len *= 2) {
+    for (int j = threadIdx.x; j < nw; j += kBlock)
+      T.win[cur ^ 1][j] = max(T.win[cur][j], j + len < nw ? T.win[cur][j + len] : (unsigned char)0);
+    cur ^= 1;
+    __syncthreads();
+  }
+  for (int j = threadIdx.x; j < kCellTile + 1; j += kBlock)
+    T.depth[j] = max(T.win[cur][j], T.win[cur][j + nl + 1 - len]);
+  __syncthreads();
+  return full;
 }
 
-__global__ __launch_bounds__(kBlock) void k_level_scan(LevelArgs a) {
-  BT_BUILD_PRIO();
-  constexpr int kItems = (kLevelBlocks + kBlock - 1) / kBlock;
-  __shared__ int shw[kBlock / kWave];
-  __shared__ int s_run;
-  // thread t scans block sums [t * kItems, (t + 1) * kItems)
-  int v[kItems];
-  int own = 0;
+// c(i) and D(i) of particle i = t0 + j; an index past the last particle begins
+// nothing (c = kMaxLevel) except that i = n ends what the last particle is in.
+template <bool FOREST>
+__device__ __forceinline__ void cell_span(const LevelArgs &a, const CellTile &T, int t0, int j,
+                                          int &c, int &d, int &dprev) {
+  const int i = t0 + j, e = j + a.nleaf + 1;   // e: entry of particle i in the key array
+  d = i < a.n ? (int)T.depth[j + 1] : -1;
+  dprev = i > 0 && i <= a.n ? (int)T.depth[j] : -1;
+  if (i >= a.n) c = i == a.n ? 0 : kMaxLevel;
+  else if (i == 0 || (FOREST && T.sys[e] != T.sys[e - 1])) c = 0;
+  else c = shared_digits(T.key[e], T.key[e - 1]);
+}
+
+// Lane L of the result counts the beginnings of level L among the wave's
+// kCellRounds * 64 particles, lane 0 its leaves.
+template <bool FOREST>
+__device__ __forceinline__ int wave_cell_counts(const LevelArgs &a, const CellTile &T, int t0) {
+  const int lane = lane_id(), w = threadIdx.x >> 6;
+  int cnt = 0;
 #pragma unroll
-  for (int k = 0; k < kItems; k++) {
-    const int i = threadIdx.x * kItems + k;
-    v[k] = i < kLevelBlocks ? a.blk[i] : 0;
-    own += v[k];
+  for (int r = 0; r < kCellRounds; r++) {
+    int c, d, dp;
+    cell_span<FOREST>(a, T, t0, (w * kCellRounds + r) * kWave + lane, c, d, dp);
+    const int nleaves = __popcll(ballot64(c <= d));   // d >= 0 for every particle
+    cnt += lane == 0 ? nleaves : 0;
+    const int hi = wave_uniform(wave_max_int(d + 1));
+    for (int L = 1; L <= hi; L++) {
+      const int m = __popcll(ballot64(c < L && L <= d + 1));
+      cnt += lane == L ? m : 0;
+    }
   }
-  int incl = wave_incl_scan(own);
-  if (lane_id() == kWave - 1) shw[threadIdx.x >> 6] = incl;
+  return cnt;
+}
+
+template <bool FOREST>
+__global__ __launch_bounds__(kBlock) void k_cells_count(LevelArgs a) {
+  BT_BUILD_PRIO();
+  __shared__ CellTile T;
+  __shared__ int sh[kBlock / kWave][kWave];
+  const int t0 = blockIdx.x * kCellTile;
+  load_cell_tile<FOREST>(a, t0, T);
+  sh[threadIdx.x >> 6][lane_id()] = wave_cell_counts<FOREST>(a, T, t0);
   __syncthreads();
-  int pre = 0;
-  for (int w = 0; w < (int)(threadIdx.x >> 6); w++) pre += shw[w];
-  if (threadIdx.x == kBlock - 1) s_run = pre + incl;
-  int off = pre + incl - own;
-  __syncthreads();
+  if (threadIdx.x < kCellRows) {
+    int s = 0;
+    for (int w = 0; w < kBlock / kWave; w++) s += sh[w][threadIdx.x];
+    a.cnt[threadIdx.x * a.ntiles + blockIdx.x] = s;
+  }
+}
+
+// Block b: exclusive prefix of row b over the tiles, its total in lvl_total[b].
+__global__ __launch_bounds__(kScanBlock) void k_cells_scan(LevelArgs a) {
+  BT_BUILD_PRIO();
+  __shared__ int shw[kScanBlock / kWave];
+  int *row = a.cnt + (size_t)blockIdx.x * a.ntiles;
+  const int w = threadIdx.x >> 6;
+  int carry = 0;
+  for (int b0 = 0; b0 < a.ntiles; b0 += kScanBlock * kScanPer) {
+    int v[kScanPer], own = 0;
+#pragma unroll
+    for (int k = 0; k < kScanPer; k++) {
+      const int i = b0 + threadIdx.x * kScanPer + k;
+      v[k] = i < a.ntiles ? row[i] : 0;
+      own += v[k];
+    }
+    const int incl = wave_incl_scan(own);
+    if (lane_id() == kWave - 1) shw[w] = incl;
+    __syncthreads();
+    int pre = carry, tot = 0;
+    for (int k = 0; k < kScanBlock / kWave; k++) {
+      if (k < w) pre += shw[k];
+      tot += shw[k];
+    }
+    int run = pre + incl - own;
+#pragma unroll
+    for (int k = 0; k < kScanPer; k++) {
+      const int i = b0 + threadIdx.x * kScanPer + k;
+      if (i < a.ntiles) row[i] = run;
+      run += v[k];
+    }
+    carry += tot;
+    __syncthreads();
+  }
   if (threadIdx.x == 0) {
-    const int run = s_run;
-    DevCounters *dc = a.dc;
-    const int start = a.L == 1 ? 0 : dc->lvl_start[a.L - 1] + dc->lvl_count[a.L - 1];
-    int total = run;
-    if (start + total > a.cap_cells) {
-      atomicOr(&dc->err, 1);
-      atomicOr(&dc->err_sticky, 1);
-      total = 0;
+    a.dc->lvl_total[blockIdx.x] = carry;
+    if (blockIdx.x == 0) {
+      a.dc->flags = 0;
+      atomicAnd(&a.dc->err, ~1);   // other bits belong to phases that may run beside this one
     }
-    dc->lvl_start[a.L] = start;
-    dc->lvl_count[a.L] = total;
-    if (total > 0) dc->nlevels = a.L;
-  }
-#pragma unroll
-  for (int k = 0; k < kItems; k++) {
-    const int i = threadIdx.x * kItems + k;
-    if (i < kLevelBlocks) a.blk[i] = off;
-    off += v[k];
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_level_emit(LevelArgs a) {
+// The cells in octant order.  Level L of the loop: a particle that begins a cell
+// of level L takes the next slot of the level; it writes the cell one level up
+// that begins with it as soon as this one's slot, its first child, is known.
+template <bool FOREST>
+__global__ __launch_bounds__(kBlock) void k_cells_emit(LevelArgs a) {
   BT_BUILD_PRIO();
-  __shared__ int shw[4];
-  __shared__ int sh_nodes, sh_leaves;
+  __shared__ CellTile T;
+  __shared__ int sh[kBlock / kWave][kWave];
   DevCounters *dc = a.dc;
-  const int total = dc->lvl_count[a.L];
-  if (total == 0) return;  // nothing at this level (or capacity exceeded)
-  if (threadIdx.x == 0) { sh_nodes = 0; sh_leaves = 0; }
-  const int np = level_parent_count(a);
-  const int chunk = (np + kLevelBlocks - 1) / kLevelBlocks;
-  const int p0 = blockIdx.x * chunk, p1 = min(np, p0 + chunk);
-  const int o = threadIdx.x & 7;
-  const int gsub = (threadIdx.x & 63) >> 3;  // 8-lane group within the wave
-  const int start = dc->lvl_start[a.L];
-  const int pstart = a.L == 1 ? 0 : dc->lvl_start[a.L - 1];
-  int run = a.blk[blockIdx.x];
-  int nodes = 0, leaves = 0, capped = 0;
-  __syncthreads();
-  for (int pb = p0; pb < p1; pb += kBlock / 8) {
-    const int p = pb + (threadIdx.x >> 3);
-    const bool active = p < p1;
-    int b = 0, e = 0;
-    bool splits = false;
-    if (active) parent_range(a, p, b, e, splits);
-    int end = b, beg = b;
-    if (active && splits) {
-      end = a.bnd[8 * p + o];
-      beg = (o == 0) ? b : a.bnd[8 * p + o - 1];
+  const int t0 = blockIdx.x * kCellTile;
+  const int lane = lane_id(), w = threadIdx.x >> 6;
+  const bool full = load_cell_tile<FOREST>(a, t0, T);
+  sh[w][lane] = wave_cell_counts<FOREST>(a, T, t0);
+  // lane L: first slot of level L
+  const int tot = lane >= 1 && lane <= kMaxLevel ? dc->lvl_total[lane] : 0;
+  const int start = wave_incl_scan(tot) - tot;
+  const int total = __shfl(start, kWave - 1, kWave);
+  const bool fits = total <= a.cap_cells;
+  if (blockIdx.x == 0 && w == 0) {
+    const int nleaves = dc->lvl_total[0];
+    const uint64_t filled = ballot64(tot > 0);
+    if (lane < kLevels) {
+      dc->lvl_start[lane] = fits ? start : 0;
+      dc->lvl_count[lane] = fits ? tot : 0;
+      a.level_beg[lane] = fits && tot > 0 ? make_int2(start, start + tot - 1) : make_int2(0, 0);
     }
-    const int cnt = (active && splits) ? end - beg : 0;
-    const bool is_child = cnt > 0;
-    const bool is_node = is_child && cnt > a.nleaf && a.L < kMaxLevel;
-    // 8-bit masks of this parent's children / node children
-    const uint64_t mc = ballot64(is_child), mn = ballot64(is_node);
-    const int sh = gsub * 8;
-    const uint32_t gc = (uint32_t)((mc >> sh) & 0xFFull), gn = (uint32_t)((mn >> sh) & 0xFFull);
-    const int nchild = __popc(gc), nnode = __popc(gn);
-    // exclusive scan of nchild over the parents of this block, in order
-    const int per_parent = (o == 0) ? nchild : 0;
-    const int incl = wave_incl_scan(per_parent);
-    if (lane_id() == 63) shw[threadIdx.x >> 6] = incl;
-    __syncthreads();
-    int wpre = 0;
-    for (int k = 0; k < (threadIdx.x >> 6); k++) wpre += shw[k];
-    const int tot = shw[0] + shw[1] + shw[2] + shw[3];
-    __syncthreads();
-    // value at the group's lane 0 (its exclusive prefix)
-    const int excl_lane0 = __shfl(incl - per_parent, (threadIdx.x & 63) & ~7, kWave);
-    const int first = start + run + wpre + excl_lane0;
-    run += tot;
-    if (is_child) {
-      const uint32_t below = (1u << o) - 1u;
-      const int rank = is_node ? __popc(gn & below) : nnode + __popc((gc & ~gn) & below);
-      const int ci = first + rank;
-      const uint32_t parent_idx = a.L == 1 ? 0u : (uint32_t)(pstart + p);
-      uint4 cell;
-      cell.x = parent_idx | ((uint32_t)a.L << 27);
-      cell.y = is_node ? 0u : 0xFFFFFFFFu;  // node's first/nchild set one level down
-      cell.z = (uint32_t)beg;
-      cell.w = (uint32_t)end;
-      a.cells[ci] = cell;
-      if (is_node) nodes++; else leaves++;
-      if (cnt > a.nleaf && !is_node) capped = 1;
-    }
-    if (active && splits && o == 0) {
-      if (a.L == 1) {
-        a.root_cells[p] = make_int2(first, nchild);
-      } else {
-        a.cells[pstart + p].y = nchild > 0 ? cell_pack_y(first, nchild) : 0xFFFFFFFFu;
+    if (lane == 0) {
+      dc->nlevels = fits ? kWave - 1 - __clzll((long long)filled) : 0;
+      dc->ncells = fits ? total : 0;
+      dc->nnodes = fits ? total - nleaves : 0;
+      dc->nleaves = fits ? nleaves : 0;
+      if (!fits) {
+        atomicOr(&dc->err, 1);
+        atomicOr(&dc->err_sticky, 1);
       }
     }
   }
-  nodes = wave_sum(nodes);
-  leaves = wave_sum(leaves);
-  if (lane_id() == 0) {
-    atomicAdd(&sh_nodes, nodes);
-    atomicAdd(&sh_leaves, leaves);
-  }
-  if (capped) atomicOr(&dc->flags, (int)BT_FLAG_DEPTH_CAP);
+  if (full) atomicOr(&dc->flags, (int)BT_FLAG_DEPTH_CAP);
+  if (!fits) return;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    if (sh_nodes) atomicAdd(&dc->nnodes, sh_nodes);
-    if (sh_leaves) atomicAdd(&dc->nleaves, sh_leaves);
+  // lane L: the next slot of level L for this wave
+  int next = lane >= 1 && lane <= kMaxLevel ? start + a.cnt[lane * a.ntiles + blockIdx.x] : 0;
+  for (int k = 0; k < w; k++) next += lane >= 1 ? sh[k][lane] : 0;
+  for (int r = 0; r < kCellRounds; r++) {
+    const int j = (w * kCellRounds + r) * kWave + lane;
+    const int i = t0 + j;
+    int c, d, dp;
+    cell_span<FOREST>(a, T, t0, j, c, d, dp);
+    const int hi = wave_uniform(wave_max_int(max(d, dp) + 1));
+    uint32_t up = 0;       // raw slot of the cell of level L - 1 that holds this particle
+    int mine = -1;         // raw slot of the node of level L - 1 that begins here
+    uint32_t mine_x = 0;
+    for (int L = 1; L <= hi; L++) {
+      const bool begins = c < L && L <= d + 1;
+      const uint64_t m = ballot64(begins);
+      const int base = __builtin_amdgcn_readlane(next, L);
+      const int slot = base + __popcll(m & lanemask_lt());
+      if (c < L && L <= dp + 1) a.raw[slot - 1].w = (uint32_t)i;   // ends here
+      if (begins) {
+        uint3 *rec;
+        if (mine >= 0) {
+          rec = reinterpret_cast<uint3 *>(a.raw + mine);
+          *rec = make_uint3(mine_x, (uint32_t)slot, (uint32_t)i);
+        }
+        const uint32_t x = up | ((uint32_t)L << 27);
+        if (L == d + 1) {
+          rec = reinterpret_cast<uint3 *>(a.raw + slot);
+          *rec = make_uint3(x, 0xFFFFFFFFu, (uint32_t)i);
+        } else {
+          mine = slot;
+          mine_x = x;
+        }
+        const int e = j + a.nleaf + 1;   // this particle in the tile's arrays
+        if (L == 1 && (i == 0 || (FOREST && T.sys[e] != T.sys[e - 1])))
+          a.root_cells[FOREST ? T.sys[e] : 0] = make_int2(slot, 0);
+      }
+      up = (uint32_t)(begins ? slot : slot - 1);
+      next += lane == L ? __popcll(m) : 0;
+    }
   }
 }
 
-__global__ void k_levels_init(DevCounters *dc) {
-  if (threadIdx.x < kLevels + 2) {
-    dc->lvl_start[threadIdx.x] = 0;
-    dc->lvl_count[threadIdx.x] = 0;
+// Children k < nc of one parent from raw slot f on (their last ends at `end`):
+// bit k of `nodes` is set if child k is a node.
+__device__ __forceinline__ int scan_children(const LevelArgs &a, int f, uint32_t end,
+                                             uint32_t &nodes) {
+  int nc = 0;
+  nodes = 0;
+  for (; nc < 8; nc++) {
+    const uint4 r = a.raw[f + nc];
+    nodes |= (r.y != 0xFFFFFFFFu ? 1u : 0u) << nc;
+    if (r.w == end) return nc + 1;
   }
-  if (threadIdx.x == 0) {
-    dc->nnodes = dc->nleaves = dc->nlevels = dc->ncells = 0;
-    dc->flags = 0;
-    atomicAnd(&dc->err, ~1);   // other bits belong to phases that may run beside this one
+  return nc;
+}
+
+__device__ __forceinline__ void place_children(const LevelArgs &a, int f, int nc, uint32_t nodes) {
+  const int nn = __popc(nodes);
+  for (int k = 0; k < nc; k++) {
+    const int before = __popc(nodes & ((1u << k) - 1u));
+    a.fin[f + k] = f + ((nodes >> k) & 1u ? before : nn + k - before);
   }
 }
 
-__global__ void k_levels_finish(DevCounters *dc, int2 *level_beg) {
-  const int L = threadIdx.x;
-  if (L < kLevels) {
-    const int cnt = (L >= 1 && L <= kMaxLevel) ? dc->lvl_count[L] : 0;
-    level_beg[L] = cnt > 0 ? make_int2(dc->lvl_start[L], dc->lvl_start[L] + cnt - 1)
-                           : make_int2(0, 0);
+// Final slot of every cell: each parent puts its children, which fill a run of
+// slots, into the order [nodes][leaves].
+__global__ __launch_bounds__(kBlock) void k_cells_place(LevelArgs a) {
+  BT_BUILD_PRIO();
+  const int nc_all = a.dc->ncells;
+  const bool failed = a.dc->err & 1;
+  const int stride = gridDim.x * kBlock;
+  for (int s = blockIdx.x * kBlock + threadIdx.x; s < nc_all; s += stride) {
+    const uint4 r = a.raw[s];
+    if (r.y == 0xFFFFFFFFu) continue;
+    uint32_t nodes;
+    const int nc = scan_children(a, (int)r.y, r.w, nodes);
+    place_children(a, (int)r.y, nc, nodes);
+    a.nch[s] = nc;
   }
-  if (L == 0) dc->ncells = dc->nnodes + dc->nleaves;
+  for (int r = blockIdx.x * kBlock + threadIdx.x; r < a.nsys; r += stride) {
+    int2 rc = make_int2(0, 0);
+    if (!failed) {
+      rc.x = a.root_cells[r].x;
+      uint32_t nodes;
+      rc.y = scan_children(a, rc.x, (uint32_t)a.off[r + 1], nodes);
+      place_children(a, rc.x, rc.y, nodes);
+    }
+    a.root_cells[r] = rc;
+  }
+}
+
+__global__ __launch_bounds__(kBlock) void k_cells_finish(LevelArgs a) {
+  BT_BUILD_PRIO();
+  const int nc_all = a.dc->ncells;
+  for (int s = blockIdx.x * kBlock + threadIdx.x; s < nc_all; s += gridDim.x * kBlock) {
+    uint4 r = a.raw[s];
+    const uint32_t L = r.x >> 27;
+    r.x = (L == 1 ? 0u : (uint32_t)a.fin[r.x & 0x07FFFFFFu]) | (L << 27);
+    if (r.y != 0xFFFFFFFFu) r.y = cell_pack_y((int)r.y, a.nch[s]);
+    a.cells[a.fin[s]] = r;
+  }
 }
 
 // ---- bottom-up multipoles -------------------------------------------------
@@ -595,27 +697,34 @@ void launch_gather_tree(Ctx &c) {
   std::swap(c.id, c.id2);
 }
 
+int cell_tiles(int n) { return n / kCellTile + 1; }   // particle n, past the last, included
+
 void launch_levels(Ctx &c) {
-  hipLaunchKernelGGL(k_levels_init, dim3(1), dim3(64), 0, c.stream, c.dc);
   LevelArgs a;
   a.nsys = c.nsys;
   a.nleaf = c.nleaf;
   a.cap_cells = c.cap_cells;
   a.n = c.n;
+  a.ntiles = cell_tiles(c.n);
   a.off = c.d_off;
   a.keys = c.geo_keys;
   a.cells = c.cells;
-  a.bnd = c.child_bnd;
-  a.blk = c.lvl_blk;
+  a.raw = c.cell_raw;
+  a.fin = c.cell_fin;
+  a.nch = c.cell_nch;
+  a.cnt = c.cell_cnt;
   a.root_cells = c.root_cells;
+  a.level_beg = c.level_beg;
   a.dc = c.dc;
-  for (int L = 1; L <= kMaxLevel; L++) {
-    a.L = L;
-    hipLaunchKernelGGL(k_level_count, dim3(kLevelBlocks), dim3(kBlock), 0, c.stream, a);
-    hipLaunchKernelGGL(k_level_scan, dim3(1), dim3(kBlock), 0, c.stream, a);
-    hipLaunchKernelGGL(k_level_emit, dim3(kLevelBlocks), dim3(kBlock), 0, c.stream, a);
-  }
-  hipLaunchKernelGGL(k_levels_finish, dim3(1), dim3(64), 0, c.stream, c.dc, c.level_beg);
+  const dim3 tiles(a.ntiles), cells(grid_for(std::max(c.cap_cells, c.nsys), kBlock, 4096));
+  const bool forest = c.nsys > 1;
+  auto count = forest ? k_cells_count<true> : k_cells_count<false>;
+  auto emit = forest ? k_cells_emit<true> : k_cells_emit<false>;
+  hipLaunchKernelGGL(count, tiles, dim3(kBlock), 0, c.stream, a);
+  hipLaunchKernelGGL(k_cells_scan, dim3(kCellRows), dim3(kScanBlock), 0, c.stream, a);
+  hipLaunchKernelGGL(emit, tiles, dim3(kBlock), 0, c.stream, a);
+  hipLaunchKernelGGL(k_cells_place, cells, dim3(kBlock), 0, c.stream, a);
+  hipLaunchKernelGGL(k_cells_finish, cells, dim3(kBlock), 0, c.stream, a);
 }
 
 namespace {
