@@ -21,6 +21,8 @@
 //     the walk, not LDS or the scalar cache;
 //   * each batch is summed in FP32 and folded into Kahan-compensated
 //     accumulators.
+// Systems of at most 2^17 particles are walked by the four waves of a block per
+// group instead (k_walk_team below).
 // The interaction set equals the reference's (the order of traversal does
 // not change which cells are opened); FP32 sums run in a different order.
 // P2P is code/computeForces.cu:58-78 (20 flops), P2C :83-128 (64 flops),
@@ -58,9 +60,6 @@ constexpr int kMaxWalkSteps = 1 << 20;
 #ifndef BT_LEARN2_WAVES_PER_EU
 #define BT_LEARN2_WAVES_PER_EU 3   // two i-particles per lane: 4 would spill VGPRs
 #endif
-#ifndef BT_XCD_QUEUE
-#define BT_XCD_QUEUE 1
-#endif
 constexpr int kXcd = 8;   // MI355X: 8 XCDs, workgroups dispatched round-robin over them
 // Entries of an FP32 walk's stack held in LDS per wave (kLdsStack = 1024,
 // 4 KiB).  The FP32 walks run at 4 waves per SIMD (their registers allow no
@@ -70,19 +69,28 @@ constexpr int kXcd = 8;   // MI355X: 8 XCDs, workgroups dispatched round-robin o
 // at least the 8 * 64 children one step can push, so a step's pushes always
 // fit after a spill.
 
-// Next group for this wave.  With per-XCD queues the groups (PH order) are cut
-// into kXcd contiguous ranges; a wave drains the range of its own XCD first,
-// so neighbouring groups share that XCD's L2, then helps the other ranges.
-// Every lane joins the atomics (lane 0 adds 1) and all branches are uniform.
+// The groups (PH order) are cut into kXcd contiguous ranges, so neighbouring
+// groups share an XCD's L2: range x.
+__device__ __forceinline__ int xcd_lo(int ngroups, int x) {
+  return (int)((long long)ngroups * x / kXcd);
+}
+// Blocks of the grid on XCD x (workgroups are dispatched round-robin).
+__device__ __forceinline__ int xcd_blocks(int x) {
+  return ((int)gridDim.x - x + kXcd - 1) / kXcd;
+}
+
+// Next group for this wave: each range has a queue, which a wave drains for its
+// own XCD first and then for the others.  Every lane joins the atomics (lane 0
+// adds 1) and all branches are uniform.  (Reading a queue's head before adding
+// to it, or a fixed first group per wave, measured 1-5% slower at 2^24: 26.8 ms
+// as it is, 27.4 and 28.2 ms.)
 __device__ __forceinline__ int next_group(DevCounters *dc, int ngroups, int home, int &xr) {
   const int lane = lane_id();
-  if (!BT_XCD_QUEUE) return wave_uniform(atomicAdd(&dc->queue, lane == 0 ? 1 : 0));
   while (xr < kXcd) {
     const int x = (home + xr) & (kXcd - 1);
-    const int lo = (int)((long long)ngroups * x / kXcd);
-    const int hi = (int)((long long)ngroups * (x + 1) / kXcd);
+    const int lo = xcd_lo(ngroups, x);
     const int k = wave_uniform(atomicAdd(&dc->xq[x], lane == 0 ? 1 : 0));
-    if (lo + k < hi) return lo + k;
+    if (lo + k < xcd_lo(ngroups, x + 1)) return lo + k;
     xr++;
   }
   return ngroups;
@@ -138,10 +146,14 @@ struct IParts {
 constexpr int kJSlots = kWave + 2;
 
 template <typename R>
-struct WaveShared {
+struct Stage {
   V4<R> jA[kJSlots];    // P2C: (com - gc, M)         P2P: (x - gc, m)
   V4<R> jB[kJSlots];    // P2C: (3Qxx, 3Qyy, 3Qzz, 3Qxy)
   V4<R> jC[kJSlots];    // P2C: (3Qxz, 3Qyz, trQ/2, 1.5 trQ)
+};
+
+template <typename R>
+struct WaveShared : Stage<R> {
   int alist[2 * kWave];
   int dlist[2 * kWave];
   int lpre[kWave];
@@ -193,7 +205,7 @@ __device__ __forceinline__ int jslot(int k, int hc) { return IPL == 2 ? k + (k >
 
 // A zero-mass entry far from the group: every term it adds is exactly zero.
 template <typename R>
-__device__ __forceinline__ void stage_pad(WaveShared<R> &S, int slot) {
+__device__ __forceinline__ void stage_pad(Stage<R> &S, int slot) {
   S.jA[slot] = make_v4<R>(R(1.0e18), R(0), R(0), R(0));
   S.jB[slot] = make_v4<R>(R(0), R(0), R(0), R(0));
   S.jC[slot] = make_v4<R>(R(0), R(0), R(0), R(0));
@@ -202,7 +214,7 @@ __device__ __forceinline__ void stage_pad(WaveShared<R> &S, int slot) {
 // Sweeps a staged batch: P2C (QUAD) or particle-like (P2P and monopole-only
 // P2C) interactions of the lane's i-particles with its half of the entries.
 template <bool KAHAN, bool QUAD, typename R, int IPL>
-__device__ __forceinline__ void sweep(const WaveShared<R> &S, int cnt, R eps2,
+__device__ __forceinline__ void sweep(const Stage<R> &S, int cnt, R eps2,
                                       IParts<R, IPL> &ip) {
   const int lane = lane_id();
   Acc4T<R> b[IPL];
@@ -279,12 +291,12 @@ __device__ __forceinline__ void sweep(const WaveShared<R> &S, int cnt, R eps2,
 }
 
 template <bool KAHAN, typename R, int IPL>
-__device__ __forceinline__ void eval_p2c(const WalkArgs<R> &a, WaveShared<R> &S, int cnt, R gcx,
+__device__ __forceinline__ void eval_p2c(const WalkArgs<R> &a, Stage<R> &S, const int *list, int cnt, R gcx,
                                          R gcy, R gcz, IParts<R, IPL> &ip) {
   const int lane = lane_id();
   const int hc = half_count<IPL>(cnt);
   if (lane < cnt) {
-    const int ci = S.alist[lane];
+    const int ci = list[lane];
     const V4<R> r0 = a.cwalk[3 * ci];
     const int d = jslot<IPL>(lane, hc);
     S.jA[d] = make_v4<R>(r0.x - gcx, r0.y - gcy, r0.z - gcz, r0.w);
@@ -299,12 +311,12 @@ __device__ __forceinline__ void eval_p2c(const WalkArgs<R> &a, WaveShared<R> &S,
 }
 
 template <bool KAHAN, typename R, int IPL>
-__device__ __forceinline__ void eval_p2p(const WalkArgs<R> &a, WaveShared<R> &S, int cnt, R gcx,
+__device__ __forceinline__ void eval_p2p(const WalkArgs<R> &a, Stage<R> &S, const int *list, int cnt, R gcx,
                                          R gcy, R gcz, IParts<R, IPL> &ip) {
   const int lane = lane_id();
   const int hc = half_count<IPL>(cnt);
   if (lane < cnt) {
-    const V4<R> p = a.pos_tree[S.dlist[lane]];
+    const V4<R> p = a.pos_tree[list[lane]];
     S.jA[jslot<IPL>(lane, hc)] = make_v4<R>(p.x - gcx, p.y - gcy, p.z - gcz, p.w);
   } else if (IPL == 2 && lane == cnt) {
     stage_pad(S, cnt + 1);
@@ -318,12 +330,12 @@ __device__ __forceinline__ void eval_p2p(const WalkArgs<R> &a, WaveShared<R> &S,
 // code/computeForces.cu:198-225): the cell's mass at its centre of mass,
 // evaluated like a particle (20 flops).
 template <bool KAHAN, typename R, int IPL>
-__device__ __forceinline__ void eval_p2c_mono(const WalkArgs<R> &a, WaveShared<R> &S, int cnt,
+__device__ __forceinline__ void eval_p2c_mono(const WalkArgs<R> &a, Stage<R> &S, const int *list, int cnt,
                                               R gcx, R gcy, R gcz, IParts<R, IPL> &ip) {
   const int lane = lane_id();
   const int hc = half_count<IPL>(cnt);
   if (lane < cnt) {
-    const V4<R> r0 = a.cwalk[3 * S.alist[lane]];
+    const V4<R> r0 = a.cwalk[3 * list[lane]];
     S.jA[jslot<IPL>(lane, hc)] = make_v4<R>(r0.x - gcx, r0.y - gcy, r0.z - gcz, r0.w);
   } else if (IPL == 2 && lane == cnt) {
     stage_pad(S, cnt + 1);
@@ -346,10 +358,10 @@ __device__ __forceinline__ float4 ld_uniform(const cf4v *p, int i) {
 
 // Scalar-load j-data (one i-particle per lane, absolute coordinates).
 template <bool KAHAN>
-__device__ __forceinline__ void eval_p2c_s(const WalkArgs<float> &a, WaveShared<float> &S,
+__device__ __forceinline__ void eval_p2c_s(const WalkArgs<float> &a, const int *list,
                                            int cnt, IParts<float, 1> &ip) {
   const cf4v *rec = (const cf4v *)a.cwalk;
-  const int my = S.alist[lane_id()];
+  const int my = list[lane_id()];
   Acc4 b = {0.f, 0.f, 0.f, 0.f};
   if (cnt == kWave) {
 #pragma unroll BT_UNROLL_S
@@ -370,10 +382,10 @@ __device__ __forceinline__ void eval_p2c_s(const WalkArgs<float> &a, WaveShared<
 }
 
 template <bool KAHAN>
-__device__ __forceinline__ void eval_p2p_s(const WalkArgs<float> &a, WaveShared<float> &S,
+__device__ __forceinline__ void eval_p2p_s(const WalkArgs<float> &a, const int *list,
                                            int cnt, IParts<float, 1> &ip) {
   const cf4v *pj = (const cf4v *)a.pos_tree;
-  const int my = S.dlist[lane_id()];
+  const int my = list[lane_id()];
   Acc4 b = {0.f, 0.f, 0.f, 0.f};
   if (cnt == kWave) {
 #pragma unroll BT_UNROLL_S
@@ -387,21 +399,95 @@ __device__ __forceinline__ void eval_p2p_s(const WalkArgs<float> &a, WaveShared<
   fold<KAHAN>(ip.s[0], ip.c[0], b);
 }
 
-// One batch of cnt P2C (list in S.alist) or P2P (S.dlist) interactions.  The
+// One batch of cnt P2C (list of cells) or P2P (list of particles) interactions.  The
 // LDS path takes i relative to the group centre, the scalar path absolute i.
 template <bool KAHAN, bool SJ, bool MONO, typename R, int IPL>
-__device__ __forceinline__ void batch_p2c(const WalkArgs<R> &a, WaveShared<R> &S, int cnt, R gcx,
+__device__ __forceinline__ void batch_p2c(const WalkArgs<R> &a, Stage<R> &S, const int *list, int cnt, R gcx,
                                           R gcy, R gcz, IParts<R, IPL> &ip) {
-  if constexpr (MONO) eval_p2c_mono<KAHAN, R, IPL>(a, S, cnt, gcx, gcy, gcz, ip);
-  else if constexpr (SJ) eval_p2c_s<KAHAN>(a, S, cnt, ip);
-  else eval_p2c<KAHAN, R, IPL>(a, S, cnt, gcx, gcy, gcz, ip);
+  if constexpr (MONO) eval_p2c_mono<KAHAN, R, IPL>(a, S, list, cnt, gcx, gcy, gcz, ip);
+  else if constexpr (SJ) eval_p2c_s<KAHAN>(a, list, cnt, ip);
+  else eval_p2c<KAHAN, R, IPL>(a, S, list, cnt, gcx, gcy, gcz, ip);
 }
 
 template <bool KAHAN, bool SJ, typename R, int IPL>
-__device__ __forceinline__ void batch_p2p(const WalkArgs<R> &a, WaveShared<R> &S, int cnt, R gcx,
+__device__ __forceinline__ void batch_p2p(const WalkArgs<R> &a, Stage<R> &S, const int *list, int cnt, R gcx,
                                           R gcy, R gcz, IParts<R, IPL> &ip) {
-  if constexpr (SJ) eval_p2p_s<KAHAN>(a, S, cnt, ip);
-  else eval_p2p<KAHAN, R, IPL>(a, S, cnt, gcx, gcy, gcz, ip);
+  if constexpr (SJ) eval_p2p_s<KAHAN>(a, list, cnt, ip);
+  else eval_p2p<KAHAN, R, IPL>(a, S, list, cnt, gcx, gcy, gcz, ip);
+}
+
+// The network's operands of one wave: matrix-core operands in registers, bias
+// and output rows in the block's LDS (64 floats).
+struct Net {
+  half8_t a1, a2_0, a2_1;
+  float b3;
+  const float *s_mlp;
+  // all threads of the block
+  __device__ __forceinline__ void load(const MlpDev *m, float *s) {
+    const int t = threadIdx.x, lane = lane_id();
+    if (t < 32) s[t] = m->c2p[t >> 4][t & 15];
+    else if (t < 64) s[t] = m->w3p[(t - 32) >> 4][t & 15];
+    a1 = m->a1[lane];
+    a2_0 = m->a2[0][lane];
+    a2_1 = m->a2[1][lane];
+    b3 = m->b3;
+    s_mlp = s;
+    __syncthreads();
+  }
+};
+
+// Whether this lane's cell is opened for the group (all lanes of the wave call;
+// `use`: the lane has a cell).  LEARN: by the network's angle for the pair.
+template <typename R, bool LEARN>
+__device__ __forceinline__ bool opens(const WalkArgs<R> &a, bool use, int ci, const uint4 cd,
+                                      const V4<R> cs, R gcx, R gcy, R gcz, R gsx, R gsy, R gsz,
+                                      const GroupGeom &geom, const Net &net) {
+  if constexpr (LEARN) {
+  float2 lsv = make_float2(0.f, 0.f);
+    if (use) lsv = a.cls[ci];
+    // A cell opened even at theta_hi or accepted even at theta_lo is
+    // decided without the network: (l/theta + s)^2 is monotone in 1/theta,
+    // so every angle of the band gives it the same answer.  Only a step
+    // with an undecided cell loads the moments and computes features, and
+    // only a 32-lane block holding one evaluates the network.
+    const float ds2 = box_ds2(cs, gcx, gcy, gcz, gsx, gsy, gsz);
+    float op_lo, op_hi;
+    {
+#pragma clang fp contract(off)
+      op_lo = lsv.x * a.it_max + lsv.y;
+      op_hi = lsv.x * a.it_min + lsv.y;
+      op_lo = op_lo * op_lo;
+      op_hi = op_hi * op_hi;
+    }
+    const bool undecided = use && ds2 < op_lo && ds2 >= op_hi;
+    const uint64_t um = ballot64(undecided);
+    float it = a.it_min;
+    if (um != 0) {
+      // every lane evaluates the network (decided and idle lanes on a zero cell)
+      float4 m = make_float4(0.f, 0.f, 0.f, 0.f), q0 = m;
+      float2 q1 = make_float2(0.f, 0.f);
+      if (undecided) {
+        m = a.cmono[ci];
+        q0 = a.cq0[ci];
+        q1 = a.cq1[ci];
+      }
+      float x[8];
+      pair_features(geom, m, lsv.x, q0, q1, x);
+      const float y = mlp_wave(net.a1, net.a2_0, net.a2_1, net.s_mlp, net.b3, pack_features(x),
+                               (um & 0xFFFFFFFFull) != 0, (um >> 32) != 0);
+      it = learned_inv_theta(y, a.shift, a.it_min, a.it_max);
+    }
+    float op;
+    {
+#pragma clang fp contract(off)
+      op = lsv.x * it + lsv.y;
+      op = op * op;
+    }
+    // the opening test of open_cell with this pair's radius (same ds^2)
+    return use && (ds2 < op || ((int)cd.w - (int)cd.z < 3));
+  } else {
+    return use && (open_cell<R>(cs, gcx, gcy, gcz, gsx, gsy, gsz) || ((int)cd.w - (int)cd.z < 3));
+  }
 }
 
 // LEARN: each popped cell gets its own opening angle from the network
@@ -425,18 +511,8 @@ void k_walk(WalkArgs<R> a) {
   // whole stack is in global memory (stk[0, top))
   int *stk = a.stack + (size_t)(blockIdx.x * kWavesPerBlock + wv) * (size_t)a.stack_ints;
   int *lstk = s_stack + (LSTK ? wv * kLdsStack : 0);
-  half8_t ma1, ma2_0, ma2_1;
-  float mb3 = 0.f;
-  if constexpr (LEARN) {
-    if (threadIdx.x < 32) s_mlp[threadIdx.x] = a.mlp->c2p[threadIdx.x >> 4][threadIdx.x & 15];
-    else if (threadIdx.x < 64)
-      s_mlp[threadIdx.x] = a.mlp->w3p[(threadIdx.x - 32) >> 4][threadIdx.x & 15];
-    ma1 = a.mlp->a1[lane];
-    ma2_0 = a.mlp->a2[0][lane];
-    ma2_1 = a.mlp->a2[1][lane];
-    mb3 = a.mlp->b3;
-    __syncthreads();
-  }
+  Net net;
+  if constexpr (LEARN) net.load(a.mlp, s_mlp);
   if (a.run_if && *a.run_if == 0) return;   // a fallback walk that is not needed
   const int ngroups = a.dc->ngroups;
   // a failed build (cell or group capacity) leaves placeholder links: do not walk it
@@ -536,59 +612,8 @@ void k_walk(WalkArgs<R> a) {
         cd = a.cells[ci];
         cs = a.csize[ci];
       }
-      bool split = false, leaf = false;
-      if constexpr (LEARN) {
-        float2 lsv = make_float2(0.f, 0.f);
-        if (use) lsv = a.cls[ci];
-        // A cell opened even at theta_hi or accepted even at theta_lo is
-        // decided without the network: (l/theta + s)^2 is monotone in 1/theta,
-        // so every angle of the band gives it the same answer.  Only a step
-        // with an undecided cell loads the moments and computes features, and
-        // only a 32-lane block holding one evaluates the network.
-        const float ds2 = box_ds2(cs, gcx, gcy, gcz, gsx, gsy, gsz);
-        float op_lo, op_hi;
-        {
-#pragma clang fp contract(off)
-          op_lo = lsv.x * a.it_max + lsv.y;
-          op_hi = lsv.x * a.it_min + lsv.y;
-          op_lo = op_lo * op_lo;
-          op_hi = op_hi * op_hi;
-        }
-        const bool undecided = use && ds2 < op_lo && ds2 >= op_hi;
-        const uint64_t um = ballot64(undecided);
-        float it = a.it_min;
-        if (um != 0) {
-          // every lane evaluates the network (decided and idle lanes on a zero cell)
-          float4 m = make_float4(0.f, 0.f, 0.f, 0.f), q0 = m;
-          float2 q1 = make_float2(0.f, 0.f);
-          if (undecided) {
-            m = a.cmono[ci];
-            q0 = a.cq0[ci];
-            q1 = a.cq1[ci];
-          }
-          float x[8];
-          pair_features(geom, m, lsv.x, q0, q1, x);
-          const float y = mlp_wave(ma1, ma2_0, ma2_1, s_mlp, mb3, pack_features(x),
-                                   (um & 0xFFFFFFFFull) != 0, (um >> 32) != 0);
-          it = learned_inv_theta(y, a.shift, a.it_min, a.it_max);
-        }
-        float op;
-        {
-#pragma clang fp contract(off)
-          op = lsv.x * it + lsv.y;
-          op = op * op;
-        }
-        if (use) {
-          // the opening test of open_cell with this pair's radius (same ds^2)
-          split = ds2 < op || ((int)cd.w - (int)cd.z < 3);
-          leaf = cell_leaf(cd);
-        }
-      } else {
-        if (use) {
-          split = open_cell<R>(cs, gcx, gcy, gcz, gsx, gsy, gsz) || ((int)cd.w - (int)cd.z < 3);
-          leaf = cell_leaf(cd);
-        }
-      }
+      const bool split = opens<R, LEARN>(a, use, ci, cd, cs, gcx, gcy, gcz, gsx, gsy, gsz, geom, net);
+      const bool leaf = cell_leaf(cd);
       const bool push = use && split && !leaf;
       const bool approx = use && !split;
       const bool direct = use && split && leaf;
@@ -663,7 +688,7 @@ void k_walk(WalkArgs<R> a) {
           nd += min(kWave, ltot - k0);
           wave_lds_sync();
           if (nd >= kWave) {
-            batch_p2p<KAHAN, SJ, R, IPL>(a, S, kWave, gcx, gcy, gcz, ip);
+            batch_p2p<KAHAN, SJ, R, IPL>(a, S, S.dlist, kWave, gcx, gcy, gcz, ip);
             n_dir += kWave;
             nd -= kWave;
             if (lane < nd) S.dlist[lane] = S.dlist[kWave + lane];
@@ -673,7 +698,7 @@ void k_walk(WalkArgs<R> a) {
       }
       wave_lds_sync();
       if (na >= kWave) {
-        batch_p2c<KAHAN, SJ, MONO, R, IPL>(a, S, kWave, gcx, gcy, gcz, ip);
+        batch_p2c<KAHAN, SJ, MONO, R, IPL>(a, S, S.alist, kWave, gcx, gcy, gcz, ip);
         n_app += kWave;
         na -= kWave;
         if (lane < na) S.alist[lane] = S.alist[kWave + lane];
@@ -690,11 +715,11 @@ void k_walk(WalkArgs<R> a) {
       nd = 0;
     }
     if (na > 0) {
-      batch_p2c<KAHAN, SJ, MONO, R, IPL>(a, S, na, gcx, gcy, gcz, ip);
+      batch_p2c<KAHAN, SJ, MONO, R, IPL>(a, S, S.alist, na, gcx, gcy, gcz, ip);
       n_app += na;
     }
     if (nd > 0) {
-      batch_p2p<KAHAN, SJ, R, IPL>(a, S, nd, gcx, gcy, gcz, ip);
+      batch_p2p<KAHAN, SJ, R, IPL>(a, S, S.dlist, nd, gcx, gcy, gcz, ip);
       n_dir += nd;
     }
     // this lane stores particle `idx`; lanes past the end of the group write
@@ -733,6 +758,247 @@ void k_walk(WalkArgs<R> a) {
     a.gpot[g] = gp;
     atomicMax(&a.dc->stack_max, lane == 0 ? deepest : 0);
     atomicMax(&a.dc->stack_hw, lane == 0 ? deepest : 0);
+  }
+}
+
+// ---- team walk ----------------------------------------------------------------
+//
+// With fewer groups than the chip has wave slots, the walk above lasts as long as
+// one wave needs for its whole group: it is bound by that wave's dependent loads
+// and by one wave's issue rate (one VALU instruction in 6-7 cycles, a SIMD takes
+// one in 2.8 from three waves).  Here the T waves of a block walk one group
+// together: a step pops up to 64 T cells from one stack in LDS, wave w lane l
+// testing the (l T + w)-th from the top's start, so siblings go to different
+// waves; children, accepted cells and opened leaves go to shared lists at offsets
+// from the waves' counts, and a list of 64 T entries is evaluated as T batches,
+// one per wave, each lane holding the same i-particle in all waves.  At the end
+// the waves share the rest of both lists out evenly and their compensated sums
+// are added in FP64.  The interaction set is that of the walk above.
+constexpr int kTeam = kWavesPerBlock;
+
+template <typename R>
+struct TeamShared {
+  static constexpr int T = kTeam;
+  static constexpr int W = T * kWave;       // cells a step pops, entries a round evaluates
+  static constexpr int kStack = T * 512;    // holds the 8 W children one step can push
+  Stage<R> stage[T];
+  int stack[kStack];
+  int alist[2 * W], dlist[2 * W];
+  int lpre[W], lbeg[W];
+  int4 tot[T];
+  double sum[T][4][kWave];
+};
+
+// All threads of the block, which all see the same counts: takes the first W
+// entries off a list of cnt >= W.
+template <int W>
+__device__ __forceinline__ void drop_round(int *list, int &cnt) {
+  __syncthreads();   // every wave has read its entries
+  cnt -= W;
+  const int t = threadIdx.x;
+  if (t < cnt) list[t] = list[W + t];
+  __syncthreads();
+}
+
+template <typename R, bool KAHAN, bool LEARN, bool MONO>
+__global__ __launch_bounds__(kBlock) void k_walk_team(WalkArgs<R> a) {
+  typedef TeamShared<R> Sh;
+  constexpr int T = kTeam, W = Sh::W, kStack = Sh::kStack;
+  __shared__ Sh sh;
+  __shared__ float s_mlp[LEARN ? 64 : 1];
+  const int lane = lane_id();
+  const int wv = wave_uniform((int)(threadIdx.x >> 6));
+  const int tid = threadIdx.x;
+  Stage<R> &S = sh.stage[wv];
+  int *spill = a.stack + (size_t)blockIdx.x * T * (size_t)a.stack_ints;
+  const int spill_cap = T * a.stack_ints;
+  Net net;
+  if constexpr (LEARN) net.load(a.mlp, s_mlp);
+  if (a.run_if && *a.run_if == 0) return;
+  const int ngroups = a.dc->ngroups;
+  if (a.dc->err & (3 | kSortErr)) return;
+
+  // the block's groups: a fixed stride over its XCD's range (every branch below
+  // is uniform over the block)
+  const int home = (int)(blockIdx.x % kXcd);
+  const int g_end = xcd_lo(ngroups, home + 1);
+  for (int g = xcd_lo(ngroups, home) + (int)(blockIdx.x / kXcd); g < g_end;
+       g += xcd_blocks(home)) {
+    const int2 grp = a.groups[g];
+    const int pbeg = grp.x, np = max(grp.y, 1);
+    const int sys = a.nsys > 1 ? a.group_sys[g] : 0;
+    const V4<R> pi = a.pos_ph[pbeg + min(lane, np - 1)];
+    const R mnx = wave_min_r(pi.x), mny = wave_min_r(pi.y), mnz = wave_min_r(pi.z);
+    const R mxx = wave_max_r(pi.x), mxy = wave_max_r(pi.y), mxz = wave_max_r(pi.z);
+    R gcx, gcy, gcz, gsx, gsy, gsz;
+    {
+#pragma clang fp contract(off)
+      gcx = R(0.5) * (mxx + mnx); gcy = R(0.5) * (mxy + mny); gcz = R(0.5) * (mxz + mnz);
+      gsx = R(0.5) * (mxx - mnx); gsy = R(0.5) * (mxy - mny); gsz = R(0.5) * (mxz - mnz);
+    }
+    GroupGeom geom;
+    if constexpr (LEARN) geom = make_group_geom(gcx, gcy, gcz, gsx, gsy, gsz, np, a.sys_scale[sys]);
+    IParts<R, 1> ip;
+    ip.x[0] = pi.x - gcx;
+    ip.y[0] = pi.y - gcy;
+    ip.z[0] = pi.z - gcz;
+    ip.s[0] = Acc4T<R>{R(0), R(0), R(0), R(0)};
+    ip.c[0] = Acc4T<R>{R(0), R(0), R(0), R(0)};
+
+    const int2 rc = a.root_cells[sys];
+    if (tid < rc.y) sh.stack[tid] = rc.x + tid;
+    int top = rc.y, gtop = 0;    // entries in LDS, older ones in the spill area
+    int na = 0, nd = 0;          // pending list lengths
+    int n_app = 0, n_dir = 0;    // interactions evaluated (stats)
+    int deepest = top;
+    bool overflow = false;
+    int steps = 0;
+    __syncthreads();
+
+    while (top > 0 || gtop > 0) {
+      if (++steps > kMaxWalkSteps) {
+        overflow = true;
+        break;
+      }
+      if (top < W && gtop > 0) {
+        // the newest spilled entries slide in below the ones left
+        const int r = min(gtop, kStack / 2);
+        const int v = tid < top ? sh.stack[tid] : 0;
+        __syncthreads();
+        if (tid < top) sh.stack[r + tid] = v;
+        for (int k = tid; k < r; k += W) sh.stack[k] = spill[gtop - r + k];
+        gtop -= r;
+        top += r;
+        __syncthreads();
+      }
+      const int take = min(W, top);
+      top -= take;
+      const int e = lane * T + wv;
+      const bool use = e < take;
+      int ci = 0;
+      uint4 cd = make_uint4(0, 0, 0, 0);
+      V4<R> cs = make_v4<R>(R(0), R(0), R(0), R(0));
+      if (use) {
+        ci = sh.stack[top + e];
+        cd = a.cells[ci];
+        cs = a.csize[ci];
+      }
+      const bool split = opens<R, LEARN>(a, use, ci, cd, cs, gcx, gcy, gcz, gsx, gsy, gsz, geom, net);
+      const bool leaf = cell_leaf(cd);
+      const bool push = split && !leaf;
+      const bool approx = use && !split;
+      const bool direct = split && leaf;
+      const int nch = push ? cell_nchild(cd) : 0;
+      const int lsz = direct ? (int)cd.w - (int)cd.z : 0;
+      const int chi = wave_incl_scan(nch);
+      const int li = wave_incl_scan(lsz);
+      const uint64_t am = ballot64(approx), dm = ballot64(direct);
+      // this wave's counts (the same values from its last lane)
+      if (lane == kWave - 1) sh.tot[wv] = make_int4(chi, __popcll(am), __popcll(dm), li);
+      __syncthreads();
+      int4 before = make_int4(0, 0, 0, 0), all = before;
+#pragma unroll
+      for (int w = 0; w < T; w++) {
+        const int4 t = sh.tot[w];
+        if (w < wv) { before.x += t.x; before.y += t.y; before.z += t.z; before.w += t.w; }
+        all.x += t.x; all.y += t.y; all.z += t.z; all.w += t.w;
+      }
+      if (top + all.x > kStack) {
+        // the oldest entries leave for the spill area, a quarter stays free
+        const int sp = min(top, top + all.x - kStack + kStack / 4);
+        if (top - sp + all.x > kStack || gtop + sp > spill_cap) {
+          overflow = true;
+          break;
+        }
+        for (int k = tid; k < sp; k += W) spill[gtop + k] = sh.stack[k];
+        __syncthreads();
+        for (int k0 = 0; k0 < top - sp; k0 += W) {   // each chunk is read before it is written
+          const int k = k0 + tid;
+          const int v = k < top - sp ? sh.stack[sp + k] : 0;
+          __syncthreads();
+          if (k < top - sp) sh.stack[k] = v;
+          __syncthreads();
+        }
+        gtop += sp;
+        top -= sp;
+      }
+      if (push) {
+        const int f = cell_first(cd);
+        const int base = top + before.x + chi - nch;
+        for (int k = 0; k < nch; k++) sh.stack[base + k] = f + k;
+      }
+      if (approx) sh.alist[na + before.y + __popcll(am & lanemask_lt())] = ci;
+      if (direct) {
+        const int r = before.z + __popcll(dm & lanemask_lt());
+        sh.lpre[r] = before.w + li - lsz;
+        sh.lbeg[r] = (int)cd.z;
+      }
+      top += all.x;
+      na += all.y;
+      deepest = max(deepest, top + gtop);
+      __syncthreads();
+      // expand the opened leaves' particle ranges, W at a time
+      for (int k0 = 0; k0 < all.w; k0 += W) {
+        const int k = k0 + tid;
+        if (k < all.w) {
+          int lo = 0, hi = all.z - 1;  // last leaf with lpre <= k
+          while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (sh.lpre[mid] <= k) lo = mid; else hi = mid - 1;
+          }
+          sh.dlist[nd + tid] = sh.lbeg[lo] + (k - sh.lpre[lo]);
+        }
+        nd += min(W, all.w - k0);
+        __syncthreads();
+        if (nd >= W) {
+          batch_p2p<KAHAN, false, R, 1>(a, S, sh.dlist + wv * kWave, kWave, gcx, gcy, gcz, ip);
+          n_dir += W;
+          drop_round<W>(sh.dlist, nd);
+        }
+      }
+      if (na >= W) {
+        batch_p2c<KAHAN, false, MONO, R, 1>(a, S, sh.alist + wv * kWave, kWave, gcx, gcy, gcz, ip);
+        n_app += W;
+        drop_round<W>(sh.alist, na);
+      }
+    }
+    if (overflow) {
+      atomicOr(&a.dc->err, 4);  // every lane, same bit
+      atomicOr(&a.dc->err_sticky, 4);
+      na = 0;
+      nd = 0;
+    }
+    {
+      const int a0 = na * wv / T, a1 = na * (wv + 1) / T;
+      if (a1 > a0)
+        batch_p2c<KAHAN, false, MONO, R, 1>(a, S, sh.alist + a0, a1 - a0, gcx, gcy, gcz, ip);
+      const int d0 = nd * wv / T, d1 = nd * (wv + 1) / T;
+      if (d1 > d0)
+        batch_p2p<KAHAN, false, R, 1>(a, S, sh.dlist + d0, d1 - d0, gcx, gcy, gcz, ip);
+      n_app += na;
+      n_dir += nd;
+    }
+    // the waves' sums, in the order of the waves
+    const Acc4T<R> s = ip.s[0], c = ip.c[0];
+    sh.sum[wv][0][lane] = KAHAN ? (double)s.x - (double)c.x : (double)s.x;
+    sh.sum[wv][1][lane] = KAHAN ? (double)s.y - (double)c.y : (double)s.y;
+    sh.sum[wv][2][lane] = KAHAN ? (double)s.z - (double)c.z : (double)s.z;
+    sh.sum[wv][3][lane] = KAHAN ? (double)s.w - (double)c.w : (double)s.w;
+    __syncthreads();
+    if (wv == 0) {
+      double t[4] = {0.0, 0.0, 0.0, 0.0};
+      for (int w = 0; w < T; w++)
+        for (int q = 0; q < 4; q++) t[q] += sh.sum[w][q][lane];
+      const bool valid = lane < np;
+      const Acc4T<R> res = Acc4T<R>{(R)t[0], (R)t[1], (R)t[2], (R)t[3]};
+      a.acc[valid ? pbeg + lane : a.n + lane] = make_v4<R>(res.x, res.y, res.z, res.w);
+      const double gp = wave_sum(valid ? (double)pi.w * (double)res.w : 0.0);
+      a.gcounts[g] = overflow ? make_int2(-1, -1) : make_int2(n_app, n_dir);
+      a.gpot[g] = gp;
+      atomicMax(&a.dc->stack_max, lane == 0 ? deepest : 0);
+      atomicMax(&a.dc->stack_hw, lane == 0 ? deepest : 0);
+    }
+    __syncthreads();   // the stack and the sums are free for the next group
   }
 }
 
@@ -857,39 +1123,69 @@ WalkArgs<R> walk_args(Ctx &c, const int *run_if) {
   return a;
 }
 
+// Stack entries no walk can exceed: a step pops 64 cells and pushes at most 512,
+// so at most 448 more than it takes stay behind on each of the 21 levels.  A
+// context whose stack may be too small keeps to one wave per group, so that the
+// same calls report BT_ERR_STACK.
+constexpr int kSafeStack = 8 + kMaxLevel * 448;
+
+// Whether the blocks walk groups as teams: below the sizes at which one wave per
+// group fills the chip.  Walk times on Plummer spheres (theta 0.5), one wave per
+// group / teams: 2^10 509 / 45 us, 2^16 753 / 416, 2^18 1187 / 1286; learned angle
+// 2^17 660 / 590, 2^18 868 / 984.  Up to 0.45 ms of the former is its queue: most of
+// its 8192 waves find no group and add to all eight heads; with the groups handed
+// out without a queue it takes 77, 586 and 1283 us.  FP64 (without a queue): 2^14
+// 422 / 282, 2^16 1062 / 779, 2^17 1478 / 1325.  Teams of 2: 215 us at 2^14, of 4:
+// 170, of 8: 185.
+bool walk_as_team(const Ctx &c) {
+  return c.n <= 1 << 17 && c.walk_variant == 0 && c.blocks_per_cu == 0 &&
+         c.lds_stack == kLdsStack && c.stack_ints >= kSafeStack;
+}
+
+// variant 0: LDS j-data, one i-particle per lane; 1: scalar-load j-data, one
+// i-particle per lane; 2: two i-particles per lane, batches split between the
+// half-waves (LDS j-data)
+template <bool KAHAN, bool LEARN, bool MONO>
+auto wave_kernel(int variant) {
+  if constexpr (!MONO) {
+    if (variant == 1) return k_walk<float, KAHAN, true, LEARN, MONO, 1>;
+  }
+  return variant == 2 ? k_walk<float, KAHAN, false, LEARN, MONO, 2>
+                      : k_walk<float, KAHAN, false, LEARN, MONO, 1>;
+}
+
+template <bool KAHAN, bool LEARN, bool MONO>
+auto float_kernel(bool team, int variant) {
+  return team ? k_walk_team<float, KAHAN, LEARN, MONO> : wave_kernel<KAHAN, LEARN, MONO>(variant);
+}
+
+template <bool KAHAN>
+auto float_kernel_of(const Ctx &c, bool team) {
+  if (!c.quadrupole) return float_kernel<KAHAN, false, true>(team, c.walk_variant);
+  if (c.opening == 1 && c.have_mlp) return float_kernel<KAHAN, true, false>(team, c.walk_variant);
+  return float_kernel<KAHAN, false, false>(team, c.walk_variant);
+}
+
+template <bool MONO>
+auto double_kernel(bool team) {
+  return team ? k_walk_team<double, false, false, MONO>
+              : k_walk<double, false, false, false, MONO, 1>;
+}
+
 }  // namespace
 
 void launch_walk(Ctx &c, const int *run_if) {
   c.h_wstats_valid = false;   // d_wstats changes with this walk
+  const bool team = walk_as_team(c);
+  const dim3 blocks(c.walk_blocks), threads(kBlock);
   hipLaunchKernelGGL(k_walk_reset, dim3(1), dim3(64), 0, c.stream, c.dc, run_if);
   if (c.fp64) {
     // Treecode<double>: one i-particle per lane, LDS j-data, FP64 sums
-    const WalkArgs<double> a = walk_args<double>(c, run_if);
-    void (*kern)(WalkArgs<double>) = c.quadrupole ? k_walk<double, false, false, false, false, 1>
-                                                  : k_walk<double, false, false, false, true, 1>;
-    hipLaunchKernelGGL(kern, dim3(c.walk_blocks), dim3(kBlock), 0, c.stream, a);
+    auto kern = c.quadrupole ? double_kernel<false>(team) : double_kernel<true>(team);
+    hipLaunchKernelGGL(kern, blocks, threads, 0, c.stream, walk_args<double>(c, run_if));
   } else {
-    // variant 0: LDS j-data, one i-particle per lane; 1: scalar-load j-data,
-    // one i-particle per lane; 2: two i-particles per lane, batches split
-    // between the half-waves (LDS j-data)
-    const WalkArgs<float> a = walk_args<float>(c, run_if);
-    void (*kern)(WalkArgs<float>);
-    const bool learn = c.opening == 1 && c.have_mlp;
-    const int v = c.walk_variant;
-#define BT_PICK(K, LEARN, MONO)                                                     \
-  (v == 1 ? k_walk<float, K, true, LEARN, MONO, 1>                                  \
-          : v == 2 ? k_walk<float, K, false, LEARN, MONO, 2> : k_walk<float, K, false, LEARN, MONO, 1>)
-    if (!c.quadrupole)
-      kern = c.kahan ? (v == 2 ? k_walk<float, true, false, false, true, 2>
-                               : k_walk<float, true, false, false, true, 1>)
-                     : (v == 2 ? k_walk<float, false, false, false, true, 2>
-                               : k_walk<float, false, false, false, true, 1>);
-    else if (learn)
-      kern = c.kahan ? BT_PICK(true, true, false) : BT_PICK(false, true, false);
-    else
-      kern = c.kahan ? BT_PICK(true, false, false) : BT_PICK(false, false, false);
-#undef BT_PICK
-    hipLaunchKernelGGL(kern, dim3(c.walk_blocks), dim3(kBlock), 0, c.stream, a);
+    auto kern = c.kahan ? float_kernel_of<true>(c, team) : float_kernel_of<false>(c, team);
+    hipLaunchKernelGGL(kern, blocks, threads, 0, c.stream, walk_args<float>(c, run_if));
   }
   WStat *part = reinterpret_cast<WStat *>(c.d_wstats + 4);
   hipLaunchKernelGGL(k_walk_stats_part, dim3(kWalkStatBlocks), dim3(kBlock), 0, c.stream, c.groups,
