@@ -738,9 +738,8 @@ int put_particles(Ctx &c, const void *pos4, const void *vel4, hipMemcpyKind kind
   const size_t bytes = sizeof(float4) * rw(c) * (size_t)c.n;
   BT_CK(hipMemcpyAsync(c.pos, pos4, bytes, kind, c.stream));
   BT_CK(hipMemcpyAsync(c.vel, vel4, bytes, kind, c.stream));
-  std::vector<int> ids(c.n);
-  for (int i = 0; i < c.n; i++) ids[i] = i;
-  BT_CK(hipMemcpyAsync(c.id, ids.data(), sizeof(int) * c.n, hipMemcpyHostToDevice, c.stream));
+  launch_iota(c, c.n, c.id);
+  BT_CK(hipGetLastError());   // (the text of an earlier call's error is no failure here)
   BT_CK(hipStreamSynchronize(c.stream));
   c.have_particles = true;
   c.pending_kick = 0.0;
@@ -940,61 +939,49 @@ int bt_step_f64(bt_ctx *h, double dt, int nleaf, int level_split, int ncrit) {
 
 namespace {
 
+// n values of the context's 4-vector type to the host: as they are, or
+// reordered on the device through idx into tmp, one of the tree-order gather's
+// target arrays (which hold nothing between two builds).
+int read_in_order(Ctx &c, void *host, const void *src, void *tmp, bool as_is, const int *idx,
+                  bool scatter) {
+  const size_t bytes = sizeof(float4) * rw(c) * (size_t)c.n;
+  if (!as_is) {
+    if (join_check(c)) return BT_ERR_HIP;   // a check sum may still read the old particles
+    launch_permute(c, scatter, idx, src, tmp);
+    BT_CK(hipGetLastError());
+    src = tmp;
+  }
+  BT_CK(d2h(c, host, src, bytes));
+  return 0;
+}
+
 // acc (PH order on the device) in the requested order; T = the context's real type
 template <typename T>
 int get_acc_t(Ctx &c, T *acc4, int order) {
-  typedef typename RealVec<T>::v4 V;
   if (check_real<T>(c)) return BT_ERR_STATE;
   if (!c.have_acc) return fail(c, BT_ERR_STATE, "no forces");
   if (order != BT_ORDER_PH && order != BT_ORDER_TREE && order != BT_ORDER_INPUT)
     return fail(c, BT_ERR_ARG, "bad order");
-  std::vector<V> a(c.n);
-  BT_CK(hipMemcpyAsync(a.data(), c.acc, sizeof(V) * c.n, hipMemcpyDeviceToHost, c.stream));
-  V *o = reinterpret_cast<V *>(acc4);
-  if (order == BT_ORDER_PH) {
-    BT_CK(hipStreamSynchronize(c.stream));
-    std::memcpy(o, a.data(), sizeof(V) * c.n);
-    return 0;
-  }
-  std::vector<int> map(c.n);
-  BT_CK(hipMemcpyAsync(map.data(), order == BT_ORDER_TREE ? c.perm : c.id_ph,
-                       sizeof(int) * c.n, hipMemcpyDeviceToHost, c.stream));
-  BT_CK(hipStreamSynchronize(c.stream));
-  for (int k = 0; k < c.n; k++) o[map[k]] = a[k];
-  return 0;
+  return read_in_order(c, acc4, c.acc, c.pos2, order == BT_ORDER_PH,
+                       order == BT_ORDER_TREE ? c.perm : c.id_ph, true);
 }
 
 template <typename T>
 int get_particles_t(Ctx &c, T *pos4, T *vel4, int order) {
-  typedef typename RealVec<T>::v4 V;
   if (check_real<T>(c)) return BT_ERR_STATE;
   if (!c.have_particles) return fail(c, BT_ERR_STATE, "no particles");
   if (order != BT_ORDER_PH && order != BT_ORDER_TREE && order != BT_ORDER_INPUT)
     return fail(c, BT_ERR_ARG, "bad order");
   if (order == BT_ORDER_PH && !c.have_groups)
     return fail(c, BT_ERR_STATE, "no PH order before makeGroups");
-  std::vector<V> p(c.n), v(c.n);
-  std::vector<int> id(c.n), perm;
-  BT_CK(hipMemcpyAsync(p.data(), c.pos, sizeof(V) * c.n, hipMemcpyDeviceToHost, c.stream));
-  BT_CK(hipMemcpyAsync(v.data(), c.vel, sizeof(V) * c.n, hipMemcpyDeviceToHost, c.stream));
-  BT_CK(hipMemcpyAsync(id.data(), c.id, sizeof(int) * c.n, hipMemcpyDeviceToHost, c.stream));
-  if (order == BT_ORDER_PH) {
-    perm.resize(c.n);
-    BT_CK(hipMemcpyAsync(perm.data(), c.perm, sizeof(int) * c.n, hipMemcpyDeviceToHost,
-                         c.stream));
-  }
-  BT_CK(hipStreamSynchronize(c.stream));
-  V *po = reinterpret_cast<V *>(pos4);
-  V *vo = reinterpret_cast<V *>(vel4);
-  for (int k = 0; k < c.n; k++) {
-    // tree order: the arrays as they are; input order: through the ids;
-    // PH order: slot k holds tree particle perm[k]
-    const int src = order == BT_ORDER_PH ? perm[k] : k;
-    const int dst = order == BT_ORDER_INPUT ? id[k] : k;
-    if (po) po[dst] = p[src];
-    if (vo) vo[dst] = v[src];
-  }
-  return 0;
+  // tree order: the arrays as they are; input order: through the ids; PH
+  // order: slot k holds tree particle perm[k]
+  const bool as_is = order == BT_ORDER_TREE, scatter = order == BT_ORDER_INPUT;
+  const int *idx = scatter ? c.id : c.perm;
+  int rc = 0;
+  if (pos4) rc = read_in_order(c, pos4, c.pos, c.pos2, as_is, idx, scatter);
+  if (!rc && vel4) rc = read_in_order(c, vel4, c.vel, c.vel2, as_is, idx, scatter);
+  return rc;
 }
 
 }  // namespace
