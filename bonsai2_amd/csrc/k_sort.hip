@@ -597,6 +597,154 @@ void scan_impl(Ctx &c, const int *in, int *out, int n, int *total_dev) {
                      c.stream, in, n, c.scan_blk, out, nullptr);
 }
 
+// ---- small sorts -------------------------------------------------------------
+// Up to kSmallTiles tiles of 4096 pairs take two launches instead of 32: each tile
+// is sorted in LDS by one block (all digits, the ranking of the passes above), then
+// every pair finds its place: its place in its own tile plus, for every other
+// tile, the number of pairs that go before it, by binary searches that do not
+// depend on each other.  Ties go to the earlier tile, so the sort is stable.  Bound
+// by latency (launches, LDS passes, the search's loads from L2).  Tile sort and
+// merge take 32 + 11 us at 2^16 pairs (30 us in all up to one tile), the 32 launches
+// took 163 us and, at 2^10, 117 us plus the gaps between them.  The searches grow
+// with the square of the number of tiles.
+constexpr int kTileThreads = 1024;
+constexpr int kTileWaves = kTileThreads / kWave;
+constexpr int kTileRounds = kSortTile / kTileThreads;
+constexpr int kSmallTiles = 32;
+
+__global__ __launch_bounds__(kTileThreads) void k_tile_sort(const uint64_t *__restrict__ keys,
+                                                            const int *__restrict__ vals, int n,
+                                                            int key_bits, uint64_t *keys_out,
+                                                            int *vals_out) {
+  BT_BUILD_PRIO();
+  __shared__ uint64_t skeys[kSortTile];
+  __shared__ int svals[kSortTile];
+  __shared__ unsigned short wcnt[kTileWaves][256];
+  __shared__ int sh_wave[4];
+  const int tid = threadIdx.x, lane = lane_id();
+  const int w = wave_uniform(tid >> 6);
+  const int base = blockIdx.x * kSortTile;
+  const int tile_n = min(kSortTile, n - base);
+  // keys have fewer than 64 bits: the pairs past the end, all ones, stay last
+  uint64_t kk[kTileRounds];
+  int vv[kTileRounds];
+#pragma unroll
+  for (int r = 0; r < kTileRounds; r++) {
+    const int j = (w * kTileRounds + r) * kWave + lane;
+    kk[r] = j < tile_n ? keys[base + j] : ~0ull;
+    vv[r] = j < tile_n ? vals[base + j] : 0;
+  }
+  for (int shift = 0; shift < key_bits; shift += 8) {
+    for (int k = tid; k < kTileWaves * 256 / 2; k += kTileThreads)
+      reinterpret_cast<int *>(&wcnt[0][0])[k] = 0;
+    __syncthreads();
+    int dd[kTileRounds], rr[kTileRounds];
+#pragma unroll
+    for (int r = 0; r < kTileRounds; r++) {
+      const int d = (int)(kk[r] >> shift) & 0xFF;
+      uint64_t peers = ~0ull;
+#pragma unroll
+      for (int b = 0; b < 8; b++) {
+        const bool bit = (d >> b) & 1;
+        const uint64_t m = ballot64(bit);
+        peers &= bit ? m : ~m;
+      }
+      const int rank = __popcll(peers & lanemask_lt());
+      const int before = wcnt[w][d];
+      wave_lds_sync();
+      if (rank == 0) wcnt[w][d] = (unsigned short)(before + __popcll(peers));
+      wave_lds_sync();
+      dd[r] = d;
+      rr[r] = before + rank;
+    }
+    __syncthreads();
+    // thread d < 256: digit d's first place, then the waves' pairs in tile order
+    int total = 0, incl = 0;
+    if (tid < 256) {
+#pragma unroll
+      for (int k = 0; k < kTileWaves; k++) total += wcnt[k][tid];
+      incl = wave_incl_scan(total);
+      if (lane == kWave - 1) sh_wave[w] = incl;
+    }
+    __syncthreads();
+    if (tid < 256) {
+      int acc = incl - total;
+      for (int k = 0; k < w; k++) acc += sh_wave[k];
+#pragma unroll
+      for (int k = 0; k < kTileWaves; k++) {
+        const int c = wcnt[k][tid];
+        wcnt[k][tid] = (unsigned short)acc;
+        acc += c;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kTileRounds; r++) {
+      const int pos = wcnt[w][dd[r]] + rr[r];
+      skeys[pos] = kk[r];
+      svals[pos] = vv[r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kTileRounds; r++) {
+      const int j = (w * kTileRounds + r) * kWave + lane;
+      kk[r] = skeys[j];
+      vv[r] = svals[j];
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < kTileRounds; r++) {
+    const int j = (w * kTileRounds + r) * kWave + lane;
+    if (j < tile_n) {
+      keys_out[base + j] = kk[r];
+      vals_out[base + j] = vv[r];
+    }
+  }
+}
+
+// One pair per thread; kTileSearches tiles are searched at a time, so that their
+// loads are in flight together.
+constexpr int kTileSearches = 8;
+
+__global__ __launch_bounds__(256) void k_tile_merge(const uint64_t *__restrict__ keys,
+                                                    const int *__restrict__ vals, int n,
+                                                    uint64_t *__restrict__ keys_out,
+                                                    int *__restrict__ vals_out) {
+  BT_BUILD_PRIO();
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int own = i / kSortTile;   // uniform over the block
+  const int ntiles = (n + kSortTile - 1) / kSortTile;
+  const uint64_t x = keys[i];
+  int place = i - own * kSortTile;
+  for (int t0 = 0; t0 < ntiles; t0 += kTileSearches) {
+    int pos[kTileSearches], len[kTileSearches];
+    const uint64_t *tile[kTileSearches];
+#pragma unroll
+    for (int q = 0; q < kTileSearches; q++) {
+      const int t = t0 + q;
+      tile[q] = keys + (size_t)min(t, ntiles - 1) * kSortTile;
+      len[q] = t < ntiles && t != own ? min(kSortTile, n - t * kSortTile) : 0;
+      pos[q] = 0;
+    }
+#pragma unroll
+    for (int step = kSortTile; step >= 1; step >>= 1) {
+#pragma unroll
+      for (int q = 0; q < kTileSearches; q++) {
+        // pairs of earlier tiles go before an equal key, those of later ones after
+        const int p = pos[q] + step;
+        const uint64_t y = tile[q][max(min(p, len[q]) - 1, 0)];
+        const bool before = t0 + q < own ? y <= x : y < x;
+        if (p <= len[q] && before) pos[q] = p;
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < kTileSearches; q++) place += pos[q];
+  }
+  keys_out[place] = x;
+  vals_out[place] = vals[i];
+}
+
 template <typename T>
 void dev_free_raw(T *&p) {
   if (p) (void)hipFree(p);
@@ -634,6 +782,17 @@ void radix_sort_pairs(Ctx &c, uint64_t *keys, int *vals, uint64_t *keys_tmp, int
                       int n, int key_bits, bool by_system_after) {
   if (n <= 1) return;
   const int nblocks = (n + kSortTile - 1) / kSortTile;
+  // One system, few tiles, whole keys below the all-ones pad
+  if (nblocks <= kSmallTiles && !(by_system_after && c.nsys > 1) && key_bits < 64 &&
+      !c.sort_onesweep) {
+    const bool one = nblocks == 1;
+    hipLaunchKernelGGL(k_tile_sort, dim3(nblocks), dim3(kTileThreads), 0, c.stream, keys, vals, n,
+                       key_bits, one ? keys : keys_tmp, one ? vals : vals_tmp);
+    if (!one)
+      hipLaunchKernelGGL(k_tile_merge, dim3((n + 255) / 256), dim3(256), 0, c.stream, keys_tmp,
+                         vals_tmp, n, keys, vals);
+    return;
+  }
   const int hist_n = 256 * nblocks;
   if (hist_n > c.sort_hist_cap) {
     if (c.sort_hist) (void)hipFree(c.sort_hist);
