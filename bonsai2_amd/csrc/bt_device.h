@@ -40,35 +40,69 @@ __device__ __forceinline__ T wave_bcast(T v, int src) { return __shfl(v, src, kW
 
 __device__ __forceinline__ int wave_uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-__device__ __forceinline__ float wave_min(float v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v = fminf(v, __shfl_xor(v, m, kWave));
-  return v;
-}
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v = fmaxf(v, __shfl_xor(v, m, kWave));
-  return v;
-}
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v) {
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, kWave);
   return v;
 }
+// One step of a wave-wide scan or reduction: the value CTRL moves to this lane
+// (DPP: row_shr:k within rows of 16 lanes, row_bcast:15/31 from the last lane of
+// one row or two rows to the next), `old` in lanes that nothing moves to and in
+// rows outside ROWS.  One VALU operation, where a shuffle goes through the LDS
+// crossbar (about 100 cycles before its result can be used).  All lanes active.
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ int dpp_move(int old, int v) {
+  return __builtin_amdgcn_update_dpp(old, v, CTRL, ROWS, 0xF, false);
+}
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ float dpp_move(float old, float v) {
+  return __builtin_bit_cast(
+      float, dpp_move<CTRL, ROWS>(__builtin_bit_cast(int, old), __builtin_bit_cast(int, v)));
+}
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ double dpp_move(double old, double v) {
+  const long long o = __builtin_bit_cast(long long, old), x = __builtin_bit_cast(long long, v);
+  const unsigned lo = (unsigned)dpp_move<CTRL, ROWS>((int)o, (int)x);
+  const unsigned hi = (unsigned)dpp_move<CTRL, ROWS>((int)(o >> 32), (int)(x >> 32));
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+constexpr int kRowShr = 0x110, kRowBcast15 = 0x142, kRowBcast31 = 0x143;
+
+// Lane 63's value, in every lane.
+__device__ __forceinline__ int last_lane(int v) { return __builtin_amdgcn_readlane(v, kWave - 1); }
+__device__ __forceinline__ float last_lane(float v) {
+  return __builtin_bit_cast(float, last_lane(__builtin_bit_cast(int, v)));
+}
+__device__ __forceinline__ double last_lane(double v) {
+  const long long x = __builtin_bit_cast(long long, v);
+  const unsigned lo = (unsigned)last_lane((int)x), hi = (unsigned)last_lane((int)(x >> 32));
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+// op over the 64 lanes; op(x, x) = x.
+template <typename T, typename Op>
+__device__ __forceinline__ T wave_reduce(T v, Op op) {
+  v = op(v, dpp_move<kRowShr + 1>(v, v));
+  v = op(v, dpp_move<kRowShr + 2>(v, v));
+  v = op(v, dpp_move<kRowShr + 4>(v, v));
+  v = op(v, dpp_move<kRowShr + 8>(v, v));
+  v = op(v, dpp_move<kRowBcast15, 0xA>(v, v));
+  v = op(v, dpp_move<kRowBcast31, 0xC>(v, v));
+  return last_lane(v);
+}
+
 __device__ __forceinline__ int wave_max_int(int v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v = max(v, __shfl_xor(v, m, kWave));
-  return v;
+  return wave_reduce(v, [](int a, int b) { return max(a, b); });
 }
 // Inclusive prefix sum over the 64 lanes.
 __device__ __forceinline__ int wave_incl_scan(int v) {
-  const int l = lane_id();
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    const int t = __shfl_up(v, d, kWave);
-    if (l >= d) v += t;
-  }
+  v += dpp_move<kRowShr + 1>(0, v);
+  v += dpp_move<kRowShr + 2>(0, v);
+  v += dpp_move<kRowShr + 4>(0, v);
+  v += dpp_move<kRowShr + 8>(0, v);
+  v += dpp_move<kRowBcast15, 0xA>(0, v);
+  v += dpp_move<kRowBcast31, 0xC>(0, v);
   return v;
 }
 
@@ -110,15 +144,11 @@ template <>
 __device__ __forceinline__ float rmax(float a, float b) { return fmaxf(a, b); }
 template <typename R>
 __device__ __forceinline__ R wave_min_r(R v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v = rmin(v, __shfl_xor(v, m, kWave));
-  return v;
+  return wave_reduce(v, [](R a, R b) { return rmin<R>(a, b); });
 }
 template <typename R>
 __device__ __forceinline__ R wave_max_r(R v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v = rmax(v, __shfl_xor(v, m, kWave));
-  return v;
+  return wave_reduce(v, [](R a, R b) { return rmax<R>(a, b); });
 }
 
 // System (root) of a particle index: offsets[0..nsys] partition [0, n).

@@ -140,8 +140,8 @@ __device__ __forceinline__ void group_box(const PairArgs &a, int g, int &pbeg, i
   pbeg = grp.x;
   np = max(grp.y, 1);
   pi = a.pos_ph[pbeg + min(lane, np - 1)];
-  const float mnx = wave_min(pi.x), mny = wave_min(pi.y), mnz = wave_min(pi.z);
-  const float mxx = wave_max(pi.x), mxy = wave_max(pi.y), mxz = wave_max(pi.z);
+  const float mnx = wave_min_r(pi.x), mny = wave_min_r(pi.y), mnz = wave_min_r(pi.z);
+  const float mxx = wave_max_r(pi.x), mxy = wave_max_r(pi.y), mxz = wave_max_r(pi.z);
   {
 #pragma clang fp contract(off)
     gcx = 0.5f * (mxx + mnx); gcy = 0.5f * (mxy + mny); gcz = 0.5f * (mxz + mnz);

@@ -309,7 +309,7 @@ __device__ __forceinline__ int wave_cell_counts(const LevelArgs &a, const CellTi
     cell_span<FOREST>(a, T, t0, (w * kCellRounds + r) * kWave + lane, c, d, dp);
     const int nleaves = __popcll(ballot64(c <= d));   // d >= 0 for every particle
     cnt += lane == 0 ? nleaves : 0;
-    const int hi = wave_uniform(wave_max_int(d + 1));
+    const int hi = wave_max_int(d + 1);
     for (int L = 1; L <= hi; L++) {
       const int m = __popcll(ballot64(c < L && L <= d + 1));
       cnt += lane == L ? m : 0;
@@ -392,7 +392,7 @@ __global__ __launch_bounds__(kBlock) void k_cells_emit(LevelArgs a) {
   // lane L: first slot of level L
   const int tot = lane >= 1 && lane <= kMaxLevel ? dc->lvl_total[lane] : 0;
   const int start = wave_incl_scan(tot) - tot;
-  const int total = __shfl(start, kWave - 1, kWave);
+  const int total = last_lane(start);
   const bool fits = total <= a.cap_cells;
   if (blockIdx.x == 0 && w == 0) {
     const int nleaves = dc->lvl_total[0];
@@ -424,7 +424,7 @@ __global__ __launch_bounds__(kBlock) void k_cells_emit(LevelArgs a) {
     const int i = t0 + j;
     int c, d, dp;
     cell_span<FOREST>(a, T, t0, j, c, d, dp);
-    const int hi = wave_uniform(wave_max_int(max(d, dp) + 1));
+    const int hi = wave_max_int(max(d, dp) + 1);
     uint32_t up = 0;       // raw slot of the cell of level L - 1 that holds this particle
     int mine = -1;         // raw slot of the node of level L - 1 that begins here
     uint32_t mine_x = 0;

@@ -621,7 +621,7 @@ void k_walk(WalkArgs<R> a) {
       // children of opened nodes go on the stack
       const int nch = push ? cell_nchild(cd) : 0;
       const int chi = wave_incl_scan(nch);
-      const int ctot = __shfl(chi, kWave - 1, kWave);
+      const int ctot = last_lane(chi);
       if (LSTK && top + ctot > a.lstk_cap) {
         // spill the oldest LDS entries to the global stack, leaving a quarter
         // of the LDS part free after this step's pushes where possible
@@ -668,7 +668,7 @@ void k_walk(WalkArgs<R> a) {
       if (ndl > 0) {
         const int lsz = direct ? (int)cd.w - (int)cd.z : 0;
         const int li = wave_incl_scan(lsz);
-        const int ltot = __shfl(li, kWave - 1, kWave);
+        const int ltot = last_lane(li);
         if (direct) {
           const int r = __popcll(dm & lanemask_lt());
           S.lpre[r] = li - lsz;
@@ -781,12 +781,15 @@ struct TeamShared {
   static constexpr int T = kTeam;
   static constexpr int W = T * kWave;       // cells a step pops, entries a round evaluates
   static constexpr int kStack = T * 512;    // holds the 8 W children one step can push
-  Stage<R> stage[T];
+  union {
+    Stage<R> stage[T];
+    double sum[T][4][kWave];                // after the group's last batch
+  };
   int stack[kStack];
   int alist[2 * W], dlist[2 * W];
   int lpre[W], lbeg[W];
   int4 tot[T];
-  double sum[T][4][kWave];
+  __device__ TeamShared() {}
 };
 
 // All threads of the block, which all see the same counts: takes the first W
@@ -978,6 +981,7 @@ __global__ __launch_bounds__(kBlock) void k_walk_team(WalkArgs<R> a) {
       n_app += na;
       n_dir += nd;
     }
+    __syncthreads();   // every wave is done with its stage
     // the waves' sums, in the order of the waves
     const Acc4T<R> s = ip.s[0], c = ip.c[0];
     sh.sum[wv][0][lane] = KAHAN ? (double)s.x - (double)c.x : (double)s.x;
