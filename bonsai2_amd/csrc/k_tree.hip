@@ -559,13 +559,13 @@ __device__ void write_cell(const MpArgs<T> &a, int c, T rx, T ry, T rz, double M
   a.q0[c] = make_v4<T>((T)qxx, (T)qyy, (T)qzz, (T)qxy);
   a.q1[c] = make_v2<T>((T)qxz, (T)qyz);
   a.ls[c] = make_v2<T>(l, s);
-  // walk record: quadrupole pre-multiplied by 3, trace terms precomputed
+  // walk record (p2c_rec): quadrupole pre-multiplied, trace terms precomputed
   const T fqxx = (T)qxx, fqyy = (T)qyy, fqzz = (T)qzz;
   const T tr = fqxx + fqyy + fqzz;
   a.wrec[3 * (size_t)c] = make_v4<T>(comx, comy, comz, (T)M);
-  a.wrec[3 * (size_t)c + 1] = make_v4<T>(T(3) * fqxx, T(3) * fqyy, T(3) * fqzz, T(3) * (T)qxy);
+  a.wrec[3 * (size_t)c + 1] = make_v4<T>(T(-7.5) * fqxx, T(-7.5) * fqyy, T(-7.5) * fqzz, T(-7.5) * (T)qxy);
   a.wrec[3 * (size_t)c + 2] =
-      make_v4<T>(T(3) * (T)qxz, T(3) * (T)qyz, T(0.5) * tr, T(1.5) * tr);
+      make_v4<T>(T(-7.5) * (T)qxz, T(-7.5) * (T)qyz, tr, T(1.5) * tr);
   V4<T> *s6 = a.scr + 6 * (size_t)c;
   s6[0] = make_v4<T>(rx, ry, rz, (T)M);
   s6[1] = make_v4<T>((T)dx, (T)dy, (T)dz, T(0));

@@ -27,7 +27,7 @@
 // not change which cells are opened); FP32 sums run in a different order.
 // P2P is code/computeForces.cu:58-78 (20 flops), P2C :83-128 (64 flops),
 // rearranged algebraically on a per-cell record with the quadrupole
-// pre-scaled by 3 and the trace terms precomputed (35 VALU instructions).
+// pre-scaled and the trace terms precomputed (34 VALU instructions).
 #include "bt_device.h"
 #include "bt_internal.h"
 #include "bt_interact.h"
@@ -112,7 +112,7 @@ struct WalkArgs {
   const V4<R> *cmono;
   const V4<R> *cq0;
   const V2<R> *cq1;
-  const V4<R> *cwalk;    // 3 per cell: (com, M) (3Qxx,3Qyy,3Qzz,3Qxy) (3Qxz,3Qyz,trQ/2,1.5trQ)
+  const V4<R> *cwalk;    // 3 per cell: (com, M) -7.5(Qxx,Qyy,Qzz,Qxy) (-7.5Qxz,-7.5Qyz,trQ,1.5trQ)
   // learned opening angle (Treecode<float> only)
   const float2 *cls;     // (l, s) per cell
   const float2 *sys_scale;
@@ -148,8 +148,8 @@ constexpr int kJSlots = kWave + 2;
 template <typename R>
 struct Stage {
   V4<R> jA[kJSlots];    // P2C: (com - gc, M)         P2P: (x - gc, m)
-  V4<R> jB[kJSlots];    // P2C: (3Qxx, 3Qyy, 3Qzz, 3Qxy)
-  V4<R> jC[kJSlots];    // P2C: (3Qxz, 3Qyz, trQ/2, 1.5 trQ)
+  V4<R> jB[kJSlots];    // P2C: -7.5 (Qxx, Qyy, Qzz, Qxy)
+  V4<R> jC[kJSlots];    // P2C: (-7.5 Qxz, -7.5 Qyz, trQ, 1.5 trQ)
 };
 
 template <typename R>
@@ -217,9 +217,9 @@ template <bool KAHAN, bool QUAD, typename R, int IPL>
 __device__ __forceinline__ void sweep(const Stage<R> &S, int cnt, R eps2,
                                       IParts<R, IPL> &ip) {
   const int lane = lane_id();
-  Acc4T<R> b[IPL];
+  Acc4T<R> b[IPL], e[IPL];
 #pragma unroll
-  for (int k = 0; k < IPL; k++) b[k] = Acc4T<R>{R(0), R(0), R(0), R(0)};
+  for (int k = 0; k < IPL; k++) b[k] = e[k] = Acc4T<R>{R(0), R(0), R(0), R(0)};
   // One entry's j-data, and its interactions with the lane's i-particles.
   struct J {
     V4<R> A, B, C;
@@ -236,7 +236,8 @@ __device__ __forceinline__ void sweep(const Stage<R> &S, int cnt, R eps2,
   auto eval = [&](const J &j) {
     if (QUAD) {
 #pragma unroll
-      for (int k = 0; k < IPL; k++) p2c_rec(b[k], ip.x[k], ip.y[k], ip.z[k], j.A, j.B, j.C, eps2);
+      for (int k = 0; k < IPL; k++)
+        p2c_rec(b[k], e[k], ip.x[k], ip.y[k], ip.z[k], j.A, j.B, j.C, eps2);
     } else {
 #pragma unroll
       for (int k = 0; k < IPL; k++) p2p(b[k], ip.x[k], ip.y[k], ip.z[k], j.A, eps2);
@@ -287,7 +288,10 @@ __device__ __forceinline__ void sweep(const Stage<R> &S, int cnt, R eps2,
     }
   }
 #pragma unroll
-  for (int k = 0; k < IPL; k++) fold<KAHAN, R>(ip.s[k], ip.c[k], b[k]);
+  for (int k = 0; k < IPL; k++) {
+    if (QUAD) p2c_finish(b[k], e[k]);
+    fold<KAHAN, R>(ip.s[k], ip.c[k], b[k]);
+  }
 }
 
 template <bool KAHAN, typename R, int IPL>
@@ -362,22 +366,23 @@ __device__ __forceinline__ void eval_p2c_s(const WalkArgs<float> &a, const int *
                                            int cnt, IParts<float, 1> &ip) {
   const cf4v *rec = (const cf4v *)a.cwalk;
   const int my = list[lane_id()];
-  Acc4 b = {0.f, 0.f, 0.f, 0.f};
+  Acc4 b = {0.f, 0.f, 0.f, 0.f}, e = b;
   if (cnt == kWave) {
 #pragma unroll BT_UNROLL_S
     for (int j = 0; j < kWave; j++) {
       const int r = 3 * __builtin_amdgcn_readlane(my, j);
-      p2c_rec(b, ip.x[0], ip.y[0], ip.z[0], ld_uniform(rec, r), ld_uniform(rec, r + 1),
+      p2c_rec(b, e, ip.x[0], ip.y[0], ip.z[0], ld_uniform(rec, r), ld_uniform(rec, r + 1),
               ld_uniform(rec, r + 2), a.eps2);
     }
   } else {
 #pragma unroll 2
     for (int j = 0; j < cnt; j++) {
       const int r = 3 * __builtin_amdgcn_readlane(my, j);
-      p2c_rec(b, ip.x[0], ip.y[0], ip.z[0], ld_uniform(rec, r), ld_uniform(rec, r + 1),
+      p2c_rec(b, e, ip.x[0], ip.y[0], ip.z[0], ld_uniform(rec, r), ld_uniform(rec, r + 1),
               ld_uniform(rec, r + 2), a.eps2);
     }
   }
+  p2c_finish(b, e);
   fold<KAHAN>(ip.s[0], ip.c[0], b);
 }
 
