@@ -276,8 +276,12 @@ void launch_learn_errors(Ctx &c, LearnBuffers &L, int npairs);
 void launch_learn_amag(Ctx &c, int ns, const int *d_idx, const double *d_direct, double *amag);
 int mlp_grad_blocks();
 void launch_mlp_grad(Ctx &c, const float *params, int n, const float *feat, const float *target,
-                     int batch, unsigned long long seed, int step, float *partial, double *grad);
-void launch_mlp_adam(Ctx &c, float *p, float *m, float *v, const double *grad, float lr, int step);
+                     int batch, unsigned long long seed, int step, float *partial);
+// the rows of partial summed: grad[kMlpParams] and the loss behind it, or an Adam
+// update with them and the loss alone
+void launch_mlp_reduce(Ctx &c, const float *partial, int batch, double *grad);
+void launch_mlp_adam(Ctx &c, float *p, float *m, float *v, const float *partial, int batch,
+                     double *loss, float lr, int step);
 // targets of the next check, drawn on the device from check_seed and the
 // device's check count: indices into the current particle arrays (c.pos,
 // c.id), and their input ids sorted for launch_check_map

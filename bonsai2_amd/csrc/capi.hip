@@ -1366,7 +1366,8 @@ int bt_mlp_grad(bt_ctx *h, int n, const float *x, const float *t, double *grad, 
   TrainBufs b;
   int rc = upload_samples(c, b, n, x, t, 1);
   if (!rc) {
-    launch_mlp_grad(c, c.mlp_params, n, b.x, b.t, n, 0ull, 0, b.partial, b.grad);
+    launch_mlp_grad(c, c.mlp_params, n, b.x, b.t, n, 0ull, 0, b.partial);
+    launch_mlp_reduce(c, b.partial, n, b.grad);
     std::vector<double> g(kMlpParams + 1);
     if (hipGetLastError() != hipSuccess ||
         hipMemcpyAsync(g.data(), b.grad, sizeof(double) * (kMlpParams + 1), hipMemcpyDeviceToHost,
@@ -1398,11 +1399,9 @@ int bt_mlp_train(bt_ctx *h, int n, const float *x, const float *t, int steps, in
       // cosine decay to lr / 20
       const float lr_k =
           lr * (0.05f + 0.95f * 0.5f * (1.0f + std::cos(3.14159265f * (float)k / (float)steps)));
-      launch_mlp_grad(c, c.mlp_params, n, b.x, b.t, batch, seed, k, b.partial, b.grad);
-      launch_mlp_adam(c, c.mlp_params, c.mlp_m, c.mlp_v, b.grad, lr_k, k + 1);
-      if (hipMemcpyAsync(b.losses + k, b.grad + kMlpParams, sizeof(double),
-                         hipMemcpyDeviceToDevice, c.stream) != hipSuccess)
-        rc = BT_ERR_HIP;
+      launch_mlp_grad(c, c.mlp_params, n, b.x, b.t, batch, seed, k, b.partial);
+      launch_mlp_adam(c, c.mlp_params, c.mlp_m, c.mlp_v, b.partial, batch, b.losses + k, lr_k,
+                      k + 1);
     }
     if (!rc) {
       launch_mlp_prepare(c);

@@ -328,24 +328,41 @@ __device__ __forceinline__ uint64_t mix64(uint64_t z) {
 
 // Partial gradient of L = 1/B sum (y - t)^2 over a minibatch of B samples:
 // sample k of the batch is k itself when B == n, else a hashed draw from
-// [0, n).  Block b writes row b of partial[kGradBlocks][kMlpParams + 1]
-// (the last entry is the block's sum of squared residuals).  The forward
+// [0, n).  The blocks (b, *) write row b of partial[kGradBlocks][kMlpParams + 1]
+// (the last entry is the row's sum of squared residuals).  The forward
 // pass rounds parameters, inputs and the first hidden layer to FP16 as the
 // inference routine does; the backward pass treats the rounding as identity.
-__global__ __launch_bounds__(64) void k_mlp_grad(const float *__restrict__ params, int n,
-                                                 const float *__restrict__ feat,
-                                                 const float *__restrict__ target, int batch,
-                                                 unsigned long long seed, int step,
-                                                 float *__restrict__ partial) {
+//
+// A row takes 64 samples at a time.  Wave p of a block computes hidden units
+// [4p, 4p + 4) of all 64 (lane = sample), passing activations and their gradients
+// through LDS; then each thread sums its gradient entries over the samples.  Two
+// blocks share the entries of a row, so that the 128 rows fill 256 CUs.  Bound by
+// latency: 46 us a batch of 8192 with one wave per row, 12 us like this.
+// Each sum runs over the same terms in the same order as it did there.
+constexpr int kGradWaves = kMlpH / 4;
+constexpr int kGradThreads = kGradWaves * kWave;
+constexpr int kGradSplit = 2;
+constexpr int kGradOwn = (kMlpParams + kGradSplit - 1) / kGradSplit;     // entries per block
+constexpr int kGradPer = (kGradOwn + kGradThreads - 1) / kGradThreads;   // ... per thread
+
+__global__ __launch_bounds__(kGradThreads) void k_mlp_grad(const float *__restrict__ params, int n,
+                                                           const float *__restrict__ feat,
+                                                           const float *__restrict__ target,
+                                                           int batch, unsigned long long seed,
+                                                           int step, float *__restrict__ partial) {
   __shared__ float pr[kMlpParams];
   __shared__ float row[64 * kRow];
   const int t = threadIdx.x;
-  for (int i = t; i < kMlpParams; i += 64) pr[i] = f16r(params[i]);
-  // owned gradient entries: i = t + 64 q
-  int ou[22], ov[22];
-  float acc[22];
-  int nown = 0;
-  for (int i = t; i < kMlpParams; i += 64, nown++) {
+  const int lane = lane_id();
+  const int u0 = 4 * wave_uniform(t >> 6);   // this wave's hidden units
+  for (int i = t; i < kMlpParams; i += kGradThreads) pr[i] = f16r(params[i]);
+  // owned gradient entries
+  const int e0 = (int)blockIdx.y * kGradOwn, e1 = min(kMlpParams, e0 + kGradOwn);
+  int ou[kGradPer], ov[kGradPer];
+  float acc[kGradPer];
+#pragma unroll
+  for (int q = 0; q < kGradPer; q++) {
+    const int i = min(e0 + t + q * kGradThreads, kMlpParams - 1);
     int u, v;
     if (i < kOffB1) { u = kRowDz1 + i / kMlpIn; v = kRowXh + i % kMlpIn; }
     else if (i < kOffW2) { u = kRowDz1 + (i - kOffB1); v = kRowOne; }
@@ -353,16 +370,16 @@ __global__ __launch_bounds__(64) void k_mlp_grad(const float *__restrict__ param
     else if (i < kOffW3) { u = kRowDz2 + (i - kOffB2); v = kRowOne; }
     else if (i < kOffB3) { u = kRowG3; v = kRowA2 + (i - kOffW3); }
     else { u = kRowG3; v = kRowOne; }
-    ou[nown] = u;
-    ov[nown] = v;
-    acc[nown] = 0.f;
+    ou[q] = u;
+    ov[q] = v;
+    acc[q] = 0.f;
   }
   __syncthreads();
   float sq = 0.f;
   const float inv_b = 1.0f / (float)batch;
+  float *r = row + lane * kRow;
   for (int k0 = blockIdx.x * 64; k0 < batch; k0 += gridDim.x * 64) {
-    const int k = k0 + t;
-    float *r = row + t * kRow;
+    const int k = k0 + lane;
     const bool live = k < batch;
     int s = 0;
     if (live) {
@@ -371,72 +388,121 @@ __global__ __launch_bounds__(64) void k_mlp_grad(const float *__restrict__ param
                              (unsigned long long)n);
     }
     float xh[kMlpIn];
-    for (int f = 0; f < kMlpIn; f++) {
-      xh[f] = live ? f16r(feat[8 * (size_t)s + f]) : 0.f;
-      r[kRowXh + f] = xh[f];
+#pragma unroll
+    for (int f = 0; f < kMlpIn; f++) xh[f] = live ? f16r(feat[8 * (size_t)s + f]) : 0.f;
+    const float tgt = live ? target[s] : 0.f;
+    if (u0 == 0) {
+#pragma unroll
+      for (int f = 0; f < kMlpIn; f++) r[kRowXh + f] = xh[f];
     }
-    float z1[kMlpH];
-    for (int h = 0; h < kMlpH; h++) {
+    float z1[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int h = u0 + q;
       float z = pr[kOffB1 + h];
+#pragma unroll
       for (int f = 0; f < kMlpIn; f++) z = fmaf(pr[kOffW1 + h * kMlpIn + f], xh[f], z);
-      z1[h] = z;
+      z1[q] = z;
       r[kRowA1 + h] = f16r(silu_acc(z));
     }
-    float y = pr[kOffB3];
-    for (int h = 0; h < kMlpH; h++) {
-      float z = pr[kOffB2 + h];
-      for (int j = 0; j < kMlpH; j++) z = fmaf(pr[kOffW2 + h * kMlpH + j], r[kRowA1 + j], z);
-      const float a2 = silu_acc(z);
-      r[kRowA2 + h] = a2;
-      r[kRowDz2 + h] = dsilu_acc(z);  // holds silu'(z2) until g3 is known
-      y = fmaf(pr[kOffW3 + h], a2, y);
-    }
-    const float res = live ? y - target[s] : 0.f;
-    sq += res * res;
-    const float g3 = 2.0f * res * inv_b;
-    r[kRowG3] = g3;
-    r[kRowOne] = 1.0f;
-    for (int h = 0; h < kMlpH; h++) r[kRowDz2 + h] *= g3 * pr[kOffW3 + h];
+    __syncthreads();
+    float z2[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) z2[q] = pr[kOffB2 + u0 + q];
+#pragma unroll 8
     for (int j = 0; j < kMlpH; j++) {
-      float da = 0.f;
-      for (int h = 0; h < kMlpH; h++) da = fmaf(r[kRowDz2 + h], pr[kOffW2 + h * kMlpH + j], da);
-      r[kRowDz1 + j] = da * dsilu_acc(z1[j]);
+      const float a1 = r[kRowA1 + j];
+#pragma unroll
+      for (int q = 0; q < 4; q++) z2[q] = fmaf(pr[kOffW2 + (u0 + q) * kMlpH + j], a1, z2[q]);
+    }
+    float ds2[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      r[kRowA2 + u0 + q] = silu_acc(z2[q]);
+      ds2[q] = dsilu_acc(z2[q]);
     }
     __syncthreads();
-    for (int q = 0; q < nown; q++) {
+    float y = pr[kOffB3];
+#pragma unroll 8
+    for (int h = 0; h < kMlpH; h++) y = fmaf(pr[kOffW3 + h], r[kRowA2 + h], y);
+    const float res = live ? y - tgt : 0.f;
+    sq += res * res;
+    const float g3 = 2.0f * res * inv_b;
+    if (u0 == 0) {
+      r[kRowG3] = g3;
+      r[kRowOne] = 1.0f;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) r[kRowDz2 + u0 + q] = ds2[q] * (g3 * pr[kOffW3 + u0 + q]);
+    __syncthreads();
+    float da[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+    for (int h = 0; h < kMlpH; h++) {
+      const float dz2 = r[kRowDz2 + h];
+#pragma unroll
+      for (int q = 0; q < 4; q++) da[q] = fmaf(dz2, pr[kOffW2 + h * kMlpH + u0 + q], da[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) r[kRowDz1 + u0 + q] = da[q] * dsilu_acc(z1[q]);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kGradPer; q++) {
       float sacc = 0.f;
+#pragma unroll 8
       for (int s2 = 0; s2 < 64; s2++) sacc = fmaf(row[s2 * kRow + ou[q]], row[s2 * kRow + ov[q]], sacc);
       acc[q] += sacc;
     }
     __syncthreads();
   }
   float *out = partial + (size_t)blockIdx.x * (kMlpParams + 1);
-  for (int q = 0; q < nown; q++) out[t + 64 * q] = acc[q];
-  const float sqs = wave_sum(sq);
-  if (t == 0) out[kMlpParams] = sqs;
+#pragma unroll
+  for (int q = 0; q < kGradPer; q++) {
+    const int i = e0 + t + q * kGradThreads;
+    if (i < e1) out[i] = acc[q];
+  }
+  if (blockIdx.y == 0 && u0 == 0) {
+    const float sqs = wave_sum(sq);
+    if (t == 0) out[kMlpParams] = sqs;
+  }
 }
 
-// grad[i] = sum over blocks (fixed order) of the partial rows, in FP64.
-__global__ void k_mlp_grad_reduce(const float *__restrict__ partial, int nblocks,
-                                  double *__restrict__ grad, int batch) {
+// The sum of entry i over the rows (fixed order), in FP64; the last entry is the
+// loss.  ADAM: the parameter's update in the same launch; `grad` then receives
+// the loss alone.  Bound by the latency of the rows' loads, 32 of which are in
+// flight: 4 us with the update (one load after the other, and the update and the
+// copy of the loss as steps of their own: 41 us).
+template <bool ADAM>
+__global__ __launch_bounds__(64) void k_mlp_reduce(const float *__restrict__ partial, int nblocks,
+                                                   double *__restrict__ grad, int batch,
+                                                   float *__restrict__ p, float *__restrict__ m,
+                                                   float *__restrict__ v, float lr, float b1,
+                                                   float b2, float eps, float bc1, float bc2) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i > kMlpParams) return;
   double s = 0.0;
-  for (int b = 0; b < nblocks; b++) s += (double)partial[(size_t)b * (kMlpParams + 1) + i];
-  grad[i] = i == kMlpParams ? s / batch : s;   // last entry: the loss
-}
-
-__global__ void k_mlp_adam(float *__restrict__ p, float *__restrict__ m, float *__restrict__ v,
-                           const double *__restrict__ grad, float lr, float b1, float b2,
-                           float eps, float bc1, float bc2) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= kMlpParams) return;
-  const float g = (float)grad[i];
-  const float mi = b1 * m[i] + (1.0f - b1) * g;
-  const float vi = b2 * v[i] + (1.0f - b2) * g * g;
-  m[i] = mi;
-  v[i] = vi;
-  p[i] -= lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
+  constexpr int kAhead = 32;   // rows whose loads are in flight together
+  int b = 0;
+  for (; b + kAhead <= nblocks; b += kAhead) {
+    float x[kAhead];
+#pragma unroll
+    for (int k = 0; k < kAhead; k++) x[k] = partial[(size_t)(b + k) * (kMlpParams + 1) + i];
+#pragma unroll
+    for (int k = 0; k < kAhead; k++) s += (double)x[k];
+  }
+  for (; b < nblocks; b++) s += (double)partial[(size_t)b * (kMlpParams + 1) + i];
+  if (!ADAM) {
+    grad[i] = i == kMlpParams ? s / batch : s;
+  } else if (i == kMlpParams) {
+    *grad = s / batch;
+  } else {
+    const float g = (float)s;
+    // (fused as written, so that the rounding does not depend on the compiler)
+    const float mi = fmaf(b1, m[i], (1.0f - b1) * g);
+    const float vi = fmaf(b2, v[i], (1.0f - b2) * g * g);
+    m[i] = mi;
+    v[i] = vi;
+    p[i] -= lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
+  }
 }
 
 // ---- per-step check of the learned walk -------------------------------------------
@@ -625,19 +691,23 @@ void launch_learn_amag(Ctx &c, int ns, const int *d_idx, const double *d_direct,
 int mlp_grad_blocks() { return kGradBlocks; }
 
 void launch_mlp_grad(Ctx &c, const float *params, int n, const float *feat, const float *target,
-                     int batch, unsigned long long seed, int step, float *partial,
-                     double *grad) {
-  hipLaunchKernelGGL(k_mlp_grad, dim3(kGradBlocks), dim3(64), 0, c.stream, params, n, feat, target,
-                     batch, seed, step, partial);
-  hipLaunchKernelGGL(k_mlp_grad_reduce, dim3((kMlpParams + 1 + 255) / 256), dim3(256), 0,
-                     c.stream, partial, kGradBlocks, grad, batch);
+                     int batch, unsigned long long seed, int step, float *partial) {
+  hipLaunchKernelGGL(k_mlp_grad, dim3(kGradBlocks, kGradSplit), dim3(kGradThreads), 0, c.stream,
+                     params, n, feat, target, batch, seed, step, partial);
 }
 
-void launch_mlp_adam(Ctx &c, float *p, float *m, float *v, const double *grad, float lr, int step) {
+void launch_mlp_reduce(Ctx &c, const float *partial, int batch, double *grad) {
+  hipLaunchKernelGGL(k_mlp_reduce<false>, dim3((kMlpParams + 1 + 63) / 64), dim3(64), 0, c.stream,
+                     partial, kGradBlocks, grad, batch, nullptr, nullptr, nullptr, 0.f, 0.f, 0.f,
+                     0.f, 0.f, 0.f);
+}
+
+void launch_mlp_adam(Ctx &c, float *p, float *m, float *v, const float *partial, int batch,
+                     double *loss, float lr, int step) {
   const float b1 = 0.9f, b2 = 0.999f;
   const float bc1 = 1.0f - powf(b1, (float)step), bc2 = 1.0f - powf(b2, (float)step);
-  hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpParams + 255) / 256), dim3(256), 0, c.stream, p, m, v,
-                     grad, lr, b1, b2, 1e-8f, bc1, bc2);
+  hipLaunchKernelGGL(k_mlp_reduce<true>, dim3((kMlpParams + 1 + 63) / 64), dim3(64), 0, c.stream,
+                     partial, kGradBlocks, loss, batch, p, m, v, lr, b1, b2, 1e-8f, bc1, bc2);
 }
 
 void launch_check_idx(Ctx &c, int ns) {
