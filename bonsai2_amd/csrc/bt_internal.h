@@ -134,6 +134,7 @@ struct Ctx {
   float4 *cwalk = nullptr;     // 3 float4 per cell: walk record (com,M) -7.5(Qxx,Qyy,Qzz,Qxy) (-7.5Qxz,-7.5Qyz,trQ,1.5trQ)
   uint4 *cell_raw = nullptr;   // the cells in octant order, before [nodes][leaves] of each parent
   int *cell_fin = nullptr, *cell_nch = nullptr;  // their final slots and child counts
+  int *cell_arrived = nullptr; // per node: children whose moments are done (0 between launches)
   int *cell_cnt = nullptr;     // cells per level and tile of particles, then their prefixes
   int2 *level_beg = nullptr;   // int2[32] (reference d_level_begIdx)
   int2 *root_cells = nullptr;  // per system (first level-1 cell, count)

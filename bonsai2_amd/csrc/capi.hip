@@ -84,6 +84,7 @@ void free_cell_arrays(Ctx &c) {
   dev_free(&c.cells); dev_free(&c.csize); dev_free(&c.cmono); dev_free(&c.cq0);
   dev_free(&c.cq1); dev_free(&c.cls); dev_free(&c.cscr);
   dev_free(&c.cell_raw); dev_free(&c.cell_fin); dev_free(&c.cell_nch);
+  dev_free(&c.cell_arrived);
   dev_free(&c.cwalk);
 }
 
@@ -106,6 +107,7 @@ int alloc_cells(Ctx &c, int cap) {
   rc |= dev_alloc(c, &c.cell_raw, n);
   rc |= dev_alloc(c, &c.cell_fin, n);
   rc |= dev_alloc(c, &c.cell_nch, n);
+  rc |= dev_alloc(c, &c.cell_arrived, n);
   return rc ? BT_ERR_HIP : 0;
 }
 
@@ -720,7 +722,10 @@ int bt_alloc(bt_ctx *h, int n, int nsys, const int *offsets) {
     if (rc) return BT_ERR_HIP;
     if (alloc_cells(c, n + 1024 * nsys + 64)) return BT_ERR_HIP;
   }
-  c.bbox_blocks = std::max(1, std::min(1024, (c.max_sys_n + 16383) / 16384));
+  // partial boxes of 2048 particles each (at 2^16 particles 5 us, of 16384 20 us),
+  // fewer and larger where many systems make many of them
+  const int part_n = (long long)nsys * ((c.max_sys_n + 2047) / 2048) <= 65536 ? 2048 : 16384;
+  c.bbox_blocks = std::max(1, std::min(1024, (c.max_sys_n + part_n - 1) / part_n));
   if (dev_alloc(c, &c.bbox_part, 2 * (size_t)nsys * c.bbox_blocks * rw(c))) return BT_ERR_HIP;
   BT_CK(hipMemcpy(c.d_off, off.data(), sizeof(int) * (nsys + 1), hipMemcpyHostToDevice));
   c.have_particles = c.have_tree = c.have_mp = c.have_groups = c.have_acc = false;

@@ -19,9 +19,9 @@
 //      once from the sorted keys, in launches whose sizes the host knows, so
 //      the whole build can be graph-captured.
 //
-// Multipoles (code/computeMultipoles.cu:81-190) are computed bottom-up, one
-// launch per level from the deepest: a leaf sums its particles, a node
-// combines its children with the parallel-axis theorem.  Moments are carried
+// Multipoles (code/computeMultipoles.cu:81-190) are computed bottom-up: the
+// leaves sum their particles, then the nodes, from the deepest level, combine
+// their children with the parallel-axis theorem.  Moments are carried
 // relative to a reference point inside the cell's particle bbox (a leaf's
 // first particle; a node's first child's reference), so every offset is at
 // most the particle extent l and the FP32 sums keep their digits for small
@@ -223,6 +223,7 @@ struct LevelArgs {
   uint4 *raw;        // octant-order slots: (raw parent | L << 27, first raw child or ~0, begin, end)
   int *fin;          // final slot of each raw slot
   int *nch;          // children of each raw node
+  int *arrived;      // per node, for the multipoles: 0
   int *cnt;          // kCellRows x ntiles: counts, then their prefixes over the tiles
   int2 *root_cells;
   int2 *level_beg;
@@ -514,8 +515,12 @@ __global__ __launch_bounds__(kBlock) void k_cells_finish(LevelArgs a) {
     uint4 r = a.raw[s];
     const uint32_t L = r.x >> 27;
     r.x = (L == 1 ? 0u : (uint32_t)a.fin[r.x & 0x07FFFFFFu]) | (L << 27);
-    if (r.y != 0xFFFFFFFFu) r.y = cell_pack_y((int)r.y, a.nch[s]);
-    a.cells[a.fin[s]] = r;
+    const int f = a.fin[s];
+    if (r.y != 0xFFFFFFFFu) {
+      r.y = cell_pack_y((int)r.y, a.nch[s]);
+      a.arrived[f] = 0;
+    }
+    a.cells[f] = r;
   }
 }
 
@@ -532,6 +537,7 @@ struct MpArgs {
   V4<T> *size, *mono, *q0;
   V2<T> *q1, *ls;
   V4<T> *wrec;            // 3 per cell, the walk's P2C record
+  int *arrived;           // per node: children whose records are written (zero before)
   const DevCounters *dc;
 };
 
@@ -540,7 +546,37 @@ struct Moments {
   R M, sx, sy, sz, xx, yy, zz, xy, xz, yz;
 };
 
-template <typename T>
+// The scratch record of a cell, which its parent's thread reads.  CLIMB: written
+// and read by threads of one launch, so every access is an agent-scope atomic (it
+// passes the XCD's own L2, which is not coherent with the others').
+template <typename T, bool CLIMB>
+__device__ __forceinline__ void scr_store(V4<T> *p, const V4<T> v) {
+  if constexpr (CLIMB) {
+    const unsigned long long *w = reinterpret_cast<const unsigned long long *>(&v);
+#pragma unroll
+    for (int k = 0; k < (int)(sizeof(v) / 8); k++)
+      __hip_atomic_store(reinterpret_cast<unsigned long long *>(p) + k, w[k], __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+  } else {
+    *p = v;
+  }
+}
+template <typename T, bool CLIMB>
+__device__ __forceinline__ V4<T> scr_load(const V4<T> *p) {
+  if constexpr (CLIMB) {
+    V4<T> v;
+    unsigned long long *w = reinterpret_cast<unsigned long long *>(&v);
+#pragma unroll
+    for (int k = 0; k < (int)(sizeof(v) / 8); k++)
+      w[k] = __hip_atomic_load(reinterpret_cast<const unsigned long long *>(p) + k,
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return v;
+  } else {
+    return *p;
+  }
+}
+
+template <typename T, bool CLIMB>
 __device__ void write_cell(const MpArgs<T> &a, int c, T rx, T ry, T rz, double M, double dx,
                            double dy, double dz, double qxx, double qyy, double qzz, double qxy,
                            double qxz, double qyz, const Ext<T> &e) {
@@ -567,38 +603,48 @@ __device__ void write_cell(const MpArgs<T> &a, int c, T rx, T ry, T rz, double M
   a.wrec[3 * (size_t)c + 2] =
       make_v4<T>(T(-7.5) * (T)qxz, T(-7.5) * (T)qyz, tr, T(1.5) * tr);
   V4<T> *s6 = a.scr + 6 * (size_t)c;
-  s6[0] = make_v4<T>(rx, ry, rz, (T)M);
-  s6[1] = make_v4<T>((T)dx, (T)dy, (T)dz, T(0));
-  s6[2] = make_v4<T>((T)qxx, (T)qyy, (T)qzz, (T)qxy);
-  s6[3] = make_v4<T>((T)qxz, (T)qyz, T(0), T(0));
-  s6[4] = make_v4<T>(e.nx, e.ny, e.nz, T(0));
-  s6[5] = make_v4<T>(e.xx, e.xy, e.xz, T(0));
+  scr_store<T, CLIMB>(s6, make_v4<T>(rx, ry, rz, (T)M));
+  scr_store<T, CLIMB>(s6 + 1, make_v4<T>((T)dx, (T)dy, (T)dz, T(0)));
+  scr_store<T, CLIMB>(s6 + 2, make_v4<T>((T)qxx, (T)qyy, (T)qzz, (T)qxy));
+  scr_store<T, CLIMB>(s6 + 3, make_v4<T>((T)qxz, (T)qyz, T(0), T(0)));
+  scr_store<T, CLIMB>(s6 + 4, make_v4<T>(e.nx, e.ny, e.nz, T(0)));
+  scr_store<T, CLIMB>(s6 + 5, make_v4<T>(e.xx, e.xy, e.xz, T(0)));
 }
 
-template <typename T, typename R>
+template <typename T, typename R, bool CLIMB>
 __device__ void finish_moments(const MpArgs<T> &a, int c, T rx, T ry, T rz, const Moments<R> &m,
                                const Ext<T> &e) {
   if (!(m.M > R(0))) {
-    write_cell<T>(a, c, rx, ry, rz, 0.0, 0, 0, 0, 0, 0, 0, 0, 0, 0, e);
+    write_cell<T, CLIMB>(a, c, rx, ry, rz, 0.0, 0, 0, 0, 0, 0, 0, 0, 0, 0, e);
     return;
   }
   const R im = R(1) / m.M;
   const R dx = m.sx * im, dy = m.sy * im, dz = m.sz * im;
-  write_cell<T>(a, c, rx, ry, rz, (double)m.M, (double)dx, (double)dy, (double)dz,
+  write_cell<T, CLIMB>(a, c, rx, ry, rz, (double)m.M, (double)dx, (double)dy, (double)dz,
                 (double)(m.xx * im - dx * dx), (double)(m.yy * im - dy * dy),
                 (double)(m.zz * im - dz * dz), (double)(m.xy * im - dx * dy),
                 (double)(m.xz * im - dx * dz), (double)(m.yz * im - dy * dz), e);
 }
 
-template <typename T, typename R>
+template <typename T, typename R, bool CLIMB = false>
 __device__ void node_moments(const MpArgs<T> &a, int c, const uint4 cd) {
   Moments<R> m{};
   Ext<T> e = ext_empty<T>();
   const int f = cell_first(cd), nc = cell_nchild(cd);
-  const V4<T> r0 = a.scr[6 * (size_t)f];  // this node's reference = first child's
-  for (int k = 0; k < nc; k++) {
+  // a child's six vectors are loaded while the one before it is added
+  struct Child {
+    V4<T> g, d, qa, qb, bmn, bmx;
+  };
+  auto load = [&](int k) {
     const V4<T> *s6 = a.scr + 6 * (size_t)(f + k);
-    const V4<T> g = s6[0], d = s6[1], qa = s6[2], qb = s6[3], bmn = s6[4], bmx = s6[5];
+    return Child{scr_load<T, CLIMB>(s6),     scr_load<T, CLIMB>(s6 + 1), scr_load<T, CLIMB>(s6 + 2),
+                 scr_load<T, CLIMB>(s6 + 3), scr_load<T, CLIMB>(s6 + 4), scr_load<T, CLIMB>(s6 + 5)};
+  };
+  Child cur = load(0);
+  const V4<T> r0 = cur.g;   // this node's reference = first child's
+  for (int k = 0; k < nc; k++) {
+    const Child nxt = load(min(k + 1, nc - 1));
+    const V4<T> g = cur.g, d = cur.d, qa = cur.qa, qb = cur.qb, bmn = cur.bmn, bmx = cur.bmx;
     // child com relative to this node's reference: both references lie in the
     // node's bbox, so their difference is at most l and (near-)exact in T
     const R ox = R(g.x - r0.x) + R(d.x), oy = R(g.y - r0.y) + R(d.y),
@@ -610,48 +656,89 @@ __device__ void node_moments(const MpArgs<T> &a, int c, const uint4 cd) {
     m.zz += Mc * (R(qa.z) + oz * oz); m.xy += Mc * (R(qa.w) + ox * oy);
     m.xz += Mc * (R(qb.x) + ox * oz); m.yz += Mc * (R(qb.y) + oy * oz);
     ext_merge(e, bmn.x, bmn.y, bmn.z, bmx.x, bmx.y, bmx.z);
+    cur = nxt;
   }
-  finish_moments<T, R>(a, c, r0.x, r0.y, r0.z, m, e);
+  finish_moments<T, R, CLIMB>(a, c, r0.x, r0.y, r0.z, m, e);
 }
 
 // Treecode<float>: leaves sum in FP32, nodes combine in FP32 below level
 // kFp64Levels and in FP64 at and above it.  Treecode<double>: FP64 throughout.
+template <typename T, bool CLIMB = false>
+__device__ __forceinline__ void leaf_moments(const MpArgs<T> &a, int c, const uint4 cd) {
+  const int pb = (int)cd.z, pe = (int)cd.w;
+  Moments<T> m{};
+  Ext<T> e = ext_empty<T>();
+  const V4<T> r0 = a.pos[pb];  // reference point: the first particle
+  auto add = [&](const V4<T> p) {
+    ext_add(e, p.x, p.y, p.z);
+    const T dx = p.x - r0.x, dy = p.y - r0.y, dz = p.z - r0.z, w = p.w;
+    m.M += w;
+    m.sx += w * dx; m.sy += w * dy; m.sz += w * dz;
+    m.xx += w * dx * dx; m.yy += w * dy * dy; m.zz += w * dz * dz;
+    m.xy += w * dx * dy; m.xz += w * dx * dz; m.yz += w * dy * dz;
+  };
+  // particles in order, four loads issued together
+  int i = pb;
+  for (; i + 4 <= pe; i += 4) {
+    const V4<T> p0 = a.pos[i], p1 = a.pos[i + 1], p2 = a.pos[i + 2], p3 = a.pos[i + 3];
+    add(p0);
+    add(p1);
+    add(p2);
+    add(p3);
+  }
+  for (; i < pe; i++) add(a.pos[i]);
+  finish_moments<T, T, CLIMB>(a, c, r0.x, r0.y, r0.z, m, e);
+}
+
+// The leaves of every level.
 template <typename T>
+__global__ __launch_bounds__(kBlock) void k_multipole_leaves(MpArgs<T> a) {
+  BT_BUILD_PRIO();
+  const int nc = a.dc->ncells;
+  for (int c = blockIdx.x * kBlock + threadIdx.x; c < nc; c += gridDim.x * kBlock) {
+    const uint4 cd = a.cells[c];
+    if (cell_leaf(cd)) leaf_moments<T>(a, c, cd);
+  }
+}
+
+// The nodes of one level, whose children are done.
+template <typename T, typename R>
 __global__ __launch_bounds__(kBlock) void k_multipole_level(MpArgs<T> a) {
   BT_BUILD_PRIO();
   const int cnt = a.dc->lvl_count[a.L];
   const int c0 = a.dc->lvl_start[a.L];
   for (int t = blockIdx.x * kBlock + threadIdx.x; t < cnt; t += gridDim.x * kBlock) {
-    const int c = c0 + t;
-    const uint4 cd = a.cells[c];
-    const int pb = (int)cd.z, pe = (int)cd.w;
-    if (cell_leaf(cd)) {
-      Moments<T> m{};
-      Ext<T> e = ext_empty<T>();
-      const V4<T> r0 = a.pos[pb];  // reference point: the first particle
-      auto add = [&](const V4<T> p) {
-        ext_add(e, p.x, p.y, p.z);
-        const T dx = p.x - r0.x, dy = p.y - r0.y, dz = p.z - r0.z, w = p.w;
-        m.M += w;
-        m.sx += w * dx; m.sy += w * dy; m.sz += w * dz;
-        m.xx += w * dx * dx; m.yy += w * dy * dy; m.zz += w * dz * dz;
-        m.xy += w * dx * dy; m.xz += w * dx * dz; m.yz += w * dy * dz;
-      };
-      // particles in order, four loads issued together
-      int i = pb;
-      for (; i + 4 <= pe; i += 4) {
-        const V4<T> p0 = a.pos[i], p1 = a.pos[i + 1], p2 = a.pos[i + 2], p3 = a.pos[i + 3];
-        add(p0);
-        add(p1);
-        add(p2);
-        add(p3);
-      }
-      for (; i < pe; i++) add(a.pos[i]);
-      finish_moments<T, T>(a, c, r0.x, r0.y, r0.z, m, e);
-    } else if (sizeof(T) == 8 || a.L <= kFp64Levels) {
-      node_moments<T, double>(a, c, cd);
-    } else {
-      node_moments<T, float>(a, c, cd);
+    const uint4 cd = a.cells[c0 + t];
+    if (!cell_leaf(cd)) node_moments<T, R>(a, c0 + t, cd);
+  }
+}
+
+// All cells of a small tree in one launch: the thread of a leaf climbs.  At each
+// parent it counts itself in; the last child to arrive combines the parent's
+// children (in their order, so the result does not depend on who arrives last) and
+// goes on from there.  Nothing waits.  The count of a parent is raised only after
+// the stores of the child's record have completed, and its children's records are
+// read after the count has shown them all: both by agent-scope accesses.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_multipole_climb(MpArgs<T> a) {
+  BT_BUILD_PRIO();
+  const int ncells = a.dc->ncells;
+  for (int t = blockIdx.x * kBlock + threadIdx.x; t < ncells; t += gridDim.x * kBlock) {
+    int c = t;
+    uint4 cd = a.cells[c];
+    if (!cell_leaf(cd)) continue;
+    leaf_moments<T, true>(a, c, cd);
+    for (int L = (int)(cd.x >> 27); L > 1; L--) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this cell's record is out
+      const int p = (int)(cd.x & 0x07FFFFFFu);
+      cd = a.cells[p];
+      const int before = __hip_atomic_fetch_add(a.arrived + p, 1, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT);
+      if (before + 1 < cell_nchild(cd)) break;
+      __hip_atomic_store(a.arrived + p, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next call
+      c = p;
+      if (sizeof(T) == 8 || L - 1 <= kFp64Levels) node_moments<T, double, true>(a, c, cd);
+      else node_moments<T, float, true>(a, c, cd);
     }
   }
 }
@@ -712,6 +799,7 @@ void launch_levels(Ctx &c) {
   a.raw = c.cell_raw;
   a.fin = c.cell_fin;
   a.nch = c.cell_nch;
+  a.arrived = c.cell_arrived;
   a.cnt = c.cell_cnt;
   a.root_cells = c.root_cells;
   a.level_beg = c.level_beg;
@@ -742,11 +830,22 @@ void multipoles_t(Ctx &c) {
   a.q1 = as2<T>(c.cq1);
   a.ls = as2<T>(c.cls);
   a.wrec = as4<T>(c.cwalk);
+  a.arrived = c.cell_arrived;
   a.dc = c.dc;
   const int grid = grid_for(c.cap_cells, kBlock, 2048);
-  for (int L = kMaxLevel; L >= 1; L--) {
+  // computeMultipoles, one launch per level / one in all: 2^10 87 / 26 us, 2^16 88 /
+  // 46, 2^18 106 / 58, 2^20 118 / 159 (records past the L2 cost more than launches)
+  if (c.n <= 1 << 18) {
+    hipLaunchKernelGGL(k_multipole_climb<T>, dim3(grid), dim3(kBlock), 0, c.stream, a);
+    return;
+  }
+  hipLaunchKernelGGL(k_multipole_leaves<T>, dim3(grid_for(c.cap_cells, kBlock, 8192)), dim3(kBlock),
+                     0, c.stream, a);
+  for (int L = kMaxLevel - 1; L >= 1; L--) {   // level kMaxLevel holds leaves only
     a.L = L;
-    hipLaunchKernelGGL(k_multipole_level<T>, dim3(grid), dim3(kBlock), 0, c.stream, a);
+    auto kern = sizeof(T) == 8 || L <= kFp64Levels ? k_multipole_level<T, double>
+                                                   : k_multipole_level<T, T>;
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), 0, c.stream, a);
   }
 }
 

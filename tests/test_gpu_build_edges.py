@@ -70,3 +70,42 @@ def test_forest_cells_match_single_systems(bt, oracle, sizes):
             kids = got[first:first + nchild]
             assert (kids[:, 0] & 0x07FFFFFF == i).all() and kids[:, 2].min() == pb
             assert kids[:, 3].max() == pe
+
+
+def _moments(t):
+    """Cells' moments by (level, particle range)."""
+    g = t.tree()
+    rows = {}
+    for k, (x, y, pb, pe) in enumerate(g["cells"].tolist()):
+        rows[(x >> 27, pb, pe)] = (g["size"][k].tobytes(), g["mono"][k].tobytes(),
+                                   g["q0"][k].tobytes(), g["q1"][k].tobytes())
+    return rows
+
+
+@pytest.mark.parametrize("fp64", [False, True])
+def test_moments_do_not_depend_on_the_launches(bt, fp64):
+    """Small trees take their moments in one launch, larger ones level by level: a
+    system's are the same bits alone and in a forest of more than 2^18 particles,
+    and again when they are computed once more."""
+    small, big = 5001, 1 << 18
+    ps, vs = bt.clustered(small, 8, seed=41)
+    pb, vb = bt.plummer(big, seed=42)
+    real = np.float64 if fp64 else np.float32
+    t = bt.Treecode(0.01, 0.5, 64, fp64=fp64)
+    t.alloc(small)
+    t.ptcl_h2d(ps.astype(real), vs.astype(real))
+    t.buildTree(16)
+    t.computeMultipoles()
+    alone = _moments(t)
+    t.set_params(theta=0.7)
+    t.computeMultipoles()
+    t.set_params(theta=0.5)
+    t.computeMultipoles()
+    assert _moments(t) == alone
+    t.alloc(small + big, np.array([0, small, small + big], np.int32))
+    t.ptcl_h2d(np.concatenate([ps, pb]).astype(real), np.concatenate([vs, vb]).astype(real))
+    t.buildTree(16)
+    t.computeMultipoles()
+    both = _moments(t)
+    t.close()
+    assert {k: v for k, v in both.items() if k[2] <= small} == alone
