@@ -255,11 +255,10 @@ void launch_multipoles(Ctx &c);
 void radix_sort_pairs(Ctx &c, uint64_t *keys, int *vals, uint64_t *keys_tmp, int *vals_tmp,
                       int n, int key_bits, bool by_system_after);
 void scan_exclusive_sum(Ctx &c, const int *in, int *out, int n, int *total_dev);
-void scan_inclusive_max(Ctx &c, const int *in, int *out, int n);
 void fill_int(Ctx &c, int *p, int value, int n);
 
 void launch_ph_keys(Ctx &c);
-void launch_gather_ph(Ctx &c);
+// the PH gather of the particles and the groups
 void launch_groups(Ctx &c);
 // groups = tree cells (mode 1: the leaves; mode 2: cells of <= ncrit
 // particles), in tree order; the group order is the tree order

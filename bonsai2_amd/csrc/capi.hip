@@ -215,7 +215,6 @@ int phase_groups(Ctx &c, int end_ev = 7) {
   record(c, 5);
   radix_sort_pairs(c, c.ph_keys, c.perm, c.keyB, c.valB, c.n, 63, true);
   record(c, 6);
-  launch_gather_ph(c);
   launch_groups(c);
   record(c, end_ev);
   BT_LAUNCH_CK();

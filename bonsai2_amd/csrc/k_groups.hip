@@ -6,9 +6,9 @@
 // of equal keys masked to the top level_split octal digits (:137-192) is cut
 // into chunks of ncrit (:196-223).  The reference finds run bounds with two
 // inclusive_scan_by_key calls and takes group slots from an atomic counter;
-// here a max-scan gives each particle its run start and a sum-scan over the
-// "first particle of a group" flags gives deterministic group slots in PH
-// order.
+// here each tile of particles finds the start of the run it begins in by a
+// search, and a scan of the tiles' group counts gives deterministic group slots
+// in PH order.
 #include "bt_device.h"
 #include "bt_internal.h"
 
@@ -74,41 +74,216 @@ __global__ __launch_bounds__(kBlock) void k_ph_keys(int n, int nsys, const int *
   }
 }
 
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_gather_ph(int n, const int *__restrict__ perm,
-                                                      const T *__restrict__ pos,
-                                                      const int *__restrict__ id,
-                                                      T *__restrict__ pos_ph,
-                                                      int *__restrict__ id_ph) {
-  BT_BUILD_PRIO();
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
-    const int j = perm[i];
-    pos_ph[i] = pos[j];
-    id_ph[i] = id[j];
-  }
+// ---- groups of PH-key runs ------------------------------------------------------
+//
+// Three launches: the PH gather together with the group counts of every tile, the
+// scan of the counts, and the groups.  A particle begins a group iff its distance
+// from the start of its run (equal masked keys within a system) is a multiple of
+// NCRIT.  Run starts are bits of a tile; the run a tile begins in may have started
+// in any tile before it, so a wave looks for it with a 64-way search (4 dependent
+// loads at 2^24 keys).  A group ends at the next run start or after NCRIT <= 64
+// particles, so a tile needs one word of bits beyond its own.  Bound by the gather.
+// (Run starts, a maximum scan, flags, a sum scan, emission and sizes as launches of
+// their own took 9 of them, 0.25 ms at 2^24 particles, and 30 us at 2^10.)
+
+constexpr int kGroupTile = 1024;
+constexpr int kTileWords = kGroupTile / kWave;
+constexpr int kScanThreads = 1024, kScanPer = 4;
+
+struct GroupArgs {
+  int n, nsys, ncrit, ntiles, cap;
+  const int *off;
+  const uint64_t *keys;
+  uint64_t mask;
+  int *count;      // groups of each tile, then their prefixes
+  int *carry;      // start of the run each tile begins in
+  int2 *groups;
+  int *group_sys;
+  DevCounters *dc;
+};
+
+// Whether particle i starts a run; the ones past the last do.
+template <bool FOREST>
+__device__ __forceinline__ bool run_start(const GroupArgs &a, int i) {
+  if (i == 0 || i >= a.n) return true;
+  if ((a.keys[i] & a.mask) != (a.keys[i - 1] & a.mask)) return true;
+  return FOREST && system_of(i, a.nsys, a.off) != system_of(i - 1, a.nsys, a.off);
 }
 
-// v[i] = i at the start of a run of equal masked keys (or of a system), else 0.
-__global__ __launch_bounds__(kBlock) void k_run_starts(int n, int nsys, const int *__restrict__ off,
-                                                       const uint64_t *__restrict__ keys,
-                                                       uint64_t mask, int *__restrict__ v) {
-  BT_BUILD_PRIO();
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
-    bool start = i == 0;
-    if (!start) {
-      start = (keys[i] & mask) != (keys[i - 1] & mask);
-      if (!start && nsys > 1) start = system_of(i, nsys, off) != system_of(i - 1, nsys, off);
+// The first particle of particle i's run (all lanes of the wave, same i): the
+// masked keys of a system do not decrease.
+template <bool FOREST>
+__device__ __forceinline__ int find_run_start(const GroupArgs &a, int i) {
+  const uint64_t m = a.keys[i] & a.mask;
+  int lo = FOREST ? a.off[system_of(i, a.nsys, a.off)] : 0, hi = i;   // in [lo, hi]
+  while (lo < hi) {
+    const int step = (hi - lo + kWave - 1) / kWave;
+    const int p = lo + lane_id() * step;
+    const uint64_t in_run = ballot64(p < hi && (a.keys[p] & a.mask) >= m);
+    if (in_run == 0) {
+      lo = min(hi, lo + ((hi - lo - 1) / step) * step + 1);   // past the last one looked at
+    } else {
+      const int f = __ffsll((unsigned long long)in_run) - 1;
+      hi = lo + f * step;
+      lo = f > 0 ? hi - step + 1 : lo;
     }
-    v[i] = start ? i : 0;
+  }
+  return lo;
+}
+
+// Bits and run starts of one tile: bits[k] for particles t0 + 64 k.., k <= kTileWords;
+// before[k]: the last run start before word k.
+struct GroupTile {
+  uint64_t bits[kTileWords + 1];
+  int before[kTileWords];
+  int wave_sum[kBlock / kWave];
+};
+
+template <bool FOREST>
+__device__ __forceinline__ void load_group_tile(const GroupArgs &a, int t0, int carry,
+                                                GroupTile &T) {
+  const int lane = lane_id(), w = threadIdx.x >> 6;
+  for (int k = w; k <= kTileWords; k += kBlock / kWave) {
+    const uint64_t b = ballot64(run_start<FOREST>(a, t0 + k * kWave + lane));
+    if (lane == 0) T.bits[k] = b;
+  }
+  __syncthreads();
+  if (w == 0) {
+    const uint64_t b = lane < kTileWords ? T.bits[lane] : 0;
+    int last = b != 0 ? t0 + lane * kWave + 63 - __clzll((long long)b) : carry;
+    // inclusive maximum over the words (a run start is never before an earlier one)
+    for (int d = 1; d < kTileWords; d <<= 1) {
+      const int v = __shfl_up(last, d, kWave);
+      if (lane >= d) last = max(last, v);
+    }
+    const int v = __shfl_up(last, 1, kWave);
+    if (lane < kTileWords) T.before[lane] = lane == 0 ? carry : v;
+  }
+  __syncthreads();
+}
+
+// Whether particle t0 + 64 k + lane begins a group.
+__device__ __forceinline__ bool begins_group(const GroupArgs &a, int t0, int k,
+                                             const GroupTile &T) {
+  const int lane = lane_id(), i = t0 + k * kWave + lane;
+  const uint64_t upto = T.bits[k] & (lanemask_lt() | (1ull << lane));
+  const int start = upto != 0 ? t0 + k * kWave + 63 - __clzll((long long)upto) : T.before[k];
+  return i < a.n && (unsigned)(i - start) % (unsigned)a.ncrit == 0;
+}
+
+template <typename T, bool FOREST>
+__global__ __launch_bounds__(kBlock) void k_gather_count(GroupArgs a, const int *__restrict__ perm,
+                                                         const T *__restrict__ pos,
+                                                         const int *__restrict__ id,
+                                                         T *__restrict__ pos_ph,
+                                                         int *__restrict__ id_ph) {
+  BT_BUILD_PRIO();
+  __shared__ GroupTile tile;
+  const int t0 = blockIdx.x * kGroupTile;
+  const int lane = lane_id(), w = threadIdx.x >> 6;
+#pragma unroll
+  for (int r = 0; r < kGroupTile / kBlock; r++) {
+    const int i = t0 + r * kBlock + threadIdx.x;
+    if (i < a.n) {
+      const int j = perm[i];
+      pos_ph[i] = pos[j];
+      id_ph[i] = id[j];
+    }
+  }
+  const int carry = find_run_start<FOREST>(a, t0);
+  load_group_tile<FOREST>(a, t0, carry, tile);
+  int cnt = 0;
+  for (int k = w; k < kTileWords; k += kBlock / kWave)
+    cnt += __popcll(ballot64(begins_group(a, t0, k, tile)));
+  if (lane == 0) tile.wave_sum[w] = cnt;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int s = 0;
+    for (int k = 0; k < kBlock / kWave; k++) s += tile.wave_sum[k];
+    a.count[blockIdx.x] = s;
+    a.carry[blockIdx.x] = carry;
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_group_flags(int n, int ncrit,
-                                                        const int *__restrict__ run_start,
-                                                        int *__restrict__ flag) {
+// One block: the tiles' counts to prefixes, the number of groups to the counters.
+__global__ __launch_bounds__(kScanThreads) void k_group_scan(GroupArgs a) {
   BT_BUILD_PRIO();
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock)
-    flag[i] = ((i - run_start[i]) % ncrit) == 0 ? 1 : 0;
+  __shared__ int shw[kScanThreads / kWave];
+  const int w = threadIdx.x >> 6;
+  int carry = 0;
+  for (int b0 = 0; b0 < a.ntiles; b0 += kScanThreads * kScanPer) {
+    int v[kScanPer], own = 0;
+#pragma unroll
+    for (int k = 0; k < kScanPer; k++) {
+      const int i = b0 + threadIdx.x * kScanPer + k;
+      v[k] = i < a.ntiles ? a.count[i] : 0;
+      own += v[k];
+    }
+    const int incl = wave_incl_scan(own);
+    if (lane_id() == kWave - 1) shw[w] = incl;
+    __syncthreads();
+    int pre = carry, tot = 0;
+    for (int k = 0; k < kScanThreads / kWave; k++) {
+      if (k < w) pre += shw[k];
+      tot += shw[k];
+    }
+    int run = pre + incl - own;
+#pragma unroll
+    for (int k = 0; k < kScanPer; k++) {
+      const int i = b0 + threadIdx.x * kScanPer + k;
+      if (i < a.ntiles) a.count[i] = run;
+      run += v[k];
+    }
+    carry += tot;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    a.dc->ngroups = carry;
+    atomicAnd(&a.dc->err, ~2);   // a new set of groups; the level build may run beside this
+  }
+}
+
+template <bool FOREST>
+__global__ __launch_bounds__(kBlock) void k_group_write(GroupArgs a) {
+  BT_BUILD_PRIO();
+  __shared__ GroupTile tile;
+  const int t0 = blockIdx.x * kGroupTile;
+  const int lane = lane_id(), w = threadIdx.x >> 6;
+  load_group_tile<FOREST>(a, t0, a.carry[blockIdx.x], tile);
+  // wave w takes a quarter of the words in a row
+  constexpr int kPer = kTileWords / (kBlock / kWave);
+  uint64_t first[kPer];
+  int cnt = 0;
+#pragma unroll
+  for (int q = 0; q < kPer; q++) {
+    first[q] = ballot64(begins_group(a, t0, w * kPer + q, tile));
+    cnt += __popcll(first[q]);
+  }
+  if (lane == 0) tile.wave_sum[w] = cnt;
+  __syncthreads();
+  int slot = a.count[blockIdx.x];
+  for (int k = 0; k < w; k++) slot += tile.wave_sum[k];
+#pragma unroll
+  for (int q = 0; q < kPer; q++) {
+    const int k = w * kPer + q;
+    if ((first[q] >> lane) & 1) {
+      const int i = t0 + k * kWave + lane;
+      const int g = slot + __popcll(first[q] & lanemask_lt());
+      // run starts after i: the rest of its word, then the next word
+      const uint64_t after = lane == kWave - 1 ? tile.bits[k + 1]
+                                               : (tile.bits[k] >> (lane + 1)) |
+                                                     (tile.bits[k + 1] << (kWave - 1 - lane));
+      const int next = after != 0 ? __ffsll((unsigned long long)after) : kWave;
+      if (g < a.cap) {
+        a.groups[g] = make_int2(i, min(next, a.ncrit));
+        a.group_sys[g] = FOREST ? system_of(i, a.nsys, a.off) : 0;
+      } else {
+        atomicOr(&a.dc->err, 2);
+        atomicOr(&a.dc->err_sticky, 2);
+      }
+    }
+    slot += __popcll(first[q]);
+  }
 }
 
 __global__ __launch_bounds__(kBlock) void k_group_emit(int n, int nsys, const int *__restrict__ off,
@@ -151,16 +326,6 @@ void launch_ph_keys(Ctx &c) {
   else
     hipLaunchKernelGGL(k_ph_keys<float>, g, dim3(kBlock), 0, c.stream, c.n, c.nsys, c.d_off, c.box,
                        c.pos, c.ph_keys, c.perm);
-}
-
-void launch_gather_ph(Ctx &c) {
-  const dim3 g(grid_for(c.n, kBlock, 8192));
-  if (c.fp64)
-    hipLaunchKernelGGL(k_gather_ph<double4>, g, dim3(kBlock), 0, c.stream, c.n, c.perm,
-                       as4<double>(c.pos), c.id, as4<double>(c.pos_ph), c.id_ph);
-  else
-    hipLaunchKernelGGL(k_gather_ph<float4>, g, dim3(kBlock), 0, c.stream, c.n, c.perm, c.pos,
-                       c.id, c.pos_ph, c.id_ph);
 }
 
 // A new set of groups starts without the group error bit.
@@ -236,23 +401,38 @@ void launch_leaf_groups(Ctx &c) {
 
 void launch_groups(Ctx &c) {
   const int ls = c.level_split < 1 ? 1 : c.level_split;
-  uint64_t mask = 0;  // top ls octal digits of the 63-bit key (code/makeGroups.cu:259-266)
+  GroupArgs a;
+  a.n = c.n;
+  a.nsys = c.nsys;
+  a.ncrit = c.ncrit;
+  a.ntiles = (c.n + kGroupTile - 1) / kGroupTile;
+  a.cap = c.cap_groups;
+  a.off = c.d_off;
+  a.keys = c.ph_keys;
+  a.mask = 0;  // top ls octal digits of the 63-bit key (code/makeGroups.cu:259-266)
   for (int i = 0; i < 21; i++) {
-    mask <<= 3;
-    if (i < ls) mask |= 7;
+    a.mask <<= 3;
+    if (i < ls) a.mask |= 7;
   }
-  const int g = grid_for(c.n, kBlock, 8192);
-  hipLaunchKernelGGL(k_groups_init, dim3(1), dim3(64), 0, c.stream, c.dc);
-  hipLaunchKernelGGL(k_run_starts, dim3(g), dim3(kBlock), 0, c.stream, c.n, c.nsys, c.d_off,
-                     c.ph_keys, mask, c.gtmp0);
-  scan_inclusive_max(c, c.gtmp0, c.gtmp1, c.n);
-  hipLaunchKernelGGL(k_group_flags, dim3(g), dim3(kBlock), 0, c.stream, c.n, c.ncrit, c.gtmp1,
-                     c.gtmp0);
-  scan_exclusive_sum(c, c.gtmp0, c.gtmp1, c.n, &c.dc->ngroups);
-  hipLaunchKernelGGL(k_group_emit, dim3(g), dim3(kBlock), 0, c.stream, c.n, c.nsys, c.d_off,
-                     c.gtmp0, c.gtmp1, c.cap_groups, c.groups, c.group_sys, c.dc);
-  hipLaunchKernelGGL(k_group_sizes, dim3(grid_for(c.cap_groups, kBlock, 4096)), dim3(kBlock), 0,
-                     c.stream, c.n, c.cap_groups, c.groups, c.dc);
+  a.count = c.gtmp0;
+  a.carry = c.gtmp1;
+  a.groups = c.groups;
+  a.group_sys = c.group_sys;
+  a.dc = c.dc;
+  const dim3 tiles(a.ntiles);
+  const bool forest = c.nsys > 1;
+  if (c.fp64) {
+    auto kern = forest ? k_gather_count<double4, true> : k_gather_count<double4, false>;
+    hipLaunchKernelGGL(kern, tiles, dim3(kBlock), 0, c.stream, a, c.perm, as4<double>(c.pos), c.id,
+                       as4<double>(c.pos_ph), c.id_ph);
+  } else {
+    auto kern = forest ? k_gather_count<float4, true> : k_gather_count<float4, false>;
+    hipLaunchKernelGGL(kern, tiles, dim3(kBlock), 0, c.stream, a, c.perm, c.pos, c.id, c.pos_ph,
+                       c.id_ph);
+  }
+  hipLaunchKernelGGL(k_group_scan, dim3(1), dim3(kScanThreads), 0, c.stream, a);
+  hipLaunchKernelGGL(forest ? k_group_write<true> : k_group_write<false>, tiles, dim3(kBlock), 0,
+                     c.stream, a);
 }
 
 }  // namespace bt

@@ -16,8 +16,6 @@
 // cache lines instead of one scattered store per pair).
 // A tile is 256 threads x 16 rounds = 4096 pairs; HBM traffic per pass is
 // ~8 B (histogram read) + 12 B read + 12 B written per pair.
-#include <climits>
-
 #include "bt_device.h"
 #include "bt_internal.h"
 
@@ -61,10 +59,6 @@ __device__ __forceinline__ int digit_of(uint64_t key, int val, const DigitSrc &s
 struct OpSum {
   static __device__ __forceinline__ int id() { return 0; }
   static __device__ __forceinline__ int op(int a, int b) { return a + b; }
-};
-struct OpMax {
-  static __device__ __forceinline__ int id() { return INT_MIN; }
-  static __device__ __forceinline__ int op(int a, int b) { return a > b ? a : b; }
 };
 
 // Inclusive scan across a 256-thread block; returns inclusive value, *total = block total.
@@ -506,7 +500,7 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_blocks(int *__restrict__ 
 // tiles before it itself (for few tiles: one launch instead of a separate
 // scan of the totals); the last block writes the grand total to total_dev.
 // Otherwise blk holds the tiles' exclusive prefixes (k_scan_blocks).
-template <class Op, bool kInclusive, bool kPrefix>
+template <class Op, bool kPrefix>
 __global__ __launch_bounds__(kScanThreads) void k_scan_down(const int *__restrict__ in, int n,
                                                             const int *__restrict__ blk,
                                                             int *__restrict__ out,
@@ -549,7 +543,7 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_down(const int *__restric
 #pragma unroll
   for (int k = 0; k < kScanItems; k++) {
     const int nv = Op::op(acc, vals[k]);
-    sh[threadIdx.x * kScanItems + k] = kInclusive ? nv : acc;
+    sh[threadIdx.x * kScanItems + k] = acc;
     acc = nv;
   }
   if (kPrefix && total_dev && threadIdx.x == 0 && blockIdx.x == gridDim.x - 1)
@@ -567,7 +561,7 @@ __global__ void k_fill_int(int *p, int value, int n) {
     p[i] = value;
 }
 
-template <class Op, bool kInclusive>
+template <class Op>
 void scan_impl(Ctx &c, const int *in, int *out, int n, int *total_dev) {
   if (n <= 0) {
     if (total_dev) fill_int(c, total_dev, 0, 1);
@@ -587,13 +581,13 @@ void scan_impl(Ctx &c, const int *in, int *out, int n, int *total_dev) {
   hipLaunchKernelGGL((k_scan_reduce<Op>), dim3(nb), dim3(kScanThreads), 0, c.stream, in, n,
                      c.scan_blk);
   if (nb <= kScanFusedTiles) {
-    hipLaunchKernelGGL((k_scan_down<Op, kInclusive, true>), dim3(nb), dim3(kScanThreads), 0,
+    hipLaunchKernelGGL((k_scan_down<Op, true>), dim3(nb), dim3(kScanThreads), 0,
                        c.stream, in, n, c.scan_blk, out, total_dev);
     return;
   }
   hipLaunchKernelGGL((k_scan_blocks<Op>), dim3(1), dim3(kScanThreads), 0, c.stream, c.scan_blk,
                      nb, total_dev);
-  hipLaunchKernelGGL((k_scan_down<Op, kInclusive, false>), dim3(nb), dim3(kScanThreads), 0,
+  hipLaunchKernelGGL((k_scan_down<Op, false>), dim3(nb), dim3(kScanThreads), 0,
                      c.stream, in, n, c.scan_blk, out, nullptr);
 }
 
@@ -767,11 +761,7 @@ void fill_int(Ctx &c, int *p, int value, int n) {
 }
 
 void scan_exclusive_sum(Ctx &c, const int *in, int *out, int n, int *total_dev) {
-  scan_impl<OpSum, false>(c, in, out, n, total_dev);
-}
-
-void scan_inclusive_max(Ctx &c, const int *in, int *out, int n) {
-  scan_impl<OpMax, true>(c, in, out, n, nullptr);
+  scan_impl<OpSum>(c, in, out, n, total_dev);
 }
 
 // Sorts (keys, vals)[0..n) stably by the low key_bits bits of the key; when
