@@ -21,7 +21,7 @@
 //     the walk, not LDS or the scalar cache;
 //   * each batch is summed in FP32 and folded into Kahan-compensated
 //     accumulators.
-// Systems of at most 2^17 particles are walked by the four waves of a block per
+// Systems of at most 2^19 particles are walked by the four waves of a block per
 // group instead (k_walk_team below).
 // The interaction set equals the reference's (the order of traversal does
 // not change which cells are opened); FP32 sums run in a different order.
@@ -74,11 +74,6 @@ constexpr int kXcd = 8;   // MI355X: 8 XCDs, workgroups dispatched round-robin o
 __device__ __forceinline__ int xcd_lo(int ngroups, int x) {
   return (int)((long long)ngroups * x / kXcd);
 }
-// Blocks of the grid on XCD x (workgroups are dispatched round-robin).
-__device__ __forceinline__ int xcd_blocks(int x) {
-  return ((int)gridDim.x - x + kXcd - 1) / kXcd;
-}
-
 // Next group for this wave: each range has a queue, which a wave drains for its
 // own XCD first and then for the others.  Every lane joins the atomics (lane 0
 // adds 1) and all branches are uniform.  (Reading a queue's head before adding
@@ -133,11 +128,26 @@ struct WalkArgs {
 // the wave; each batch of j-entries is split between the half-waves (lanes
 // 0-31 sweep its first half, lanes 32-63 its second), so every broadcast LDS
 // read serves two interactions, and the halves' sums are added once per group.
+//
+// A group of np <= 32 particles would leave half of the lanes or more idle: with
+// IPL = 1 the wave then holds `slices` copies of the group, lane l particle l % np,
+// and copy l / np sweeps the entries copy, copy + slices, ... of each batch.  The
+// copies' sums are added once per group, in FP64.  (A group has 28 particles on
+// average in a system of 2^16, four in one of 2^10.)  256 systems of 2^10 to 2^16:
+// 8.8 -> 7.5 ms per walk.
 template <typename R, int IPL>
 struct IParts {
   R x[IPL], y[IPL], z[IPL];
   Acc4T<R> s[IPL], c[IPL];   // Kahan sums and compensations
+  int slices, slice;         // copies of the group, and this lane's
 };
+
+// Copies of a group of np particles: as many as fit, of the numbers whose rounds
+// over a batch of 64 entries end within kJSlots slots.
+__device__ __forceinline__ int group_slices(int np) {
+  const int s = kWave / np;
+  return s >= 16 ? 16 : s >= 8 ? 8 : s >= 6 ? 6 : s;
+}
 
 // LDS slots of one batch: 64 entries; with IPL = 2 the second half-wave's
 // entries start one slot later (its broadcast address differs from the first
@@ -211,6 +221,21 @@ __device__ __forceinline__ void stage_pad(Stage<R> &S, int slot) {
   S.jC[slot] = make_v4<R>(R(0), R(0), R(0), R(0));
 }
 
+// The slots past a batch of 64 that the copies of a small group may read.
+template <typename R>
+__device__ __forceinline__ void stage_tail(Stage<R> &S) {
+  if (lane_id() < kJSlots - kWave) stage_pad(S, kWave + lane_id());
+}
+
+// Whether this lane stages a pad: the copies of a small group sweep cnt entries
+// rounded up to a multiple of their number.
+template <typename R, int IPL>
+__device__ __forceinline__ bool pads(const IParts<R, IPL> &ip, int cnt) {
+  const int lane = lane_id();
+  if (IPL == 2) return lane == cnt;
+  return ip.slices > 1 && lane >= cnt && lane < cnt + ip.slices;
+}
+
 // Sweeps a staged batch: P2C (QUAD) or particle-like (P2P and monopole-only
 // P2C) interactions of the lane's i-particles with its half of the entries.
 template <bool KAHAN, bool QUAD, typename R, int IPL>
@@ -267,6 +292,18 @@ __device__ __forceinline__ void sweep(const Stage<R> &S, int cnt, R eps2,
         cur = nxt;
       }
     }
+  } else if (ip.slices > 1) {
+    const int rounds = (cnt + ip.slices - 1) / ip.slices;
+    int slot = ip.slice;
+    J cur = load(slot);
+#pragma unroll 2
+    for (int j = 1; j <= rounds; j++) {
+      slot += j < rounds ? ip.slices : 0;
+      const J nxt = load(slot);
+      __builtin_amdgcn_sched_barrier(0);   // keep the reads ahead of the arithmetic
+      eval(cur);
+      cur = nxt;
+    }
   } else {
     J cur = load(0);
     if (cnt == kWave) {
@@ -306,8 +343,8 @@ __device__ __forceinline__ void eval_p2c(const WalkArgs<R> &a, Stage<R> &S, cons
     S.jA[d] = make_v4<R>(r0.x - gcx, r0.y - gcy, r0.z - gcz, r0.w);
     S.jB[d] = a.cwalk[3 * ci + 1];
     S.jC[d] = a.cwalk[3 * ci + 2];
-  } else if (IPL == 2 && lane == cnt) {
-    stage_pad(S, cnt + 1);
+  } else if (pads<R, IPL>(ip, cnt)) {
+    stage_pad(S, IPL == 2 ? cnt + 1 : lane);
   }
   wave_lds_sync();
   sweep<KAHAN, true, R, IPL>(S, cnt, a.eps2, ip);
@@ -322,8 +359,8 @@ __device__ __forceinline__ void eval_p2p(const WalkArgs<R> &a, Stage<R> &S, cons
   if (lane < cnt) {
     const V4<R> p = a.pos_tree[list[lane]];
     S.jA[jslot<IPL>(lane, hc)] = make_v4<R>(p.x - gcx, p.y - gcy, p.z - gcz, p.w);
-  } else if (IPL == 2 && lane == cnt) {
-    stage_pad(S, cnt + 1);
+  } else if (pads<R, IPL>(ip, cnt)) {
+    stage_pad(S, IPL == 2 ? cnt + 1 : lane);
   }
   wave_lds_sync();
   sweep<KAHAN, false, R, IPL>(S, cnt, a.eps2, ip);
@@ -341,8 +378,8 @@ __device__ __forceinline__ void eval_p2c_mono(const WalkArgs<R> &a, Stage<R> &S,
   if (lane < cnt) {
     const V4<R> r0 = a.cwalk[3 * list[lane]];
     S.jA[jslot<IPL>(lane, hc)] = make_v4<R>(r0.x - gcx, r0.y - gcy, r0.z - gcz, r0.w);
-  } else if (IPL == 2 && lane == cnt) {
-    stage_pad(S, cnt + 1);
+  } else if (pads<R, IPL>(ip, cnt)) {
+    stage_pad(S, IPL == 2 ? cnt + 1 : lane);
   }
   wave_lds_sync();
   sweep<KAHAN, false, R, IPL>(S, cnt, a.eps2, ip);
@@ -537,11 +574,13 @@ void k_walk(WalkArgs<R> a) {
     const int2 grp = a.groups[g];
     const int pbeg = grp.x, np = max(grp.y, 1);
     const int sys = a.nsys > 1 ? a.group_sys[g] : 0;
+    const int slices = IPL == 1 && !SJ ? group_slices(np) : 1;
     // the lane's i-particles (clamped to the last one, :534)
     V4<R> pi[IPL];
 #pragma unroll
     for (int k = 0; k < IPL; k++)
-      pi[k] = a.pos_ph[pbeg + min(IPL == 1 ? lane : 2 * (lane & 31) + k, np - 1)];
+      pi[k] = a.pos_ph[pbeg + (IPL == 1 ? (slices > 1 ? lane % np : min(lane, np - 1))
+                                        : min(2 * (lane & 31) + k, np - 1))];
 
     // group box (code/computeForces.cu:539-555)
     R lmnx = pi[0].x, lmny = pi[0].y, lmnz = pi[0].z;
@@ -563,6 +602,9 @@ void k_walk(WalkArgs<R> a) {
     if constexpr (LEARN) geom = make_group_geom(gcx, gcy, gcz, gsx, gsy, gsz, np, a.sys_scale[sys]);
     // i-particles: relative to the group centre (LDS path) or absolute (scalar path)
     IParts<R, IPL> ip;
+    ip.slices = slices;
+    ip.slice = min(lane / np, slices - 1);
+    if (IPL == 1) stage_tail(S);
 #pragma unroll
     for (int k = 0; k < IPL; k++) {
       ip.x[k] = SJ ? pi[k].x : pi[k].x - gcx;
@@ -734,6 +776,18 @@ void k_walk(WalkArgs<R> a) {
     int idx;
     if (IPL == 1) {
       res = ip.s[0];
+      if (slices > 1) {
+        // the copies' compensated sums, in their order
+        const Acc4T<R> cc = ip.c[0];
+        const double v[4] = {(double)res.x - (KAHAN ? (double)cc.x : 0.0),
+                             (double)res.y - (KAHAN ? (double)cc.y : 0.0),
+                             (double)res.z - (KAHAN ? (double)cc.z : 0.0),
+                             (double)res.w - (KAHAN ? (double)cc.w : 0.0)};
+        double t[4] = {v[0], v[1], v[2], v[3]};
+        for (int k = 1; k < slices; k++)
+          for (int q = 0; q < 4; q++) t[q] += __shfl(v[q], lane + k * np, kWave);
+        res = Acc4T<R>{(R)t[0], (R)t[1], (R)t[2], (R)t[3]};
+      }
       mi = pi[0].w;
       idx = lane;
     } else {
@@ -809,7 +863,9 @@ __device__ __forceinline__ void drop_round(int *list, int &cnt) {
 }
 
 template <typename R, bool KAHAN, bool LEARN, bool MONO>
-__global__ __launch_bounds__(kBlock) void k_walk_team(WalkArgs<R> a) {
+__global__ __launch_bounds__(kBlock)
+__attribute__((amdgpu_waves_per_eu(LEARN ? BT_LEARN_WAVES_PER_EU : BT_WALK_WAVES_PER_EU)))
+void k_walk_team(WalkArgs<R> a) {
   typedef TeamShared<R> Sh;
   constexpr int T = kTeam, W = Sh::W, kStack = Sh::kStack;
   __shared__ Sh sh;
@@ -826,16 +882,15 @@ __global__ __launch_bounds__(kBlock) void k_walk_team(WalkArgs<R> a) {
   const int ngroups = a.dc->ngroups;
   if (a.dc->err & (3 | kSortErr)) return;
 
-  // the block's groups: a fixed stride over its XCD's range (every branch below
-  // is uniform over the block)
-  const int home = (int)(blockIdx.x % kXcd);
-  const int g_end = xcd_lo(ngroups, home + 1);
-  for (int g = xcd_lo(ngroups, home) + (int)(blockIdx.x / kXcd); g < g_end;
-       g += xcd_blocks(home)) {
+  // the block's groups: a fixed stride over all of them, so that the groups of a
+  // dense region, neighbours in PH order with the longest lists, go to all XCDs (a
+  // small system's tree fits every L2).  Every branch below is uniform over the block.
+  for (int g = (int)blockIdx.x; g < ngroups; g += (int)gridDim.x) {
     const int2 grp = a.groups[g];
     const int pbeg = grp.x, np = max(grp.y, 1);
     const int sys = a.nsys > 1 ? a.group_sys[g] : 0;
-    const V4<R> pi = a.pos_ph[pbeg + min(lane, np - 1)];
+    const int slices = group_slices(np);
+    const V4<R> pi = a.pos_ph[pbeg + (slices > 1 ? lane % np : min(lane, np - 1))];
     const R mnx = wave_min_r(pi.x), mny = wave_min_r(pi.y), mnz = wave_min_r(pi.z);
     const R mxx = wave_max_r(pi.x), mxy = wave_max_r(pi.y), mxz = wave_max_r(pi.z);
     R gcx, gcy, gcz, gsx, gsy, gsz;
@@ -847,6 +902,9 @@ __global__ __launch_bounds__(kBlock) void k_walk_team(WalkArgs<R> a) {
     GroupGeom geom;
     if constexpr (LEARN) geom = make_group_geom(gcx, gcy, gcz, gsx, gsy, gsz, np, a.sys_scale[sys]);
     IParts<R, 1> ip;
+    ip.slices = slices;
+    ip.slice = min(lane / np, slices - 1);
+    stage_tail(S);
     ip.x[0] = pi.x - gcx;
     ip.y[0] = pi.y - gcy;
     ip.z[0] = pi.z - gcz;
@@ -996,9 +1054,10 @@ __global__ __launch_bounds__(kBlock) void k_walk_team(WalkArgs<R> a) {
     __syncthreads();
     if (wv == 0) {
       double t[4] = {0.0, 0.0, 0.0, 0.0};
-      for (int w = 0; w < T; w++)
-        for (int q = 0; q < 4; q++) t[q] += sh.sum[w][q][lane];
       const bool valid = lane < np;
+      for (int w = 0; w < T; w++)
+        for (int k = 0; k < slices; k++)   // copies of a small group
+          for (int q = 0; q < 4; q++) t[q] += sh.sum[w][q][valid ? lane + k * np : lane];
       const Acc4T<R> res = Acc4T<R>{(R)t[0], (R)t[1], (R)t[2], (R)t[3]};
       a.acc[valid ? pbeg + lane : a.n + lane] = make_v4<R>(res.x, res.y, res.z, res.w);
       const double gp = wave_sum(valid ? (double)pi.w * (double)res.w : 0.0);
@@ -1139,15 +1198,13 @@ WalkArgs<R> walk_args(Ctx &c, const int *run_if) {
 constexpr int kSafeStack = 8 + kMaxLevel * 448;
 
 // Whether the blocks walk groups as teams: below the sizes at which one wave per
-// group fills the chip.  Walk times on Plummer spheres (theta 0.5), one wave per
-// group / teams: 2^10 509 / 45 us, 2^16 753 / 416, 2^18 1187 / 1286; learned angle
-// 2^17 660 / 590, 2^18 868 / 984.  Up to 0.45 ms of the former is its queue: most of
-// its 8192 waves find no group and add to all eight heads; with the groups handed
-// out without a queue it takes 77, 586 and 1283 us.  FP64 (without a queue): 2^14
-// 422 / 282, 2^16 1062 / 779, 2^17 1478 / 1325.  Teams of 2: 215 us at 2^14, of 4:
-// 170, of 8: 185.
+// group fills the chip evenly.  Walk times on Plummer spheres (theta 0.5), one wave
+// per group / teams: 2^10 509 / 44 us, 2^16 753 / 267, 2^18 1060 / 881, 2^19 1789 /
+// 1684, 2^20 3112 / 3398; learned angle 2^18 845 / 613, 2^19 1186 / 1141, 2^20 1910 /
+// 2072; FP64 2^18 1816 / 1659, 2^19 3426 / 3150.  (Teams of 2 and 8 waves were
+// slower than of 4; with the groups cut into one range per XCD 2^16 took 407 us.)
 bool walk_as_team(const Ctx &c) {
-  return c.n <= 1 << 17 && c.walk_variant == 0 && c.blocks_per_cu == 0 &&
+  return c.n <= 1 << 19 && c.walk_variant == 0 && c.blocks_per_cu == 0 &&
          c.lds_stack == kLdsStack && c.stack_ints >= kSafeStack;
 }
 
