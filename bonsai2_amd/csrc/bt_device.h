@@ -161,6 +161,34 @@ __device__ __forceinline__ int system_of(int i, int nsys, const int *__restrict_
   return lo;
 }
 
+// The place of pair i among pairs sorted by all but the low `low` bits of their keys
+// (stably, and within systems): pairs that agree in the sorted bits form short runs,
+// in which a pair's place is the number of smaller keys, ties in their order.  A run
+// of more than kRunMax pairs is not looked through: `ok` is cleared.
+constexpr int kRunMax = 64;
+template <bool FOREST>
+__device__ __forceinline__ int place_in_run(int i, int n, int low, const uint64_t *keys,
+                                            const int *vals, int nsys, const int *off,
+                                            uint64_t key, bool &ok) {
+  int place = i, seen = 0;
+  const int sys = FOREST ? system_of(vals[i], nsys, off) : 0;
+  for (int k = i - 1; k >= 0; k--) {
+    const uint64_t x = keys[k];
+    if ((x ^ key) >> low) break;
+    if (FOREST && system_of(vals[k], nsys, off) != sys) break;
+    place -= x > key ? 1 : 0;
+    if (++seen >= kRunMax) { ok = false; break; }
+  }
+  for (int k = i + 1; k < n; k++) {
+    const uint64_t x = keys[k];
+    if ((x ^ key) >> low) break;
+    if (FOREST && system_of(vals[k], nsys, off) != sys) break;
+    place += x < key ? 1 : 0;
+    if (++seen >= kRunMax) { ok = false; break; }
+  }
+  return place;
+}
+
 // CellData bit layout (reference code/Treecode.h:45-89):
 //   x = parent | level << 27; y = first | (nchild-1) << 29, or 0xFFFFFFFF for
 //   a leaf; z = pbeg; w = pend (half-open, tree order).

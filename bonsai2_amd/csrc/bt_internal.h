@@ -11,6 +11,12 @@
 namespace bt {
 
 constexpr int kSortErr = 8;   // DevCounters::err bit: a sort pass's look-back wait timed out
+// DevCounters::err bits: the tree's or the groups' keys held a run of equal leading
+// digits too long to be put in order after a short sort (radix_sort_pairs).  The
+// phases that follow do nothing; the host sorts again, with every digit, and the
+// context keeps to that (Ctx::full_sort).
+constexpr int kShortTree = 16, kShortPh = 32;
+constexpr int kShortErr = kShortTree | kShortPh;
 constexpr int kLevels = 32;   // level table slots (reference int2[32], code/Treecode.h:171)
 constexpr int kFp64Levels = 4;     // cells at levels <= this combine moments in FP64
 
@@ -48,7 +54,8 @@ struct DevCounters {
   int nnodes, nleaves, nlevels, ncells;
   int ngroups;
   int flags;   // BT_FLAG_*
-  int err;     // 1 = cell capacity, 2 = group capacity, 4 = walk stack, 8 = sort
+  int err;     // 1 = cell capacity, 2 = group capacity, 4 = walk stack, 8 = sort,
+               // 16, 32 = short sort (kShortTree, kShortPh)
   int queue;   // walk group queue head
   int stack_max;  // deepest walk stack of the last walk (entries)
   int xq[8];      // walk group queues, one per XCD range
@@ -73,7 +80,7 @@ struct GraphKey {
   double dt, eps, theta;
   int nleaf, level_split, ncrit;
   int opening, kahan, quadrupole, walk_variant, stack_ints, blocks_per_cu, lds_stack, group_mode;
-  int overlap;
+  int overlap, full_sort;
   float learn_shift, learn_theta_lo, learn_theta_hi;
   int check_ns;
   float check_p99;
@@ -114,6 +121,11 @@ struct Ctx {
   int *sort_ctr = nullptr;          // 2 tile counters
   int sort_tiles_cap = 0;
   bool sort_onesweep = false;
+  bool full_sort = false;   // sort by every digit (a short sort met too long a run)
+  // low key bits the last sort left unsorted (the sorted pairs are then in keyB and
+  // valB, and the gather that follows puts them in order)
+  int geo_low = 0, ph_low = 0;
+  bool ids_in_order = false;   // id[k] = k: no gather since the particles were set
   uint64_t *geo_keys = nullptr;   // sorted geometric keys (tree order)
 
   // scans
@@ -252,8 +264,11 @@ int cell_tiles(int n);   // c.cell_cnt holds kCellCntRows ints per tile
 constexpr int kCellCntRows = 22;
 void launch_multipoles(Ctx &c);
 
-void radix_sort_pairs(Ctx &c, uint64_t *keys, int *vals, uint64_t *keys_tmp, int *vals_tmp,
-                      int n, int key_bits, bool by_system_after);
+// Sorts (keys, vals) by the low key_bits bits, or, if short_ok, possibly by fewer of
+// the leading ones: returns the number of low bits left unsorted, the pairs then in
+// keys_tmp and vals_tmp (0: sorted, in keys and vals).
+int radix_sort_pairs(Ctx &c, uint64_t *keys, int *vals, uint64_t *keys_tmp, int *vals_tmp,
+                     int n, int key_bits, bool by_system_after, bool short_ok);
 void scan_exclusive_sum(Ctx &c, const int *in, int *out, int n, int *total_dev);
 void fill_int(Ctx &c, int *p, int value, int n);
 

@@ -179,7 +179,7 @@ void phase_sort(Ctx &c) {
   launch_bbox(c);
   launch_geo_keys(c);
   record(c, 1);
-  radix_sort_pairs(c, c.geo_keys, c.valA, c.keyB, c.valB, c.n, 63, true);
+  c.geo_low = radix_sort_pairs(c, c.geo_keys, c.valA, c.keyB, c.valB, c.n, 63, true, true);
   record(c, 2);
   launch_gather_tree(c);
 }
@@ -213,7 +213,9 @@ int phase_groups(Ctx &c, int end_ev = 7) {
   }
   launch_ph_keys(c);
   record(c, 5);
-  radix_sort_pairs(c, c.ph_keys, c.perm, c.keyB, c.valB, c.n, 63, true);
+  // the group runs compare the top level_split digits: a short sort has 13 in order
+  c.ph_low = radix_sort_pairs(c, c.ph_keys, c.perm, c.keyB, c.valB, c.n, 63, true,
+                              c.level_split <= 13);
   record(c, 6);
   launch_groups(c);
   record(c, end_ev);
@@ -366,6 +368,10 @@ int regrow_cells(Ctx &c) {
 int build_checked(Ctx &c) {
   if (phase_build(c)) return BT_ERR_HIP;
   if (read_counters(c)) return BT_ERR_HIP;
+  if (c.hc.err & kShortTree) {   // the particles as gathered, by every digit
+    c.full_sort = true;
+    if (phase_build(c) || read_counters(c)) return BT_ERR_HIP;
+  }
   if (c.hc.err & kSortErr) return fail(c, BT_ERR_HIP, kSortErrMsg);
   if (c.hc.err & 1) {
     const int rc = regrow_cells(c);
@@ -394,16 +400,28 @@ int step_second_half(Ctx &c, double dt) {
   return 0;
 }
 
-// After the queued second half of a step: on a cell-capacity failure (the
-// walk and the closing kick were skipped, the particles hold the step's first
-// half kick and drift) grow the cells once and run the second half again.
+// What a step's second half may fail with and be run again after (the walk and the
+// closing kick were skipped, the particles hold the step's first half kick and drift
+// in some tree order): cell capacity, and a short sort that met too long a run.
+bool can_redo(const Ctx &c) { return c.hc.err_sticky && !(c.hc.err_sticky & ~(1 | kShortErr)); }
+
+// Grows the cells, or goes over to sorts by every digit, and runs it again.
+int redo_second_half(Ctx &c, double dt) {
+  if (c.hc.err_sticky & kShortErr) c.full_sort = true;
+  if (c.hc.err_sticky & 1) {
+    const int rc = regrow_cells(c);
+    if (rc) return rc;
+  }
+  launch_clear_sticky(c);
+  return step_second_half(c, dt);
+}
+
+// After the queued second half of a step.  (Sorted by every digit, the tree may
+// still outgrow its cells: two failures in a row at most.)
 int finish_step(Ctx &c, double dt) {
   if (read_counters(c)) return BT_ERR_HIP;
-  if (c.hc.err_sticky == 1) {
-    int rc = regrow_cells(c);
-    if (rc) return rc;
-    launch_clear_sticky(c);
-    rc = step_second_half(c, dt);
+  for (int k = 0; k < 2 && can_redo(c); k++) {
+    const int rc = redo_second_half(c, dt);
     if (rc) return rc;
     if (read_counters(c)) return BT_ERR_HIP;
   }
@@ -693,6 +711,8 @@ int bt_alloc(bt_ctx *h, int n, int nsys, const int *offsets) {
   c.n = n;
   c.nsys = nsys;
   c.h_off = off;
+  c.full_sort = false;
+  c.ids_in_order = false;
   c.max_sys_n = 0;
   for (int k = 0; k < nsys; k++) c.max_sys_n = std::max(c.max_sys_n, off[k + 1] - off[k]);
   if (regrow) {
@@ -744,6 +764,7 @@ int put_particles(Ctx &c, const void *pos4, const void *vel4, hipMemcpyKind kind
   BT_CK(hipMemcpyAsync(c.vel, vel4, bytes, kind, c.stream));
   launch_iota(c, c.n, c.id);
   BT_CK(hipGetLastError());   // (the text of an earlier call's error is no failure here)
+  c.ids_in_order = true;
   BT_CK(hipStreamSynchronize(c.stream));
   c.have_particles = true;
   c.pending_kick = 0.0;
@@ -812,6 +833,10 @@ int bt_make_groups(bt_ctx *h, int level_split, int ncrit) {
   record(c, 4);
   if (phase_groups(c)) return BT_ERR_HIP;
   if (read_counters(c)) return BT_ERR_HIP;
+  if (c.hc.err & kShortPh) {
+    c.full_sort = true;
+    if (phase_groups(c) || read_counters(c)) return BT_ERR_HIP;
+  }
   if (c.hc.err & kSortErr) return fail(c, BT_ERR_HIP, kSortErrMsg);
   if (c.hc.err & 2) return fail(c, BT_ERR_CAPACITY, kGroupCapacityMsg);
   c.have_groups = true;
@@ -1611,6 +1636,7 @@ int bt_step_graph(bt_ctx *h, float dt, int nleaf, int level_split, int ncrit, in
   key.lds_stack = c.lds_stack;
   key.group_mode = c.group_mode;
   key.overlap = c.overlap;
+  key.full_sort = c.full_sort;
   if (c.opening == 1) {
     key.learn_shift = c.learn_shift;
     key.learn_theta_lo = c.learn_theta_lo;
@@ -1667,15 +1693,12 @@ int bt_step_graph(bt_ctx *h, float dt, int nleaf, int level_split, int ncrit, in
   }
   if (read_counters(c)) return BT_ERR_HIP;
   c.have_tree = c.have_mp = c.have_groups = c.have_acc = false;
-  if (c.hc.err_sticky == 1) {
-    // cell capacity: steps_done steps completed, the next one stopped after
-    // its drift; grow the cells, finish that step, run the rest eagerly
+  if (can_redo(c)) {
+    // cell capacity or a short sort: steps_done steps completed, the next one stopped
+    // after its drift; finish that step with larger cells or full sorts, run the rest
+    // eagerly
     const int done = c.hc.steps_done;
-    int rc = regrow_cells(c);
-    if (!rc) {
-      launch_clear_sticky(c);
-      rc = step_second_half(c, dt);
-    }
+    int rc = redo_second_half(c, dt);
     if (!rc) rc = finish_step(c, dt);
     if (rc) return rc;
     c.have_tree = c.have_mp = c.have_groups = c.have_acc = true;

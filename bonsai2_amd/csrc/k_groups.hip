@@ -52,8 +52,9 @@ __global__ __launch_bounds__(kBlock) void k_ph_keys(int n, int nsys, const int *
                                                     const V4<R> *__restrict__ box,
                                                     const V4<R> *__restrict__ pos,
                                                     uint64_t *__restrict__ keys,
-                                                    int *__restrict__ vals) {
+                                                    int *__restrict__ vals, DevCounters *dc) {
   BT_BUILD_PRIO();
+  if (blockIdx.x == 0 && threadIdx.x == 0) atomicAnd(&dc->err, ~kShortPh);
   for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
     const int r = nsys > 1 ? system_of(i, nsys, off) : 0;
     const V4<R> b = box[r];
@@ -93,8 +94,13 @@ constexpr int kScanThreads = 1024, kScanPer = 4;
 struct GroupArgs {
   int n, nsys, ncrit, ntiles, cap;
   const int *off;
-  const uint64_t *keys;
+  const uint64_t *keys;   // in order as far as the mask goes
   uint64_t mask;
+  // a short sort's pairs and where they go (low = 0: keys and perm are final)
+  int low;
+  const int *perm;
+  uint64_t *sorted_keys;
+  int *sorted_perm;
   int *count;      // groups of each tile, then their prefixes
   int *carry;      // start of the run each tile begins in
   int2 *groups;
@@ -172,8 +178,7 @@ __device__ __forceinline__ bool begins_group(const GroupArgs &a, int t0, int k,
 }
 
 template <typename T, bool FOREST>
-__global__ __launch_bounds__(kBlock) void k_gather_count(GroupArgs a, const int *__restrict__ perm,
-                                                         const T *__restrict__ pos,
+__global__ __launch_bounds__(kBlock) void k_gather_count(GroupArgs a, const T *__restrict__ pos,
                                                          const int *__restrict__ id,
                                                          T *__restrict__ pos_ph,
                                                          int *__restrict__ id_ph) {
@@ -185,9 +190,22 @@ __global__ __launch_bounds__(kBlock) void k_gather_count(GroupArgs a, const int 
   for (int r = 0; r < kGroupTile / kBlock; r++) {
     const int i = t0 + r * kBlock + threadIdx.x;
     if (i < a.n) {
-      const int j = perm[i];
-      pos_ph[i] = pos[j];
-      id_ph[i] = id[j];
+      const int j = a.perm[i];
+      int dst = i;
+      if (a.low > 0) {
+        const uint64_t key = a.keys[i];
+        bool ok = true;
+        dst = place_in_run<FOREST>(i, a.n, a.low, a.keys, a.perm, a.nsys, a.off, key, ok);
+        if (!ok) {
+          atomicOr(&a.dc->err, kShortPh);
+          atomicOr(&a.dc->err_sticky, kShortPh);
+          dst = i;   // any order: the walk does nothing
+        }
+        a.sorted_keys[dst] = key;
+        a.sorted_perm[dst] = j;
+      }
+      pos_ph[dst] = pos[j];
+      id_ph[dst] = id[j];
     }
   }
   const int carry = find_run_start<FOREST>(a, t0);
@@ -322,10 +340,10 @@ void launch_ph_keys(Ctx &c) {
   const dim3 g(grid_for(c.n, kBlock, 8192));
   if (c.fp64)
     hipLaunchKernelGGL(k_ph_keys<double>, g, dim3(kBlock), 0, c.stream, c.n, c.nsys, c.d_off,
-                       as4<double>(c.box), as4<double>(c.pos), c.ph_keys, c.perm);
+                       as4<double>(c.box), as4<double>(c.pos), c.ph_keys, c.perm, c.dc);
   else
     hipLaunchKernelGGL(k_ph_keys<float>, g, dim3(kBlock), 0, c.stream, c.n, c.nsys, c.d_off, c.box,
-                       c.pos, c.ph_keys, c.perm);
+                       c.pos, c.ph_keys, c.perm, c.dc);
 }
 
 // A new set of groups starts without the group error bit.
@@ -408,7 +426,11 @@ void launch_groups(Ctx &c) {
   a.ntiles = (c.n + kGroupTile - 1) / kGroupTile;
   a.cap = c.cap_groups;
   a.off = c.d_off;
-  a.keys = c.ph_keys;
+  a.low = c.ph_low;
+  a.keys = a.low > 0 ? c.keyB : c.ph_keys;
+  a.perm = a.low > 0 ? c.valB : c.perm;
+  a.sorted_keys = c.ph_keys;
+  a.sorted_perm = c.perm;
   a.mask = 0;  // top ls octal digits of the 63-bit key (code/makeGroups.cu:259-266)
   for (int i = 0; i < 21; i++) {
     a.mask <<= 3;
@@ -423,11 +445,11 @@ void launch_groups(Ctx &c) {
   const bool forest = c.nsys > 1;
   if (c.fp64) {
     auto kern = forest ? k_gather_count<double4, true> : k_gather_count<double4, false>;
-    hipLaunchKernelGGL(kern, tiles, dim3(kBlock), 0, c.stream, a, c.perm, as4<double>(c.pos), c.id,
+    hipLaunchKernelGGL(kern, tiles, dim3(kBlock), 0, c.stream, a, as4<double>(c.pos), c.id,
                        as4<double>(c.pos_ph), c.id_ph);
   } else {
     auto kern = forest ? k_gather_count<float4, true> : k_gather_count<float4, false>;
-    hipLaunchKernelGGL(kern, tiles, dim3(kBlock), 0, c.stream, a, c.perm, c.pos, c.id, c.pos_ph,
+    hipLaunchKernelGGL(kern, tiles, dim3(kBlock), 0, c.stream, a, c.pos, c.id, c.pos_ph,
                        c.id_ph);
   }
   hipLaunchKernelGGL(k_group_scan, dim3(1), dim3(kScanThreads), 0, c.stream, a);

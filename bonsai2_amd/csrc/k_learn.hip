@@ -603,6 +603,11 @@ __global__ __launch_bounds__(1024) void k_learn_check(int ns, const int *__restr
       __syncthreads();
     }
   }
+  // forces of a walk that did not run (a failed build, to be done again) are not judged
+  if (t == 0 && (dc->err & (3 | kSortErr | kShortErr))) {
+    dc->fallback = 0;
+    return;
+  }
   if (t == 0 && ns > 0) {
     const double p99 = e[(int)(0.99 * (ns - 1))];
     out[0] = e[(ns - 1) / 2];

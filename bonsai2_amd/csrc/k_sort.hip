@@ -768,9 +768,16 @@ void scan_exclusive_sum(Ctx &c, const int *in, int *out, int n, int *total_dev) 
 // by_system_after is set, one or two more stable passes order by the system
 // of each value (systems of a forest stay contiguous).  The result is left in
 // keys/vals; keys_tmp/vals_tmp are scratch of the same size.
-void radix_sort_pairs(Ctx &c, uint64_t *keys, int *vals, uint64_t *keys_tmp, int *vals_tmp,
-                      int n, int key_bits, bool by_system_after) {
-  if (n <= 1) return;
+//
+// short_ok: the passes over the lowest digits may be left out.  40 bits, 13 octal
+// digits, tell almost all particles apart, and the gather that follows every sort
+// puts the runs of the others in order on its way (place_in_run), reading 8 B per
+// pair more instead of 32 B in each of three passes.  5 or 6 passes, so that with
+// the systems' the number is odd and the pairs end in keys_tmp.  2*10^7 pairs: the
+// passes 1.59 -> 0.97 ms, the PH gather 0.25 -> 0.39 ms, the tree gather as before.
+int radix_sort_pairs(Ctx &c, uint64_t *keys, int *vals, uint64_t *keys_tmp, int *vals_tmp,
+                     int n, int key_bits, bool by_system_after, bool short_ok) {
+  if (n <= 1) return 0;
   const int nblocks = (n + kSortTile - 1) / kSortTile;
   // One system, few tiles, whole keys below the all-ones pad
   if (nblocks <= kSmallTiles && !(by_system_after && c.nsys > 1) && key_bits < 64 &&
@@ -781,7 +788,7 @@ void radix_sort_pairs(Ctx &c, uint64_t *keys, int *vals, uint64_t *keys_tmp, int
     if (!one)
       hipLaunchKernelGGL(k_tile_merge, dim3((n + 255) / 256), dim3(256), 0, c.stream, keys_tmp,
                          vals_tmp, n, keys, vals);
-    return;
+    return 0;
   }
   const int hist_n = 256 * nblocks;
   if (hist_n > c.sort_hist_cap) {
@@ -791,17 +798,18 @@ void radix_sort_pairs(Ctx &c, uint64_t *keys, int *vals, uint64_t *keys_tmp, int
       c.sort_hist = nullptr;
       c.sort_hist_cap = 0;
       c.err = "sort histogram allocation failed";
-      return;
+      return 0;
     }
   }
   struct Pass { int shift, by_sys; };
   std::vector<Pass> passes;
-  for (int s = 0; s < key_bits; s += 8) passes.push_back({s, 0});
-  if (by_system_after && c.nsys > 1) {
-    passes.push_back({0, 1});
-    if (c.nsys > 256) passes.push_back({8, 1});
-    if (c.nsys > 65536) passes.push_back({16, 1});
-  }
+  const int sys_passes = !(by_system_after && c.nsys > 1) ? 0
+                         : c.nsys > 65536 ? 3 : c.nsys > 256 ? 2 : 1;
+  const int digits = sys_passes & 1 ? 6 : 5;   // of a short sort
+  const int low = short_ok && !c.full_sort && !c.sort_onesweep && key_bits > 8 * digits
+                      ? key_bits - 8 * digits : 0;
+  for (int s = low; s < key_bits; s += 8) passes.push_back({s, 0});
+  for (int k = 0; k < sys_passes; k++) passes.push_back({8 * k, 1});
   uint64_t *ks = keys, *kd = keys_tmp;
   int *vs = vals, *vd = vals_tmp;
   if (c.sort_onesweep && (int)passes.size() <= kMaxSortPasses) {
@@ -818,7 +826,7 @@ void radix_sort_pairs(Ctx &c, uint64_t *keys, int *vals, uint64_t *keys_tmp, int
           hipMalloc(&c.sort_status, sizeof(unsigned int) * 2 * 256 * (size_t)ntiles) ||
           hipMalloc(&c.sort_ctr, sizeof(int) * 2)) {
         c.err = "sort scratch allocation failed";
-        return;
+        return 0;
       }
       c.sort_tiles_cap = ntiles;
       hipLaunchKernelGGL(k_sort_clear, dim3(1024), dim3(256), 0, c.stream, c.sort_status,
@@ -868,10 +876,12 @@ void radix_sort_pairs(Ctx &c, uint64_t *keys, int *vals, uint64_t *keys_tmp, int
     std::swap(vs, vd);
   }
   }
+  if (low > 0) return low;
   if (ks != keys) {
     (void)hipMemcpyAsync(keys, ks, sizeof(uint64_t) * n, hipMemcpyDeviceToDevice, c.stream);
     (void)hipMemcpyAsync(vals, vs, sizeof(int) * n, hipMemcpyDeviceToDevice, c.stream);
   }
+  return 0;
 }
 
 }  // namespace bt

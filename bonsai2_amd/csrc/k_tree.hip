@@ -147,8 +147,9 @@ __global__ __launch_bounds__(kBlock) void k_geo_keys(int n, int nsys, const int 
                                                      const V4<R> *__restrict__ box,
                                                      const V4<R> *__restrict__ pos,
                                                      uint64_t *__restrict__ keys,
-                                                     int *__restrict__ vals) {
+                                                     int *__restrict__ vals, DevCounters *dc) {
   BT_BUILD_PRIO();
+  if (blockIdx.x == 0 && threadIdx.x == 0) atomicAnd(&dc->err, ~kShortTree);
   for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
     const int r = nsys > 1 ? system_of(i, nsys, off) : 0;
     const V4<R> b = box[r];
@@ -167,20 +168,40 @@ __global__ __launch_bounds__(kBlock) void k_geo_keys(int n, int nsys, const int 
   }
 }
 
-template <typename T>
+// The particles in the order of their sorted keys.  low > 0: the pairs come from a
+// short sort (keys, perm), and their runs are put in order here; sorted_keys receives
+// the keys.  IDENT: the ids are the particles' places still, so none is read.  Bound
+// by the lines that the permuted reads touch (on a first build, of unordered
+// particles, one per 16 B).
+template <typename T, bool SHORT, bool FOREST, bool IDENT>
 __global__ __launch_bounds__(kBlock) void k_gather3(int n, const int *__restrict__ perm,
                                                     const T *__restrict__ a,
                                                     const T *__restrict__ b,
                                                     const int *__restrict__ c,
                                                     T *__restrict__ a2,
                                                     T *__restrict__ b2,
-                                                    int *__restrict__ c2) {
+                                                    int *__restrict__ c2, int low,
+                                                    const uint64_t *__restrict__ keys,
+                                                    uint64_t *__restrict__ sorted_keys, int nsys,
+                                                    const int *__restrict__ off, DevCounters *dc) {
   BT_BUILD_PRIO();
   for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
     const int j = perm[i];
-    a2[i] = a[j];
-    b2[i] = b[j];
-    c2[i] = c[j];
+    int dst = i;
+    if (SHORT) {
+      const uint64_t key = keys[i];
+      bool ok = true;
+      dst = place_in_run<FOREST>(i, n, low, keys, perm, nsys, off, key, ok);
+      if (!ok) {
+        atomicOr(&dc->err, kShortTree);
+        atomicOr(&dc->err_sticky, kShortTree);
+        dst = i;   // any order: what follows does nothing
+      }
+      sorted_keys[dst] = key;
+    }
+    a2[dst] = a[j];
+    b2[dst] = b[j];
+    c2[dst] = IDENT ? j : c[j];
   }
 }
 
@@ -325,6 +346,10 @@ __global__ __launch_bounds__(kBlock) void k_cells_count(LevelArgs a) {
   __shared__ CellTile T;
   __shared__ int sh[kBlock / kWave][kWave];
   const int t0 = blockIdx.x * kCellTile;
+  if (a.dc->err & kShortTree) {   // keys not in order (set before this launch): no cells
+    if (threadIdx.x < kCellRows) a.cnt[threadIdx.x * a.ntiles + blockIdx.x] = 0;
+    return;
+  }
   load_cell_tile<FOREST>(a, t0, T);
   sh[threadIdx.x >> 6][lane_id()] = wave_cell_counts<FOREST>(a, T, t0);
   __syncthreads();
@@ -388,8 +413,12 @@ __global__ __launch_bounds__(kBlock) void k_cells_emit(LevelArgs a) {
   DevCounters *dc = a.dc;
   const int t0 = blockIdx.x * kCellTile;
   const int lane = lane_id(), w = threadIdx.x >> 6;
-  const bool full = load_cell_tile<FOREST>(a, t0, T);
-  sh[w][lane] = wave_cell_counts<FOREST>(a, T, t0);
+  const bool sorted = !(dc->err & kShortTree);
+  bool full = false;
+  if (sorted) {
+    full = load_cell_tile<FOREST>(a, t0, T);
+    sh[w][lane] = wave_cell_counts<FOREST>(a, T, t0);
+  }
   // lane L: first slot of level L
   const int tot = lane >= 1 && lane <= kMaxLevel ? dc->lvl_total[lane] : 0;
   const int start = wave_incl_scan(tot) - tot;
@@ -415,7 +444,7 @@ __global__ __launch_bounds__(kBlock) void k_cells_emit(LevelArgs a) {
     }
   }
   if (full) atomicOr(&dc->flags, (int)BT_FLAG_DEPTH_CAP);
-  if (!fits) return;
+  if (!fits || !sorted) return;
   __syncthreads();
   // lane L: the next slot of level L for this wave
   int next = lane >= 1 && lane <= kMaxLevel ? start + a.cnt[lane * a.ntiles + blockIdx.x] : 0;
@@ -486,7 +515,7 @@ __device__ __forceinline__ void place_children(const LevelArgs &a, int f, int nc
 __global__ __launch_bounds__(kBlock) void k_cells_place(LevelArgs a) {
   BT_BUILD_PRIO();
   const int nc_all = a.dc->ncells;
-  const bool failed = a.dc->err & 1;
+  const bool failed = a.dc->err & (1 | kShortTree);
   const int stride = gridDim.x * kBlock;
   for (int s = blockIdx.x * kBlock + threadIdx.x; s < nc_all; s += stride) {
     const uint4 r = a.raw[s];
@@ -759,21 +788,37 @@ void launch_geo_keys(Ctx &c) {
   const dim3 g(grid_for(c.n, kBlock, 8192));
   if (c.fp64)
     hipLaunchKernelGGL(k_geo_keys<double>, g, dim3(kBlock), 0, c.stream, c.n, c.nsys, c.d_off,
-                       as4<double>(c.box), as4<double>(c.pos), c.geo_keys, c.valA);
+                       as4<double>(c.box), as4<double>(c.pos), c.geo_keys, c.valA, c.dc);
   else
     hipLaunchKernelGGL(k_geo_keys<float>, g, dim3(kBlock), 0, c.stream, c.n, c.nsys, c.d_off,
-                       c.box, c.pos, c.geo_keys, c.valA);
+                       c.box, c.pos, c.geo_keys, c.valA, c.dc);
 }
+
+namespace {
+
+template <typename T>
+auto gather_kernel(bool is_short, bool forest, bool ident) {
+  if (!is_short) return ident ? k_gather3<T, false, false, true> : k_gather3<T, false, false, false>;
+  if (forest) return ident ? k_gather3<T, true, true, true> : k_gather3<T, true, true, false>;
+  return ident ? k_gather3<T, true, false, true> : k_gather3<T, true, false, false>;
+}
+
+}  // namespace
 
 void launch_gather_tree(Ctx &c) {
   const dim3 g(grid_for(c.n, kBlock, 8192));
+  const bool is_short = c.geo_low > 0, forest = c.nsys > 1;
+  const int *perm = is_short ? c.valB : c.valA;
   if (c.fp64)
-    hipLaunchKernelGGL(k_gather3<double4>, g, dim3(kBlock), 0, c.stream, c.n, c.valA,
-                       as4<double>(c.pos), as4<double>(c.vel), c.id, as4<double>(c.pos2),
-                       as4<double>(c.vel2), c.id2);
+    hipLaunchKernelGGL(gather_kernel<double4>(is_short, forest, c.ids_in_order), g, dim3(kBlock), 0,
+                       c.stream, c.n, perm, as4<double>(c.pos), as4<double>(c.vel), c.id,
+                       as4<double>(c.pos2), as4<double>(c.vel2), c.id2, c.geo_low, c.keyB,
+                       c.geo_keys, c.nsys, c.d_off, c.dc);
   else
-    hipLaunchKernelGGL(k_gather3<float4>, g, dim3(kBlock), 0, c.stream, c.n, c.valA, c.pos,
-                       c.vel, c.id, c.pos2, c.vel2, c.id2);
+    hipLaunchKernelGGL(gather_kernel<float4>(is_short, forest, c.ids_in_order), g, dim3(kBlock), 0,
+                       c.stream, c.n, perm, c.pos, c.vel, c.id, c.pos2, c.vel2, c.id2, c.geo_low,
+                       c.keyB, c.geo_keys, c.nsys, c.d_off, c.dc);
+  c.ids_in_order = false;
   std::swap(c.pos, c.pos2);
   std::swap(c.vel, c.vel2);
   std::swap(c.id, c.id2);

@@ -558,7 +558,7 @@ void k_walk(WalkArgs<R> a) {
   if (a.run_if && *a.run_if == 0) return;   // a fallback walk that is not needed
   const int ngroups = a.dc->ngroups;
   // a failed build (cell or group capacity) leaves placeholder links: do not walk it
-  if (a.dc->err & (3 | kSortErr)) return;
+  if (a.dc->err & (3 | kSortErr | kShortErr)) return;
 
   // The persistent loop has no lane-dependent branches at its ends: two
   // "if (lane == 0)" blocks around the back edge (queue fetch, stats store) are
@@ -880,7 +880,7 @@ void k_walk_team(WalkArgs<R> a) {
   if constexpr (LEARN) net.load(a.mlp, s_mlp);
   if (a.run_if && *a.run_if == 0) return;
   const int ngroups = a.dc->ngroups;
-  if (a.dc->err & (3 | kSortErr)) return;
+  if (a.dc->err & (3 | kSortErr | kShortErr)) return;
 
   // the block's groups: a fixed stride over all of them, so that the groups of a
   // dense region, neighbours in PH order with the longest lists, go to all XCDs (a
