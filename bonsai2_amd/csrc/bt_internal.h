@@ -37,8 +37,7 @@ struct LearnBuffers {
 };
 
 // Device-resident counters of one context (one allocation).
-// Blocks of the walk's statistics reduction; d_wstats holds the 4 results,
-// then 4 words of partials per block.
+// Blocks of the walk's statistics reduction (4 words of partials each).
 constexpr int kWalkStatBlocks = 256;
 
 // FP32 walks: stack entries per wave kept in LDS (bt_set_walk_lds_stack).
@@ -72,6 +71,9 @@ struct DevCounters {
   int err_sticky;
   int stack_hw;
   int steps_done;
+  // of the last walk: direct_sum, direct_max, approx_sum, approx_max, and 1/2 sum m phi
+  unsigned long long wstats[4];
+  double wpot;
 };
 
 // The values captured graphs bake into their kernel arguments: a graph is
@@ -178,12 +180,9 @@ struct Ctx {
   int walk_variant = 0;        // 0: LDS j-data, 1: scalar loads, 2: two i-particles per lane
   int quadrupole = 1;          // 0: monopole-only P2C (the reference without QUADRUPOLE)
   int num_cus = 256;
-  unsigned long long *d_wstats = nullptr;  // direct_sum, direct_max, approx_sum, approx_max
-  // host copy of d_wstats fetched with the device counters; valid until the
-  // next walk is queued
-  unsigned long long h_wstats[4] = {};
-  bool h_wstats_valid = false;
-  double *d_wpot = nullptr;
+  unsigned long long *d_wpart = nullptr;   // partials of the walk's statistics
+  // the walk results in hc are those of the last walk queued
+  bool wstats_valid = false;
 
   // learned opening angle
   float2 *sys_scale = nullptr;   // per system (root half size, total mass)
@@ -218,7 +217,8 @@ struct Ctx {
   int direct_cap = 0;
 
   DevCounters *dc = nullptr;
-  DevCounters hc;
+  DevCounters *pinned_dc = nullptr;   // where read_counters copies them
+  DevCounters hc;                     // as last read
 
   // moveParticles' half kick still owed: the next computeForces closes the
   // kick-drift-kick step with it (0 = none)

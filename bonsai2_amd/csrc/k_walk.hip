@@ -1127,8 +1127,7 @@ __global__ __launch_bounds__(kBlock) void k_walk_stats_part(const int2 *__restri
 }
 
 __global__ __launch_bounds__(kBlock) void k_walk_stats_final(const WStat *__restrict__ part,
-                                                            unsigned long long *out, double *pot,
-                                                            const int *run_if) {
+                                                            DevCounters *dc, const int *run_if) {
   if (run_if && *run_if == 0) return;
   __shared__ WStat sh[kWavesPerBlock];
   WStat v = {0ull, 0ull, 0u, 0u, 0.0};
@@ -1139,8 +1138,8 @@ __global__ __launch_bounds__(kBlock) void k_walk_stats_final(const WStat *__rest
   }
   v = block_stats(v, sh);
   if (threadIdx.x == 0) {
-    out[0] = v.ds; out[1] = v.dm; out[2] = v.as; out[3] = v.am;
-    *pot = 0.5 * v.p;
+    dc->wstats[0] = v.ds; dc->wstats[1] = v.dm; dc->wstats[2] = v.as; dc->wstats[3] = v.am;
+    dc->wpot = 0.5 * v.p;
   }
 }
 
@@ -1241,7 +1240,7 @@ auto double_kernel(bool team) {
 }  // namespace
 
 void launch_walk(Ctx &c, const int *run_if) {
-  c.h_wstats_valid = false;   // d_wstats changes with this walk
+  c.wstats_valid = false;   // they change with this walk
   const bool team = walk_as_team(c);
   const dim3 blocks(c.walk_blocks), threads(kBlock);
   hipLaunchKernelGGL(k_walk_reset, dim3(1), dim3(64), 0, c.stream, c.dc, run_if);
@@ -1253,11 +1252,10 @@ void launch_walk(Ctx &c, const int *run_if) {
     auto kern = c.kahan ? float_kernel_of<true>(c, team) : float_kernel_of<false>(c, team);
     hipLaunchKernelGGL(kern, blocks, threads, 0, c.stream, walk_args<float>(c, run_if));
   }
-  WStat *part = reinterpret_cast<WStat *>(c.d_wstats + 4);
+  WStat *part = reinterpret_cast<WStat *>(c.d_wpart);
   hipLaunchKernelGGL(k_walk_stats_part, dim3(kWalkStatBlocks), dim3(kBlock), 0, c.stream, c.groups,
                      c.gcounts, c.gpot, c.dc, part, run_if);
-  hipLaunchKernelGGL(k_walk_stats_final, dim3(1), dim3(kBlock), 0, c.stream, part, c.d_wstats,
-                     c.d_wpot, run_if);
+  hipLaunchKernelGGL(k_walk_stats_final, dim3(1), dim3(kBlock), 0, c.stream, part, c.dc, run_if);
 }
 
 }  // namespace bt
