@@ -144,7 +144,7 @@ struct Ctx {
   uint4 *cells = nullptr;
   float4 *csize = nullptr, *cmono = nullptr, *cq0 = nullptr;
   float2 *cq1 = nullptr, *cls = nullptr;
-  float4 *cscr = nullptr;      // 6 float4 per cell (bottom-up moments)
+  float4 *cscr = nullptr;      // 5 float4 per cell (bottom-up moments)
   float4 *cwalk = nullptr;     // 3 float4 per cell: walk record (com,M) -7.5(Qxx,Qyy,Qzz,Qxy) (-7.5Qxz,-7.5Qyz,trQ,1.5trQ)
   uint4 *cell_raw = nullptr;   // the cells in octant order, before [nodes][leaves] of each parent
   int *cell_fin = nullptr, *cell_nch = nullptr;  // their final slots and child counts

@@ -102,7 +102,7 @@ int alloc_cells(Ctx &c, int cap) {
   rc |= dev_alloc(c, &c.cq0, n * w);
   rc |= dev_alloc(c, &c.cq1, n * w);
   rc |= dev_alloc(c, &c.cls, n * w);
-  rc |= dev_alloc(c, &c.cscr, n * 6 * w);
+  rc |= dev_alloc(c, &c.cscr, n * 5 * w);
   rc |= dev_alloc(c, &c.cwalk, n * 3 * w);
   rc |= dev_alloc(c, &c.cell_raw, n);
   rc |= dev_alloc(c, &c.cell_fin, n);

@@ -555,6 +555,8 @@ __global__ __launch_bounds__(kBlock) void k_cells_finish(LevelArgs a) {
 
 // ---- bottom-up multipoles -------------------------------------------------
 
+constexpr int kScrVecs = 5;   // vectors of a cell's scratch record
+
 // T: the real type of particles and cell data (float or double).
 template <typename T>
 struct MpArgs {
@@ -562,7 +564,7 @@ struct MpArgs {
   T inv_theta;
   const V4<T> *pos;       // tree order
   const uint4 *cells;
-  V4<T> *scr;             // 6 per cell: (ref,M) (com-ref,-) (Qxx,Qyy,Qzz,Qxy) (Qxz,Qyz,-,-) bmin bmax
+  V4<T> *scr;             // 5 per cell: (ref,M) (com-ref,Qxz) (Qxx,Qyy,Qzz,Qxy) (bmin,Qyz) (bmax,-)
   V4<T> *size, *mono, *q0;
   V2<T> *q1, *ls;
   V4<T> *wrec;            // 3 per cell, the walk's P2C record
@@ -631,13 +633,12 @@ __device__ void write_cell(const MpArgs<T> &a, int c, T rx, T ry, T rz, double M
   a.wrec[3 * (size_t)c + 1] = make_v4<T>(T(-7.5) * fqxx, T(-7.5) * fqyy, T(-7.5) * fqzz, T(-7.5) * (T)qxy);
   a.wrec[3 * (size_t)c + 2] =
       make_v4<T>(T(-7.5) * (T)qxz, T(-7.5) * (T)qyz, tr, T(1.5) * tr);
-  V4<T> *s6 = a.scr + 6 * (size_t)c;
-  scr_store<T, CLIMB>(s6, make_v4<T>(rx, ry, rz, (T)M));
-  scr_store<T, CLIMB>(s6 + 1, make_v4<T>((T)dx, (T)dy, (T)dz, T(0)));
-  scr_store<T, CLIMB>(s6 + 2, make_v4<T>((T)qxx, (T)qyy, (T)qzz, (T)qxy));
-  scr_store<T, CLIMB>(s6 + 3, make_v4<T>((T)qxz, (T)qyz, T(0), T(0)));
-  scr_store<T, CLIMB>(s6 + 4, make_v4<T>(e.nx, e.ny, e.nz, T(0)));
-  scr_store<T, CLIMB>(s6 + 5, make_v4<T>(e.xx, e.xy, e.xz, T(0)));
+  V4<T> *rec = a.scr + kScrVecs * (size_t)c;
+  scr_store<T, CLIMB>(rec, make_v4<T>(rx, ry, rz, (T)M));
+  scr_store<T, CLIMB>(rec + 1, make_v4<T>((T)dx, (T)dy, (T)dz, (T)qxz));
+  scr_store<T, CLIMB>(rec + 2, make_v4<T>((T)qxx, (T)qyy, (T)qzz, (T)qxy));
+  scr_store<T, CLIMB>(rec + 3, make_v4<T>(e.nx, e.ny, e.nz, (T)qyz));
+  scr_store<T, CLIMB>(rec + 4, make_v4<T>(e.xx, e.xy, e.xz, T(0)));
 }
 
 template <typename T, typename R, bool CLIMB>
@@ -660,35 +661,40 @@ __device__ void node_moments(const MpArgs<T> &a, int c, const uint4 cd) {
   Moments<R> m{};
   Ext<T> e = ext_empty<T>();
   const int f = cell_first(cd), nc = cell_nchild(cd);
-  // CLIMB: a child's six vectors are loaded while the one before it is added (with
-  // many waves in flight, in the level launches, that only costs registers)
   struct Child {
-    V4<T> g, d, qa, qb, bmn, bmx;
+    V4<T> g, d, q, bmn, bmx;
   };
   auto load = [&](int k) {
-    const V4<T> *s6 = a.scr + 6 * (size_t)(f + k);
-    return Child{scr_load<T, CLIMB>(s6),     scr_load<T, CLIMB>(s6 + 1), scr_load<T, CLIMB>(s6 + 2),
-                 scr_load<T, CLIMB>(s6 + 3), scr_load<T, CLIMB>(s6 + 4), scr_load<T, CLIMB>(s6 + 5)};
+    const V4<T> *rec = a.scr + kScrVecs * (size_t)(f + k);
+    return Child{scr_load<T, CLIMB>(rec), scr_load<T, CLIMB>(rec + 1), scr_load<T, CLIMB>(rec + 2),
+                 scr_load<T, CLIMB>(rec + 3), scr_load<T, CLIMB>(rec + 4)};
   };
-  Child cur = load(0);
-  const V4<T> r0 = cur.g;   // this node's reference = first child's
-  for (int k = 0; k < nc; k++) {
-    Child nxt;
-    if (CLIMB) nxt = load(min(k + 1, nc - 1));
-    else if (k > 0) cur = load(k);
-    const V4<T> g = cur.g, d = cur.d, qa = cur.qa, qb = cur.qb, bmn = cur.bmn, bmx = cur.bmx;
-    // child com relative to this node's reference: both references lie in the
-    // node's bbox, so their difference is at most l and (near-)exact in T
-    const R ox = R(g.x - r0.x) + R(d.x), oy = R(g.y - r0.y) + R(d.y),
-            oz = R(g.z - r0.z) + R(d.z);
-    const R Mc = R(g.w);
-    m.M += Mc;
-    m.sx += Mc * ox; m.sy += Mc * oy; m.sz += Mc * oz;
-    m.xx += Mc * (R(qa.x) + ox * ox); m.yy += Mc * (R(qa.y) + oy * oy);
-    m.zz += Mc * (R(qa.z) + oz * oz); m.xy += Mc * (R(qa.w) + ox * oy);
-    m.xz += Mc * (R(qb.x) + ox * oz); m.yz += Mc * (R(qb.y) + oy * oz);
-    ext_merge(e, bmn.x, bmn.y, bmn.z, bmx.x, bmx.y, bmx.z);
-    if (CLIMB) cur = nxt;
+  // CLIMB: the records of kBatch children are in flight together (one at a time, with
+  // the next loaded meanwhile, a node cost a latency per child: 57 -> 43 us at 2^16).
+  // With many waves in flight, in the level launches, that only costs registers.
+  constexpr int kBatch = !CLIMB ? 1 : sizeof(T) == 4 ? 8 : 4;
+  V4<T> r0;   // this node's reference = first child's
+  for (int k0 = 0; k0 < nc; k0 += kBatch) {
+    Child child[kBatch];
+#pragma unroll
+    for (int q = 0; q < kBatch; q++) child[q] = load(min(k0 + q, nc - 1));
+    if (k0 == 0) r0 = child[0].g;
+#pragma unroll
+    for (int q = 0; q < kBatch; q++) {
+      if (k0 + q >= nc) break;
+      const Child &ch = child[q];
+      // child com relative to this node's reference: both references lie in the
+      // node's bbox, so their difference is at most l and (near-)exact in T
+      const R ox = R(ch.g.x - r0.x) + R(ch.d.x), oy = R(ch.g.y - r0.y) + R(ch.d.y),
+              oz = R(ch.g.z - r0.z) + R(ch.d.z);
+      const R Mc = R(ch.g.w);
+      m.M += Mc;
+      m.sx += Mc * ox; m.sy += Mc * oy; m.sz += Mc * oz;
+      m.xx += Mc * (R(ch.q.x) + ox * ox); m.yy += Mc * (R(ch.q.y) + oy * oy);
+      m.zz += Mc * (R(ch.q.z) + oz * oz); m.xy += Mc * (R(ch.q.w) + ox * oy);
+      m.xz += Mc * (R(ch.d.w) + ox * oz); m.yz += Mc * (R(ch.bmn.w) + oy * oz);
+      ext_merge(e, ch.bmn.x, ch.bmn.y, ch.bmn.z, ch.bmx.x, ch.bmx.y, ch.bmx.z);
+    }
   }
   finish_moments<T, R, CLIMB>(a, c, r0.x, r0.y, r0.z, m, e);
 }
@@ -709,14 +715,17 @@ __device__ __forceinline__ void leaf_moments(const MpArgs<T> &a, int c, const ui
     m.xx += w * dx * dx; m.yy += w * dy * dy; m.zz += w * dz * dz;
     m.xy += w * dx * dy; m.xz += w * dx * dz; m.yz += w * dy * dz;
   };
-  // particles in order, four loads issued together
+  // particles in order, the loads of kBatch issued together; CLIMB: those past the end
+  // too (of the last particle), as few waves hide a remainder's latencies
+  constexpr int kBatch = !CLIMB ? 4 : sizeof(T) == 4 ? 16 : 8;
   int i = pb;
-  for (; i + 4 <= pe; i += 4) {
-    const V4<T> p0 = a.pos[i], p1 = a.pos[i + 1], p2 = a.pos[i + 2], p3 = a.pos[i + 3];
-    add(p0);
-    add(p1);
-    add(p2);
-    add(p3);
+  for (; CLIMB ? i < pe : i + kBatch <= pe; i += kBatch) {
+    V4<T> p[kBatch];
+#pragma unroll
+    for (int q = 0; q < kBatch; q++) p[q] = a.pos[CLIMB ? min(i + q, pe - 1) : i + q];
+#pragma unroll
+    for (int q = 0; q < kBatch; q++)
+      if (!CLIMB || i + q < pe) add(p[q]);
   }
   for (; i < pe; i++) add(a.pos[i]);
   finish_moments<T, T, CLIMB>(a, c, r0.x, r0.y, r0.z, m, e);
