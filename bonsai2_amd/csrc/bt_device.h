@@ -26,6 +26,26 @@ __device__ __forceinline__ uint64_t lanemask_lt() {
   return (1ull << lane_id()) - 1ull;
 }
 
+// Which of the lanes of `peers` have this lane's digit (8 bits), and how many of a
+// mask's lanes come before this one.  In this form a bit takes 4 vector instructions
+// (the sign-extended bit, its ballot, and one three-input operation for each half of
+// the mask), with 64-bit selects it took 9.
+__device__ __forceinline__ uint64_t same_digit(uint64_t peers, int d) {
+  uint32_t lo = (uint32_t)peers, hi = (uint32_t)(peers >> 32);
+#pragma unroll
+  for (int b = 0; b < 8; b++) {
+    const uint32_t s = (uint32_t)((int)((uint32_t)d << (31 - b)) >> 31);
+    const uint64_t m = ballot64(s != 0);
+    lo &= ~((uint32_t)m ^ s);
+    hi &= ~((uint32_t)(m >> 32) ^ s);
+  }
+  return (uint64_t)hi << 32 | lo;
+}
+__device__ __forceinline__ int lanes_before(uint64_t mask) {
+  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                        __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
 // Orders LDS accesses of different lanes of one wave: all lanes' prior LDS
 // writes are visible to all lanes' later LDS reads (a wave executes its LDS
 // instructions in order; this stops the compiler from moving them).

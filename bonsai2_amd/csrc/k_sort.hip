@@ -166,14 +166,8 @@ __global__ __launch_bounds__(kCThreads) void k_radix_scatter(
     const uint64_t key = kk[r];
     const int val = vv[r];
     const int d = valid ? digit_of<BYSYS>(key, val, src) : 0;
-    uint64_t peers = ballot64(valid);
-#pragma unroll
-    for (int b = 0; b < 8; b++) {
-      const bool bit = (d >> b) & 1;
-      const uint64_t m = ballot64(bit);
-      peers &= bit ? m : ~m;
-    }
-    const int rank = __popcll(peers & lanemask_lt());
+    const uint64_t peers = same_digit(ballot64(valid), d);
+    const int rank = lanes_before(peers);
     const int before = wcnt[w][d];
     wave_lds_sync();
     if (valid && rank == 0) wcnt[w][d] = (unsigned short)(before + __popcll(peers));
@@ -362,14 +356,8 @@ __global__ __launch_bounds__(kSortThreads) void k_radix_onesweep(
     const int i = wbase + r * kWave + lane;
     const bool valid = i < n;
     const int d = valid ? digit_of<BYSYS>(kk[r], vv[r], src) : 0;
-    uint64_t peers = ballot64(valid);
-#pragma unroll
-    for (int b = 0; b < 8; b++) {
-      const bool bit = (d >> b) & 1;
-      const uint64_t m = ballot64(bit);
-      peers &= bit ? m : ~m;
-    }
-    const int rank = __popcll(peers & lanemask_lt());
+    const uint64_t peers = same_digit(ballot64(valid), d);
+    const int rank = lanes_before(peers);
     const int before = wcnt[w][d];
     wave_lds_sync();
     if (valid && rank == 0) wcnt[w][d] = before + __popcll(peers);
@@ -593,57 +581,75 @@ void scan_impl(Ctx &c, const int *in, int *out, int n, int *total_dev) {
 
 // ---- small sorts -------------------------------------------------------------
 // Up to kSmallTiles tiles of 4096 pairs take two launches instead of 32: each tile
-// is sorted in LDS by one block (all digits, the ranking of the passes above), then
-// every pair finds its place: its place in its own tile plus, for every other
-// tile, the number of pairs that go before it, by binary searches that do not
-// depend on each other.  Ties go to the earlier tile, so the sort is stable.  Bound
-// by latency (launches, LDS passes, the search's loads from L2).  Tile sort and
-// merge take 32 + 11 us at 2^16 pairs (30 us in all up to one tile), the 32 launches
-// took 163 us and, at 2^10, 117 us plus the gaps between them.  The searches grow
-// with the square of the number of tiles.
+// is sorted in LDS by one block, then every pair finds its place: its place in its own
+// tile plus, for every other tile, the number of pairs that go before it, by binary
+// searches that do not depend on each other.  Ties go to the earlier tile, so the sort
+// is stable.
+//
+// What moves in a tile's passes is a word of 8 bytes, the leading 52 bits of the key
+// and the pair's place in the input; keys and values stay where they were loaded.
+// Passes over the leading 40 bits (32 in smaller tiles) tell almost all keys of a tile
+// apart.  The pairs that agree in them find their places among each other; if more
+// than kRunMax do, the tile is sorted by every digit, from the order that it has.
+//
+// Bound by latency and, on the few CUs that have a tile, by the ranking's vector
+// instructions; the merge by the number of its loads.  Small tiles are cheaper (1024
+// pairs 7.6 us, 2048 12, 4096 20), the searches grow with the square of their number
+// (8 tiles 6 us, 16 tiles 11).  So 1024 pairs up to 8 tiles, 2048 up to 16, and 4096.
+// Sort and merge at 2^10, 10^4, 3*10^4 and 2^16 pairs: 8, 18, 22 and 31 us; with eight
+// passes in tiles of 4096, keys and values moving, 28, 36, 36 and 41; in passes of
+// three launches 117 at 2^10 and 163 at 2^16.  Searches 16 at a time spill; with three
+// probes for two steps the merge at 2^16 took 13 us.
 constexpr int kTileThreads = 1024;
 constexpr int kTileWaves = kTileThreads / kWave;
 constexpr int kTileRounds = kSortTile / kTileThreads;
 constexpr int kSmallTiles = 32;
 
+template <int ROUNDS>
 __global__ __launch_bounds__(kTileThreads) void k_tile_sort(const uint64_t *__restrict__ keys,
                                                             const int *__restrict__ vals, int n,
                                                             int key_bits, uint64_t *keys_out,
                                                             int *vals_out) {
   BT_BUILD_PRIO();
-  __shared__ uint64_t skeys[kSortTile];
-  __shared__ int svals[kSortTile];
-  __shared__ unsigned short wcnt[kTileWaves][256];
-  __shared__ int sh_wave[4];
+  static_assert(ROUNDS <= kTileRounds && kSortTile == 4096, "places of 12 bits");
+  constexpr int kPairs = ROUNDS * kTileThreads;
+  constexpr int kTileLow = ROUNDS == kTileRounds ? 24 : 32;   // bits without a pass
+  __shared__ uint64_t skeys[kPairs], swords[kPairs];
+  __shared__ int svals[kPairs];
+  __shared__ __align__(16) unsigned short wcnt[kTileWaves][256];
+  __shared__ __align__(16) int sh_wave[kTileWaves];
+  __shared__ int sh_long;
   const int tid = threadIdx.x, lane = lane_id();
   const int w = wave_uniform(tid >> 6);
-  const int base = blockIdx.x * kSortTile;
-  const int tile_n = min(kSortTile, n - base);
+  const int base = blockIdx.x * kPairs;
+  const int tile_n = min(kPairs, n - base);
+  if (tid == 0) sh_long = 0;
   // keys have fewer than 64 bits: the pairs past the end, all ones, stay last
-  uint64_t kk[kTileRounds];
-  int vv[kTileRounds];
+  uint64_t ww[ROUNDS];
+  int vv[ROUNDS];
 #pragma unroll
-  for (int r = 0; r < kTileRounds; r++) {
-    const int j = (w * kTileRounds + r) * kWave + lane;
-    kk[r] = j < tile_n ? keys[base + j] : ~0ull;
-    vv[r] = j < tile_n ? vals[base + j] : 0;
+  for (int r = 0; r < ROUNDS; r++) {   // without branches: all loads in flight together
+    const int j = min((w * ROUNDS + r) * kWave + lane, tile_n - 1);
+    ww[r] = keys[base + j];
+    vv[r] = vals[base + j];
   }
-  for (int shift = 0; shift < key_bits; shift += 8) {
-    for (int k = tid; k < kTileWaves * 256 / 2; k += kTileThreads)
-      reinterpret_cast<int *>(&wcnt[0][0])[k] = 0;
-    __syncthreads();
-    int dd[kTileRounds], rr[kTileRounds];
 #pragma unroll
-    for (int r = 0; r < kTileRounds; r++) {
-      const int d = (int)(kk[r] >> shift) & 0xFF;
-      uint64_t peers = ~0ull;
+  for (int r = 0; r < ROUNDS; r++) {
+    const int j = (w * ROUNDS + r) * kWave + lane;
+    const uint64_t key = j < tile_n ? ww[r] : ~0ull;
+    skeys[j] = key;
+    svals[j] = vv[r];
+    ww[r] = ((key << (64 - key_bits)) & ~0xFFFull) | (uint64_t)j;
+  }
+  auto pass = [&](auto digit) {
+    reinterpret_cast<uint64_t *>(wcnt[w])[lane] = 0;   // this wave's counters
+    wave_lds_sync();
+    int dd[ROUNDS], rr[ROUNDS];
 #pragma unroll
-      for (int b = 0; b < 8; b++) {
-        const bool bit = (d >> b) & 1;
-        const uint64_t m = ballot64(bit);
-        peers &= bit ? m : ~m;
-      }
-      const int rank = __popcll(peers & lanemask_lt());
+    for (int r = 0; r < ROUNDS; r++) {
+      const int d = digit(ww[r]);
+      const uint64_t peers = same_digit(~0ull, d);
+      const int rank = lanes_before(peers);
       const int before = wcnt[w][d];
       wave_lds_sync();
       if (rank == 0) wcnt[w][d] = (unsigned short)(before + __popcll(peers));
@@ -652,46 +658,67 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_sort(const uint64_t *__re
       rr[r] = before + rank;
     }
     __syncthreads();
-    // thread d < 256: digit d's first place, then the waves' pairs in tile order
-    int total = 0, incl = 0;
-    if (tid < 256) {
+    // thread 4d + q: digit d in waves 4q to 4q + 3, the order in which places are given
+    int cnt[4], total = 0;
 #pragma unroll
-      for (int k = 0; k < kTileWaves; k++) total += wcnt[k][tid];
-      incl = wave_incl_scan(total);
-      if (lane == kWave - 1) sh_wave[w] = incl;
-    }
+    for (int k = 0; k < 4; k++) total += cnt[k] = wcnt[4 * (tid & 3) + k][tid >> 2];
+    const int incl = wave_incl_scan(total);
+    if (lane == kWave - 1) sh_wave[w] = incl;
     __syncthreads();
-    if (tid < 256) {
-      int acc = incl - total;
-      for (int k = 0; k < w; k++) acc += sh_wave[k];
+    int acc = incl - total;
 #pragma unroll
-      for (int k = 0; k < kTileWaves; k++) {
-        const int c = wcnt[k][tid];
-        wcnt[k][tid] = (unsigned short)acc;
-        acc += c;
-      }
+    for (int k = 0; k < kTileWaves; k++) acc += k < w ? sh_wave[k] : 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      wcnt[4 * (tid & 3) + k][tid >> 2] = (unsigned short)acc;
+      acc += cnt[k];
     }
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < kTileRounds; r++) {
-      const int pos = wcnt[w][dd[r]] + rr[r];
-      skeys[pos] = kk[r];
-      svals[pos] = vv[r];
-    }
+    for (int r = 0; r < ROUNDS; r++) swords[wcnt[w][dd[r]] + rr[r]] = ww[r];
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < kTileRounds; r++) {
-      const int j = (w * kTileRounds + r) * kWave + lane;
-      kk[r] = skeys[j];
-      vv[r] = svals[j];
+    for (int r = 0; r < ROUNDS; r++) ww[r] = swords[(w * ROUNDS + r) * kWave + lane];
+  };
+#pragma unroll 1
+  for (int shift = kTileLow; shift < 64; shift += 8)
+    pass([&](uint64_t word) { return (int)(word >> shift) & 0xFF; });
+  int place[ROUNDS];
+#pragma unroll
+  for (int r = 0; r < ROUNDS; r++) {
+    const int j = (w * ROUNDS + r) * kWave + lane;
+    place[r] = j;
+    if ((int)(ww[r] & 0xFFF) >= tile_n) continue;
+    const uint64_t key = skeys[ww[r] & 0xFFF];
+    int seen = 0;
+    for (int k = j - 1; k >= 0; k--) {
+      const uint64_t x = swords[k];
+      if ((x ^ ww[r]) >> kTileLow) break;
+      place[r] -= skeys[x & 0xFFF] > key ? 1 : 0;
+      if (++seen >= kRunMax) break;
     }
+    for (int k = j + 1; k < tile_n && seen < kRunMax; k++) {
+      const uint64_t x = swords[k];
+      if ((x ^ ww[r]) >> kTileLow) break;
+      place[r] += skeys[x & 0xFFF] < key ? 1 : 0;
+      seen++;
+    }
+    if (seen >= kRunMax) sh_long = 1;
+  }
+  __syncthreads();
+  if (sh_long) {   // by every digit, from this order
+#pragma unroll 1
+    for (int shift = 0; shift < key_bits; shift += 8)
+      pass([&](uint64_t word) { return (int)(skeys[word & 0xFFF] >> shift) & 0xFF; });
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) place[r] = (w * ROUNDS + r) * kWave + lane;
   }
 #pragma unroll
-  for (int r = 0; r < kTileRounds; r++) {
-    const int j = (w * kTileRounds + r) * kWave + lane;
+  for (int r = 0; r < ROUNDS; r++) {
+    const int j = (int)(ww[r] & 0xFFF);
     if (j < tile_n) {
-      keys_out[base + j] = kk[r];
-      vals_out[base + j] = vv[r];
+      keys_out[base + place[r]] = skeys[j];
+      vals_out[base + place[r]] = svals[j];
     }
   }
 }
@@ -700,6 +727,7 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_sort(const uint64_t *__re
 // loads are in flight together.
 constexpr int kTileSearches = 8;
 
+template <int TILE>
 __global__ __launch_bounds__(256) void k_tile_merge(const uint64_t *__restrict__ keys,
                                                     const int *__restrict__ vals, int n,
                                                     uint64_t *__restrict__ keys_out,
@@ -707,22 +735,22 @@ __global__ __launch_bounds__(256) void k_tile_merge(const uint64_t *__restrict__
   BT_BUILD_PRIO();
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
-  const int own = i / kSortTile;   // uniform over the block
-  const int ntiles = (n + kSortTile - 1) / kSortTile;
+  const int own = i / TILE;   // uniform over the block
+  const int ntiles = (n + TILE - 1) / TILE;
   const uint64_t x = keys[i];
-  int place = i - own * kSortTile;
+  int place = i - own * TILE;
   for (int t0 = 0; t0 < ntiles; t0 += kTileSearches) {
     int pos[kTileSearches], len[kTileSearches];
     const uint64_t *tile[kTileSearches];
 #pragma unroll
     for (int q = 0; q < kTileSearches; q++) {
       const int t = t0 + q;
-      tile[q] = keys + (size_t)min(t, ntiles - 1) * kSortTile;
-      len[q] = t < ntiles && t != own ? min(kSortTile, n - t * kSortTile) : 0;
+      tile[q] = keys + (size_t)min(t, ntiles - 1) * TILE;
+      len[q] = t < ntiles && t != own ? min(TILE, n - t * TILE) : 0;
       pos[q] = 0;
     }
 #pragma unroll
-    for (int step = kSortTile; step >= 1; step >>= 1) {
+    for (int step = TILE; step >= 1; step >>= 1) {
 #pragma unroll
       for (int q = 0; q < kTileSearches; q++) {
         // pairs of earlier tiles go before an equal key, those of later ones after
@@ -737,6 +765,19 @@ __global__ __launch_bounds__(256) void k_tile_merge(const uint64_t *__restrict__
   }
   keys_out[place] = x;
   vals_out[place] = vals[i];
+}
+
+template <int ROUNDS>
+void tile_sort_pairs(Ctx &c, uint64_t *keys, int *vals, uint64_t *keys_tmp, int *vals_tmp, int n,
+                     int key_bits) {
+  constexpr int kPairs = ROUNDS * kTileThreads;
+  const int ntiles = (n + kPairs - 1) / kPairs;
+  const bool one = ntiles == 1;
+  hipLaunchKernelGGL(k_tile_sort<ROUNDS>, dim3(ntiles), dim3(kTileThreads), 0, c.stream, keys,
+                     vals, n, key_bits, one ? keys : keys_tmp, one ? vals : vals_tmp);
+  if (!one)
+    hipLaunchKernelGGL(k_tile_merge<kPairs>, dim3((n + 255) / 256), dim3(256), 0, c.stream,
+                       keys_tmp, vals_tmp, n, keys, vals);
 }
 
 template <typename T>
@@ -782,12 +823,12 @@ int radix_sort_pairs(Ctx &c, uint64_t *keys, int *vals, uint64_t *keys_tmp, int 
   // One system, few tiles, whole keys below the all-ones pad
   if (nblocks <= kSmallTiles && !(by_system_after && c.nsys > 1) && key_bits < 64 &&
       !c.sort_onesweep) {
-    const bool one = nblocks == 1;
-    hipLaunchKernelGGL(k_tile_sort, dim3(nblocks), dim3(kTileThreads), 0, c.stream, keys, vals, n,
-                       key_bits, one ? keys : keys_tmp, one ? vals : vals_tmp);
-    if (!one)
-      hipLaunchKernelGGL(k_tile_merge, dim3((n + 255) / 256), dim3(256), 0, c.stream, keys_tmp,
-                         vals_tmp, n, keys, vals);
+    if (n <= 8 * kTileThreads)
+      tile_sort_pairs<1>(c, keys, vals, keys_tmp, vals_tmp, n, key_bits);
+    else if (n <= 16 * 2 * kTileThreads)
+      tile_sort_pairs<2>(c, keys, vals, keys_tmp, vals_tmp, n, key_bits);
+    else
+      tile_sort_pairs<kTileRounds>(c, keys, vals, keys_tmp, vals_tmp, n, key_bits);
     return 0;
   }
   const int hist_n = 256 * nblocks;
