@@ -260,7 +260,7 @@ void launch_bbox(Ctx &c);
 void launch_geo_keys(Ctx &c);
 void launch_gather_tree(Ctx &c);
 void launch_levels(Ctx &c);
-int cell_tiles(int n);   // c.cell_cnt holds kCellCntRows ints per tile
+int max_cell_tiles(int n);   // c.cell_cnt holds kCellCntRows ints per tile
 constexpr int kCellCntRows = 22;
 void launch_multipoles(Ctx &c);
 

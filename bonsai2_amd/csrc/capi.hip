@@ -740,7 +740,7 @@ int bt_alloc(bt_ctx *h, int n, int nsys, const int *offsets) {
     rc |= dev_alloc(c, &c.gcounts, n); rc |= dev_alloc(c, &c.gpot, n);
     rc |= dev_alloc(c, &c.box, (size_t)nsys * w); rc |= dev_alloc(c, &c.root_cells, nsys);
     rc |= dev_alloc(c, &c.sys_scale, nsys);
-    rc |= dev_alloc(c, &c.cell_cnt, (size_t)kCellCntRows * cell_tiles(n));
+    rc |= dev_alloc(c, &c.cell_cnt, (size_t)kCellCntRows * max_cell_tiles(n));
     rc |= dev_alloc(c, &c.d_off, nsys + 1);
     rc |= dev_alloc(c, &c.d_energy, 2 * (size_t)nsys * 65);
     if (rc) return BT_ERR_HIP;

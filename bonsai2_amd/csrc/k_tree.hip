@@ -229,8 +229,12 @@ __global__ __launch_bounds__(kBlock) void k_gather3(int n, const int *__restrict
 // A launch triple per level with binary searches for the children (64 launches)
 // took 0.26 ms at 2^16 and 0.83 ms at 2^24 particles.
 
-constexpr int kCellTile = 1024;                      // particles per block
-constexpr int kCellRounds = kCellTile / kBlock;      // per wave: rounds of 64 in a row
+// Particles per block: ROUNDS rounds of 64 in a row per wave.  Four are worth the
+// window's halo (2 NLEAF keys) and the fewer counts; up to kCellSmall particles, where a
+// round's latency is what a tile costs, one
+// (count and emit: 7 + 14 -> 4.5 + 7 us at 2^10, 9 + 15 -> 5 + 7.5 at 2^16).
+constexpr int kCellRounds = 4;
+constexpr int kCellSmall = 1 << 17;
 constexpr int kCellRows = kCellCntRows;                // row 0: leaves; row L: cells of level L
 static_assert(kCellRows == kMaxLevel + 1, "a row per level and one for the leaves");
 constexpr int kMaxLeaf = 64;
@@ -259,7 +263,9 @@ __device__ __forceinline__ int shared_digits(uint64_t a, uint64_t b) {
 
 // One tile's keys and depths.  Entry j of a window array belongs to particle
 // t0 - 1 - NLEAF + j, entry j of depth to particle t0 - 1 + j.
+template <int ROUNDS>
 struct CellTile {
+  static constexpr int kCellTile = ROUNDS * kBlock;
   uint64_t key[kCellTile + 2 * kMaxLeaf + 2];
   int sys[kCellTile + 2 * kMaxLeaf + 2];   // forest: the particle's system
   unsigned char win[2][kCellTile + kMaxLeaf + 2];
@@ -268,8 +274,9 @@ struct CellTile {
 
 // Fills the tile and returns whether one of its windows shares all digits (a
 // level-21 cell of more than NLEAF particles).
-template <bool FOREST>
-__device__ __forceinline__ bool load_cell_tile(const LevelArgs &a, int t0, CellTile &T) {
+template <bool FOREST, int ROUNDS>
+__device__ __forceinline__ bool load_cell_tile(const LevelArgs &a, int t0, CellTile<ROUNDS> &T) {
+  constexpr int kCellTile = ROUNDS * kBlock;
   const int nl = a.nleaf;
   const int k0 = t0 - 1 - nl;   // particle of entry 0
   for (int j = threadIdx.x; j < kCellTile + 2 * nl + 1; j += kBlock) {
@@ -308,8 +315,8 @@ __device__ __forceinline__ bool load_cell_tile(const LevelArgs &a, int t0, CellT
 
 // c(i) and D(i) of particle i = t0 + j; an index past the last particle begins
 // nothing (c = kMaxLevel) except that i = n ends what the last particle is in.
-template <bool FOREST>
-__device__ __forceinline__ void cell_span(const LevelArgs &a, const CellTile &T, int t0, int j,
+template <bool FOREST, int ROUNDS>
+__device__ __forceinline__ void cell_span(const LevelArgs &a, const CellTile<ROUNDS> &T, int t0, int j,
                                           int &c, int &d, int &dprev) {
   const int i = t0 + j, e = j + a.nleaf + 1;   // e: entry of particle i in the key array
   d = i < a.n ? (int)T.depth[j + 1] : -1;
@@ -320,15 +327,16 @@ __device__ __forceinline__ void cell_span(const LevelArgs &a, const CellTile &T,
 }
 
 // Lane L of the result counts the beginnings of level L among the wave's
-// kCellRounds * 64 particles, lane 0 its leaves.
-template <bool FOREST>
-__device__ __forceinline__ int wave_cell_counts(const LevelArgs &a, const CellTile &T, int t0) {
+// ROUNDS * 64 particles, lane 0 its leaves.
+template <bool FOREST, int ROUNDS>
+__device__ __forceinline__ int wave_cell_counts(const LevelArgs &a, const CellTile<ROUNDS> &T,
+                                                int t0) {
   const int lane = lane_id(), w = threadIdx.x >> 6;
   int cnt = 0;
 #pragma unroll
-  for (int r = 0; r < kCellRounds; r++) {
+  for (int r = 0; r < ROUNDS; r++) {
     int c, d, dp;
-    cell_span<FOREST>(a, T, t0, (w * kCellRounds + r) * kWave + lane, c, d, dp);
+    cell_span<FOREST, ROUNDS>(a, T, t0, (w * ROUNDS + r) * kWave + lane, c, d, dp);
     const int nleaves = __popcll(ballot64(c <= d));   // d >= 0 for every particle
     cnt += lane == 0 ? nleaves : 0;
     const int hi = wave_max_int(d + 1);
@@ -340,18 +348,18 @@ __device__ __forceinline__ int wave_cell_counts(const LevelArgs &a, const CellTi
   return cnt;
 }
 
-template <bool FOREST>
+template <bool FOREST, int ROUNDS>
 __global__ __launch_bounds__(kBlock) void k_cells_count(LevelArgs a) {
   BT_BUILD_PRIO();
-  __shared__ CellTile T;
+  __shared__ CellTile<ROUNDS> T;
   __shared__ int sh[kBlock / kWave][kWave];
-  const int t0 = blockIdx.x * kCellTile;
+  const int t0 = blockIdx.x * (ROUNDS * kBlock);
   if (a.dc->err & kShortTree) {   // keys not in order (set before this launch): no cells
     if (threadIdx.x < kCellRows) a.cnt[threadIdx.x * a.ntiles + blockIdx.x] = 0;
     return;
   }
-  load_cell_tile<FOREST>(a, t0, T);
-  sh[threadIdx.x >> 6][lane_id()] = wave_cell_counts<FOREST>(a, T, t0);
+  load_cell_tile<FOREST, ROUNDS>(a, t0, T);
+  sh[threadIdx.x >> 6][lane_id()] = wave_cell_counts<FOREST, ROUNDS>(a, T, t0);
   __syncthreads();
   if (threadIdx.x < kCellRows) {
     int s = 0;
@@ -405,19 +413,19 @@ __global__ __launch_bounds__(kScanBlock) void k_cells_scan(LevelArgs a) {
 // The cells in octant order.  Level L of the loop: a particle that begins a cell
 // of level L takes the next slot of the level; it writes the cell one level up
 // that begins with it as soon as this one's slot, its first child, is known.
-template <bool FOREST>
+template <bool FOREST, int ROUNDS>
 __global__ __launch_bounds__(kBlock) void k_cells_emit(LevelArgs a) {
   BT_BUILD_PRIO();
-  __shared__ CellTile T;
+  __shared__ CellTile<ROUNDS> T;
   __shared__ int sh[kBlock / kWave][kWave];
   DevCounters *dc = a.dc;
-  const int t0 = blockIdx.x * kCellTile;
+  const int t0 = blockIdx.x * (ROUNDS * kBlock);
   const int lane = lane_id(), w = threadIdx.x >> 6;
   const bool sorted = !(dc->err & kShortTree);
   bool full = false;
   if (sorted) {
-    full = load_cell_tile<FOREST>(a, t0, T);
-    sh[w][lane] = wave_cell_counts<FOREST>(a, T, t0);
+    full = load_cell_tile<FOREST, ROUNDS>(a, t0, T);
+    sh[w][lane] = wave_cell_counts<FOREST, ROUNDS>(a, T, t0);
   }
   // lane L: first slot of level L
   const int tot = lane >= 1 && lane <= kMaxLevel ? dc->lvl_total[lane] : 0;
@@ -449,11 +457,11 @@ __global__ __launch_bounds__(kBlock) void k_cells_emit(LevelArgs a) {
   // lane L: the next slot of level L for this wave
   int next = lane >= 1 && lane <= kMaxLevel ? start + a.cnt[lane * a.ntiles + blockIdx.x] : 0;
   for (int k = 0; k < w; k++) next += lane >= 1 ? sh[k][lane] : 0;
-  for (int r = 0; r < kCellRounds; r++) {
-    const int j = (w * kCellRounds + r) * kWave + lane;
+  for (int r = 0; r < ROUNDS; r++) {
+    const int j = (w * ROUNDS + r) * kWave + lane;
     const int i = t0 + j;
     int c, d, dp;
-    cell_span<FOREST>(a, T, t0, j, c, d, dp);
+    cell_span<FOREST, ROUNDS>(a, T, t0, j, c, d, dp);
     const int hi = wave_max_int(max(d, dp) + 1);
     uint32_t up = 0;       // raw slot of the cell of level L - 1 that holds this particle
     int mine = -1;         // raw slot of the node of level L - 1 that begins here
@@ -833,7 +841,12 @@ void launch_gather_tree(Ctx &c) {
   std::swap(c.id, c.id2);
 }
 
-int cell_tiles(int n) { return n / kCellTile + 1; }   // particle n, past the last, included
+int cell_tiles(int n) {   // particle n, past the last, included
+  return n / (kBlock * (n <= kCellSmall ? 1 : kCellRounds)) + 1;
+}
+
+// the most tiles that any number of particles up to n takes
+int max_cell_tiles(int n) { return std::max(cell_tiles(n), cell_tiles(std::min(n, kCellSmall))); }
 
 void launch_levels(Ctx &c) {
   LevelArgs a;
@@ -855,8 +868,11 @@ void launch_levels(Ctx &c) {
   a.dc = c.dc;
   const dim3 tiles(a.ntiles), cells(grid_for(std::max(c.cap_cells, c.nsys), kBlock, 4096));
   const bool forest = c.nsys > 1;
-  auto count = forest ? k_cells_count<true> : k_cells_count<false>;
-  auto emit = forest ? k_cells_emit<true> : k_cells_emit<false>;
+  const bool small = c.n <= kCellSmall;
+  auto count = small ? (forest ? k_cells_count<true, 1> : k_cells_count<false, 1>)
+                     : (forest ? k_cells_count<true, kCellRounds> : k_cells_count<false, kCellRounds>);
+  auto emit = small ? (forest ? k_cells_emit<true, 1> : k_cells_emit<false, 1>)
+                    : (forest ? k_cells_emit<true, kCellRounds> : k_cells_emit<false, kCellRounds>);
   hipLaunchKernelGGL(count, tiles, dim3(kBlock), 0, c.stream, a);
   hipLaunchKernelGGL(k_cells_scan, dim3(kCellRows), dim3(kScanBlock), 0, c.stream, a);
   hipLaunchKernelGGL(emit, tiles, dim3(kBlock), 0, c.stream, a);
