@@ -76,6 +76,12 @@ struct DevCounters {
   double wpot;
 };
 
+__device__ __forceinline__ void clear_sticky(DevCounters *dc) {
+  dc->err_sticky = 0;
+  dc->stack_hw = 0;
+  dc->steps_done = 0;
+}
+
 // The values captured graphs bake into their kernel arguments: a graph is
 // replayed only while all of them are unchanged (compared bytewise).
 struct GraphKey {
@@ -281,7 +287,7 @@ void launch_leaf_groups(Ctx &c);
 
 // run_if: device flag; the walk (reset, traversal, statistics) does nothing
 // unless it is nonzero (nullptr = always run)
-void launch_walk(Ctx &c, const int *run_if = nullptr);
+void launch_walk(Ctx &c, const int *run_if = nullptr, bool clear = false);
 
 void launch_mlp_prepare(Ctx &c);
 void launch_mlp_forward(Ctx &c, int n, const float *x, float *y);

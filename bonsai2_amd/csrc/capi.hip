@@ -198,7 +198,6 @@ int phase_build(Ctx &c) {
 // end_ev: the event recorded when the phase's work is queued.
 int phase_multipoles(Ctx &c, int end_ev = 4) {
   launch_multipoles(c);
-  if (!c.fp64) launch_sys_scale(c);   // the learned angle's scales (Treecode<float> only)
   record(c, end_ev);
   BT_LAUNCH_CK();
   return 0;
@@ -254,9 +253,10 @@ int phase_tree_and_groups(Ctx &c) {
   return rc_groups ? rc_groups : rc_mp;
 }
 
-int phase_forces(Ctx &c) {
+// clear: the sticky state is cleared with the walk's own (launch_clear_sticky).
+int phase_forces(Ctx &c, bool clear = false) {
   if (ensure_stack(c)) return BT_ERR_HIP;
-  launch_walk(c);
+  launch_walk(c, nullptr, clear);
   record(c, 8);
   BT_LAUNCH_CK();
   return 0;
@@ -855,12 +855,11 @@ int bt_compute_forces(bt_ctx *h, int intcount, double stats[4]) {
   c.err.clear();
   if (!c.have_mp || !c.have_groups)
     return fail(c, BT_ERR_STATE, "computeMultipoles and makeGroups first");
-  launch_clear_sticky(c);
   record(c, 7);
   // the check's sum runs after this walk, from the tree-order particles
   if (join_check(c)) return BT_ERR_HIP;
   c.check_state = 0;
-  if (phase_forces(c) || launch_learned_check(c)) return BT_ERR_HIP;
+  if (phase_forces(c, true) || launch_learned_check(c)) return BT_ERR_HIP;
   // a moveParticles before this evaluation owes its step's closing half kick
   if (c.pending_kick != 0.0) launch_kick(c, c.pending_kick, true);
   BT_LAUNCH_CK();

@@ -679,6 +679,7 @@ static PairArgs pair_args(Ctx &c, LearnBuffers &L) {
 
 
 void launch_learn_pairs(Ctx &c, LearnBuffers &L) {
+  launch_sys_scale(c);
   const PairArgs a = pair_args(c, L);
   hipLaunchKernelGGL(k_learn_pairs, dim3(c.walk_blocks), dim3(kBlock), 0, c.stream, a);
 }

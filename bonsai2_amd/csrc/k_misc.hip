@@ -75,11 +75,7 @@ __global__ __launch_bounds__(kBlock) void k_kick_drift(int n, const int *__restr
 }
 
 __global__ void k_clear_sticky(DevCounters *dc) {
-  if (threadIdx.x == 0) {
-    dc->err_sticky = 0;
-    dc->stack_hw = 0;
-    dc->steps_done = 0;
-  }
+  if (threadIdx.x == 0) clear_sticky(dc);
 }
 
 // dst[idx[k]] = src[k] (SCATTER) or dst[k] = src[idx[k]]: results into the order

@@ -142,17 +142,30 @@ __device__ __forceinline__ void child_step(R &cx, R &cy, R &cz, R &h, int o) {
   h = s;
 }
 
-template <typename R>
+// BOX: one system whose partial boxes are kBoxParts at most: every wave makes the box of
+// them (2^16 particles: 3 + 4 -> 4 us, and a launch gap less).
+constexpr int kBoxParts = kWave;
+template <typename R, bool BOX>
 __global__ __launch_bounds__(kBlock) void k_geo_keys(int n, int nsys, const int *__restrict__ off,
-                                                     const V4<R> *__restrict__ box,
+                                                     V4<R> *__restrict__ box,
+                                                     const V4<R> *__restrict__ part, int nb,
                                                      const V4<R> *__restrict__ pos,
                                                      uint64_t *__restrict__ keys,
                                                      int *__restrict__ vals, DevCounters *dc) {
   BT_BUILD_PRIO();
   if (blockIdx.x == 0 && threadIdx.x == 0) atomicAnd(&dc->err, ~kShortTree);
+  V4<R> own;
+  if constexpr (BOX) {
+    const int k = min(lane_id(), nb - 1);
+    const V4<R> mn = part[2 * k], mx = part[2 * k + 1];
+    const Ext<R> e{wave_min_r(mn.x), wave_min_r(mn.y), wave_min_r(mn.z),
+                   wave_max_r(mx.x), wave_max_r(mx.y), wave_max_r(mx.z)};
+    own = box_from_extent(e);
+    if (blockIdx.x == 0 && threadIdx.x == 0) box[0] = own;
+  }
   for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
     const int r = nsys > 1 ? system_of(i, nsys, off) : 0;
-    const V4<R> b = box[r];
+    const V4<R> b = BOX ? own : box[r];
     const V4<R> p = pos[i];
     R cx = b.x, cy = b.y, cz = b.z, h = b.w;
     uint64_t k = 0;
@@ -786,29 +799,39 @@ __global__ __launch_bounds__(kBlock) void k_multipole_climb(MpArgs<T> a) {
 
 }  // namespace
 
-void launch_bbox(Ctx &c) {
+namespace {
+
+bool box_with_keys(const Ctx &c) { return c.nsys == 1 && c.bbox_blocks <= kBoxParts; }
+
+template <typename R>
+void bbox_t(Ctx &c) {
   const int nb = c.bbox_blocks;
-  if (c.fp64) {
-    hipLaunchKernelGGL(k_bbox_partial<double>, dim3(nb, c.nsys), dim3(kBlock), 0, c.stream,
-                       as4<double>(c.pos), c.d_off, nb, as4<double>(c.bbox_part));
-    hipLaunchKernelGGL(k_bbox_final<double>, dim3(c.nsys), dim3(kBlock), 0, c.stream,
-                       as4<double>(c.bbox_part), nb, as4<double>(c.box));
-  } else {
-    hipLaunchKernelGGL(k_bbox_partial<float>, dim3(nb, c.nsys), dim3(kBlock), 0, c.stream, c.pos,
-                       c.d_off, nb, c.bbox_part);
-    hipLaunchKernelGGL(k_bbox_final<float>, dim3(c.nsys), dim3(kBlock), 0, c.stream, c.bbox_part,
-                       nb, c.box);
-  }
+  hipLaunchKernelGGL(k_bbox_partial<R>, dim3(nb, c.nsys), dim3(kBlock), 0, c.stream, as4<R>(c.pos),
+                     c.d_off, nb, as4<R>(c.bbox_part));
+  if (box_with_keys(c)) return;
+  hipLaunchKernelGGL(k_bbox_final<R>, dim3(c.nsys), dim3(kBlock), 0, c.stream,
+                     as4<R>(c.bbox_part), nb, as4<R>(c.box));
 }
 
+template <typename R>
+void geo_keys_t(Ctx &c) {
+  auto kern = box_with_keys(c) ? k_geo_keys<R, true> : k_geo_keys<R, false>;
+  hipLaunchKernelGGL(kern, dim3(grid_for(c.n, kBlock, 8192)), dim3(kBlock), 0, c.stream, c.n,
+                     c.nsys, c.d_off, as4<R>(c.box), as4<R>(c.bbox_part), c.bbox_blocks,
+                     as4<R>(c.pos), c.geo_keys, c.valA, c.dc);
+}
+
+}  // namespace
+
+void launch_bbox(Ctx &c) {
+  if (c.fp64) bbox_t<double>(c);
+  else bbox_t<float>(c);
+}
+
+// After launch_bbox, which may have left the box to this launch.
 void launch_geo_keys(Ctx &c) {
-  const dim3 g(grid_for(c.n, kBlock, 8192));
-  if (c.fp64)
-    hipLaunchKernelGGL(k_geo_keys<double>, g, dim3(kBlock), 0, c.stream, c.n, c.nsys, c.d_off,
-                       as4<double>(c.box), as4<double>(c.pos), c.geo_keys, c.valA, c.dc);
-  else
-    hipLaunchKernelGGL(k_geo_keys<float>, g, dim3(kBlock), 0, c.stream, c.n, c.nsys, c.d_off,
-                       c.box, c.pos, c.geo_keys, c.valA, c.dc);
+  if (c.fp64) geo_keys_t<double>(c);
+  else geo_keys_t<float>(c);
 }
 
 namespace {

@@ -1073,15 +1073,18 @@ void k_walk_team(WalkArgs<R> a) {
 // Interaction statistics (code/computeForces.cu:567-609, :701-715): per valid
 // i-particle its group's counts; {direct_sum, direct_max, approx_sum,
 // approx_max} and 1/2 sum m phi.  kWalkStatBlocks blocks reduce contiguous
-// group ranges, one block combines their partials: a fixed order, so the
-// FP64 potential sum is the same on every run.
+// group ranges, one block combines their partials; up to kStatSmall particles one block
+// does it all (2^16: 9 -> 5 us).  A fixed order, so the FP64 potential sum is the same on every
+// run.
+constexpr int kStatSmall = 1 << 17;
+constexpr int kStatThreads = 1024;
 struct WStat {
   unsigned long long ds, as;
   unsigned int dm, am;
   double p;
 };
 
-// 256 threads; the block's total in thread 0
+// The block's total in thread 0.
 __device__ __forceinline__ WStat block_stats(WStat v, WStat *sh) {
   v.ds = wave_sum(v.ds);
   v.as = wave_sum(v.as);
@@ -1094,12 +1097,44 @@ __device__ __forceinline__ WStat block_stats(WStat v, WStat *sh) {
   if (lane_id() == 0) sh[w] = v;
   __syncthreads();
   if (threadIdx.x == 0) {
-    for (int k = 1; k < kWavesPerBlock; k++) {
+    for (int k = 1; k < (int)(blockDim.x >> 6); k++) {
       v.ds += sh[k].ds; v.as += sh[k].as; v.p += sh[k].p;
       v.dm = max(v.dm, sh[k].dm); v.am = max(v.am, sh[k].am);
     }
   }
   return v;
+}
+
+// This thread's share of groups [g0, g1).
+__device__ __forceinline__ WStat group_stats(const int2 *__restrict__ groups,
+                                             const int2 *__restrict__ gcounts,
+                                             const double *__restrict__ gpot, int g0, int g1) {
+  WStat v = {0ull, 0ull, 0u, 0u, 0.0};
+  for (int g = g0 + threadIdx.x; g < g1; g += blockDim.x) {
+    const int2 c = gcounts[g];
+    const int np = groups[g].y;
+    v.ds += (unsigned long long)c.y * (unsigned long long)np;
+    v.as += (unsigned long long)c.x * (unsigned long long)np;
+    v.dm = max(v.dm, (unsigned int)c.y);
+    v.am = max(v.am, (unsigned int)c.x);
+    v.p += gpot[g];
+  }
+  return v;
+}
+
+__device__ __forceinline__ void put_stats(DevCounters *dc, const WStat &v) {
+  dc->wstats[0] = v.ds; dc->wstats[1] = v.dm; dc->wstats[2] = v.as; dc->wstats[3] = v.am;
+  dc->wpot = 0.5 * v.p;
+}
+
+__global__ __launch_bounds__(kStatThreads) void k_walk_stats(const int2 *__restrict__ groups,
+                                                             const int2 *__restrict__ gcounts,
+                                                             const double *__restrict__ gpot,
+                                                             DevCounters *dc, const int *run_if) {
+  if (run_if && *run_if == 0) return;
+  __shared__ WStat sh[kStatThreads / kWave];
+  const WStat v = block_stats(group_stats(groups, gcounts, gpot, 0, dc->ngroups), sh);
+  if (threadIdx.x == 0) put_stats(dc, v);
 }
 
 __global__ __launch_bounds__(kBlock) void k_walk_stats_part(const int2 *__restrict__ groups,
@@ -1112,17 +1147,7 @@ __global__ __launch_bounds__(kBlock) void k_walk_stats_part(const int2 *__restri
   const int ng = dc->ngroups;
   const int chunk = (ng + gridDim.x - 1) / gridDim.x;
   const int g0 = blockIdx.x * chunk, g1 = min(ng, g0 + chunk);
-  WStat v = {0ull, 0ull, 0u, 0u, 0.0};
-  for (int g = g0 + threadIdx.x; g < g1; g += kBlock) {
-    const int2 c = gcounts[g];
-    const int np = groups[g].y;
-    v.ds += (unsigned long long)c.y * (unsigned long long)np;
-    v.as += (unsigned long long)c.x * (unsigned long long)np;
-    v.dm = max(v.dm, (unsigned int)c.y);
-    v.am = max(v.am, (unsigned int)c.x);
-    v.p += gpot[g];
-  }
-  v = block_stats(v, sh);
+  const WStat v = block_stats(group_stats(groups, gcounts, gpot, g0, g1), sh);
   if (threadIdx.x == 0) part[blockIdx.x] = v;
 }
 
@@ -1137,18 +1162,17 @@ __global__ __launch_bounds__(kBlock) void k_walk_stats_final(const WStat *__rest
     v.dm = max(v.dm, q.dm); v.am = max(v.am, q.am);
   }
   v = block_stats(v, sh);
-  if (threadIdx.x == 0) {
-    dc->wstats[0] = v.ds; dc->wstats[1] = v.dm; dc->wstats[2] = v.as; dc->wstats[3] = v.am;
-    dc->wpot = 0.5 * v.p;
-  }
+  if (threadIdx.x == 0) put_stats(dc, v);
 }
 
-__global__ void k_walk_reset(DevCounters *dc, const int *run_if) {
+// clear: the sticky state too, where the walk is the first launch of an API call.
+__global__ void k_walk_reset(DevCounters *dc, const int *run_if, bool clear) {
   if (threadIdx.x == 0 && !(run_if && *run_if == 0)) {
     dc->queue = 0;
     dc->stack_max = 0;
     for (int x = 0; x < kXcd; x++) dc->xq[x] = 0;
     atomicAnd(&dc->err, ~4);
+    if (clear) clear_sticky(dc);
   }
 }
 
@@ -1239,11 +1263,12 @@ auto double_kernel(bool team) {
 
 }  // namespace
 
-void launch_walk(Ctx &c, const int *run_if) {
+void launch_walk(Ctx &c, const int *run_if, bool clear) {
   c.wstats_valid = false;   // they change with this walk
   const bool team = walk_as_team(c);
   const dim3 blocks(c.walk_blocks), threads(kBlock);
-  hipLaunchKernelGGL(k_walk_reset, dim3(1), dim3(64), 0, c.stream, c.dc, run_if);
+  hipLaunchKernelGGL(k_walk_reset, dim3(1), dim3(64), 0, c.stream, c.dc, run_if, clear);
+  if (c.opening == 1 && !c.fp64) launch_sys_scale(c);   // the learned angle's scales
   if (c.fp64) {
     // Treecode<double>: one i-particle per lane, LDS j-data, FP64 sums
     auto kern = c.quadrupole ? double_kernel<false>(team) : double_kernel<true>(team);
@@ -1251,6 +1276,11 @@ void launch_walk(Ctx &c, const int *run_if) {
   } else {
     auto kern = c.kahan ? float_kernel_of<true>(c, team) : float_kernel_of<false>(c, team);
     hipLaunchKernelGGL(kern, blocks, threads, 0, c.stream, walk_args<float>(c, run_if));
+  }
+  if (c.n <= kStatSmall) {
+    hipLaunchKernelGGL(k_walk_stats, dim3(1), dim3(kStatThreads), 0, c.stream, c.groups, c.gcounts,
+                       c.gpot, c.dc, run_if);
+    return;
   }
   WStat *part = reinterpret_cast<WStat *>(c.d_wpart);
   hipLaunchKernelGGL(k_walk_stats_part, dim3(kWalkStatBlocks), dim3(kBlock), 0, c.stream, c.groups,
