@@ -390,7 +390,7 @@ int build_checked(Ctx &c) {
 // synchronisation.
 int step_second_half(Ctx &c, double dt) {
   if (queue_check_direct(c, c.overlap)) return BT_ERR_HIP;
-  if (c.overlap) {
+  if (c.overlap && c.group_mode == 0) {   // leaf groups read the cells: after the levels
     if (phase_tree_and_groups(c)) return BT_ERR_HIP;
   } else if (phase_build(c) || phase_multipoles(c) || phase_groups(c)) {
     return BT_ERR_HIP;

@@ -200,7 +200,8 @@ int bt_set_walk_lds_stack(bt_ctx *ctx, int entries);
  * reference's phases run in sequence on one stream, code/treecode.cu:137-165):
  * on = 1 (default) runs makeGroups' work (PH keys, their sort, the groups) on
  * a second stream beside the level build and the multipoles, both after the
- * geometric-key sort, and the walk after both; on = 0 runs the phases in
+ * geometric-key sort, and the walk after both (leaf groups, bt_set_group_mode,
+ * come after the level build, in sequence); on = 0 runs the phases in
  * sequence, so that bt_get_timings gives each phase alone.  The results are
  * bitwise the same.  bt_build_tree, bt_compute_multipoles and bt_make_groups
  * always run on the context stream. */
