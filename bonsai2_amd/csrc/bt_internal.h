@@ -76,6 +76,20 @@ struct DevCounters {
   double wpot;
 };
 
+// All threads of one block, of the last kernel that changes the counters before the
+// host reads them: the counters to pinned memory (host is null where nothing reads
+// them).  A copy after the kernel would be a launch more.
+__device__ __forceinline__ void write_counters(const DevCounters *dc, DevCounters *host) {
+  if (!host) return;
+  static_assert(sizeof(DevCounters) % sizeof(int) == 0, "copied by words");
+  const int *src = reinterpret_cast<const int *>(dc);
+  int *dst = reinterpret_cast<int *>(host);
+  for (int k = threadIdx.x; k < (int)(sizeof(DevCounters) / sizeof(int)); k += blockDim.x)
+    __hip_atomic_store(dst + k,
+                       __hip_atomic_load(src + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __device__ __forceinline__ void clear_sticky(DevCounters *dc) {
   dc->err_sticky = 0;
   dc->stack_hw = 0;
@@ -223,7 +237,7 @@ struct Ctx {
   int direct_cap = 0;
 
   DevCounters *dc = nullptr;
-  DevCounters *pinned_dc = nullptr;   // where read_counters copies them
+  DevCounters *pinned_dc = nullptr;   // where read_counters or a kernel copies them
   DevCounters hc;                     // as last read
 
   // moveParticles' half kick still owed: the next computeForces closes the
@@ -265,7 +279,8 @@ struct Ctx {
 void launch_bbox(Ctx &c);
 void launch_geo_keys(Ctx &c);
 void launch_gather_tree(Ctx &c);
-void launch_levels(Ctx &c);
+// read: the last kernel writes the counters to c.pinned_dc (also below)
+void launch_levels(Ctx &c, bool read = false);
 int max_cell_tiles(int n);   // c.cell_cnt holds kCellCntRows ints per tile
 constexpr int kCellCntRows = 22;
 void launch_multipoles(Ctx &c);
@@ -280,14 +295,15 @@ void fill_int(Ctx &c, int *p, int value, int n);
 
 void launch_ph_keys(Ctx &c);
 // the PH gather of the particles and the groups
-void launch_groups(Ctx &c);
+void launch_groups(Ctx &c, bool read = false);
 // groups = tree cells (mode 1: the leaves; mode 2: cells of <= ncrit
 // particles), in tree order; the group order is the tree order
 void launch_leaf_groups(Ctx &c);
 
 // run_if: device flag; the walk (reset, traversal, statistics) does nothing
 // unless it is nonzero (nullptr = always run)
-void launch_walk(Ctx &c, const int *run_if = nullptr, bool clear = false);
+void launch_walk(Ctx &c, const int *run_if = nullptr, bool clear = false, bool read = false);
+bool walk_stats_in_one(const Ctx &c);   // the walks that can do so
 
 void launch_mlp_prepare(Ctx &c);
 void launch_mlp_forward(Ctx &c, int n, const float *x, float *y);
@@ -314,7 +330,7 @@ void launch_check_map(Ctx &c, int ns);
 void launch_learn_check(Ctx &c, int ns, const int *d_idx, const double *d_direct, double *out);
 
 // closing: the second half kick of a step (counted in steps_done)
-void launch_kick(Ctx &c, double dt_half, bool closing = false);
+void launch_kick(Ctx &c, double dt_half, bool closing = false, bool read = false);
 // the opening half kick (dth) and the drift (dt) of a step, in one pass
 void launch_kick_drift(Ctx &c, double dth, double dt);
 void launch_clear_sticky(Ctx &c);

@@ -161,12 +161,15 @@ hipError_t d2h(Ctx &c, void *dst, const void *src, size_t bytes) {
   return e != hipSuccess ? e : hipStreamSynchronize(c.stream);
 }
 
-// The counters, the last walk's results among them, in one copy to pinned memory.
-// (As two copies to pageable memory, which each wait for themselves, and a third for
-// the potential, an evaluation of 1000 particles, which reads them four times, took
-// 465 us instead of 343.)
-int read_counters(Ctx &c) {
-  BT_CK(hipMemcpyAsync(c.pinned_dc, c.dc, sizeof(DevCounters), hipMemcpyDeviceToHost, c.stream));
+// The counters, the last walk's results among them.  written: the last kernel queued
+// wrote them to pinned memory itself; otherwise one copy brings them there.  (An
+// evaluation of 1000 particles reads them four times.  From two copies to pageable
+// memory, which each wait for themselves, and a third for the potential, to one copy to
+// pinned memory: 465 -> 343 us; and, some steps later, to kernels that write them:
+// 280 -> 271.)
+int read_counters(Ctx &c, bool written = false) {
+  if (!written)
+    BT_CK(hipMemcpyAsync(c.pinned_dc, c.dc, sizeof(DevCounters), hipMemcpyDeviceToHost, c.stream));
   BT_CK(hipStreamSynchronize(c.stream));
   c.hc = *c.pinned_dc;
   c.wstats_valid = true;
@@ -186,10 +189,11 @@ void phase_sort(Ctx &c) {
   launch_gather_tree(c);
 }
 
-int phase_build(Ctx &c) {
+// read, here and below: the phase's last kernel writes the counters for the host.
+int phase_build(Ctx &c, bool read = false) {
   c.forked = false;
   phase_sort(c);
-  launch_levels(c);
+  launch_levels(c, read);
   record(c, 3);
   BT_LAUNCH_CK();
   return 0;
@@ -203,7 +207,7 @@ int phase_multipoles(Ctx &c, int end_ev = 4) {
   return 0;
 }
 
-int phase_groups(Ctx &c, int end_ev = 7) {
+int phase_groups(Ctx &c, int end_ev = 7, bool read = false) {
   if (c.group_mode != 0) {
     record(c, 5);
     record(c, 6);
@@ -218,7 +222,7 @@ int phase_groups(Ctx &c, int end_ev = 7) {
   c.ph_low = radix_sort_pairs(c, c.ph_keys, c.perm, c.keyB, c.valB, c.n, 63, true,
                               c.level_split <= 13);
   record(c, 6);
-  launch_groups(c);
+  launch_groups(c, read);
   record(c, end_ev);
   BT_LAUNCH_CK();
   return 0;
@@ -254,9 +258,9 @@ int phase_tree_and_groups(Ctx &c) {
 }
 
 // clear: the sticky state is cleared with the walk's own (launch_clear_sticky).
-int phase_forces(Ctx &c, bool clear = false) {
+int phase_forces(Ctx &c, bool clear = false, bool read = false) {
   if (ensure_stack(c)) return BT_ERR_HIP;
-  launch_walk(c, nullptr, clear);
+  launch_walk(c, nullptr, clear, read);
   record(c, 8);
   BT_LAUNCH_CK();
   return 0;
@@ -368,11 +372,10 @@ int regrow_cells(Ctx &c) {
 
 // Build, growing the cell arrays once if they were too small.
 int build_checked(Ctx &c) {
-  if (phase_build(c)) return BT_ERR_HIP;
-  if (read_counters(c)) return BT_ERR_HIP;
+  if (phase_build(c, true) || read_counters(c, true)) return BT_ERR_HIP;
   if (c.hc.err & kShortTree) {   // the particles as gathered, by every digit
     c.full_sort = true;
-    if (phase_build(c) || read_counters(c)) return BT_ERR_HIP;
+    if (phase_build(c, true) || read_counters(c, true)) return BT_ERR_HIP;
   }
   if (c.hc.err & kSortErr) return fail(c, BT_ERR_HIP, kSortErrMsg);
   if (c.hc.err & 1) {
@@ -388,7 +391,7 @@ int build_checked(Ctx &c) {
 // The second half of a kick-drift-kick step, after the drift: the forces at
 // the new positions and the closing half kick.  Queued without host
 // synchronisation.
-int step_second_half(Ctx &c, double dt) {
+int step_second_half(Ctx &c, double dt, bool read) {
   if (queue_check_direct(c, c.overlap)) return BT_ERR_HIP;
   if (c.overlap && c.group_mode == 0) {   // leaf groups read the cells: after the levels
     if (phase_tree_and_groups(c)) return BT_ERR_HIP;
@@ -396,7 +399,7 @@ int step_second_half(Ctx &c, double dt) {
     return BT_ERR_HIP;
   }
   if (phase_forces(c) || launch_learned_check(c)) return BT_ERR_HIP;
-  launch_kick(c, 0.5 * dt, true);
+  launch_kick(c, 0.5 * dt, true, read);
   record(c, 9);
   BT_LAUNCH_CK();
   return 0;
@@ -415,17 +418,17 @@ int redo_second_half(Ctx &c, double dt) {
     if (rc) return rc;
   }
   launch_clear_sticky(c);
-  return step_second_half(c, dt);
+  return step_second_half(c, dt, true);
 }
 
 // After the queued second half of a step.  (Sorted by every digit, the tree may
 // still outgrow its cells: two failures in a row at most.)
 int finish_step(Ctx &c, double dt) {
-  if (read_counters(c)) return BT_ERR_HIP;
+  if (read_counters(c, true)) return BT_ERR_HIP;
   for (int k = 0; k < 2 && can_redo(c); k++) {
     const int rc = redo_second_half(c, dt);
     if (rc) return rc;
-    if (read_counters(c)) return BT_ERR_HIP;
+    if (read_counters(c, true)) return BT_ERR_HIP;
   }
   if (c.hc.err_sticky & kSortErr) return fail(c, BT_ERR_HIP, kSortErrMsg);
   if (c.hc.err_sticky & 1) return fail(c, BT_ERR_CAPACITY, "cell capacity exceeded");
@@ -531,7 +534,7 @@ int create_ctx(bt_ctx **out, double eps, double theta, int ncrit, bool fp64) {
   if (const char *e = std::getenv("BT_CHECK_SLICES"))
     c.check_slices = std::max(1, std::min(2048, std::atoi(e)));
   for (int k = 0; k < 12; k++) (void)hipEventCreate(&c.ev[k]);
-  if (hipHostMalloc((void **)&c.pinned_dc, sizeof(DevCounters), hipHostMallocDefault) !=
+  if (hipHostMalloc((void **)&c.pinned_dc, sizeof(DevCounters), hipHostMallocCoherent) !=
       hipSuccess)
     c.pinned_dc = nullptr;
   if (!c.pinned_dc || dev_alloc(c, &c.dc, 1) || dev_alloc(c, &c.level_beg, kLevels) ||
@@ -836,11 +839,11 @@ int bt_make_groups(bt_ctx *h, int level_split, int ncrit) {
   c.level_split = std::max(1, level_split);
   c.ncrit = ncrit;
   record(c, 4);
-  if (phase_groups(c)) return BT_ERR_HIP;
-  if (read_counters(c)) return BT_ERR_HIP;
+  const bool read = c.group_mode == 0;
+  if (phase_groups(c, 7, read) || read_counters(c, read)) return BT_ERR_HIP;
   if (c.hc.err & kShortPh) {
     c.full_sort = true;
-    if (phase_groups(c) || read_counters(c)) return BT_ERR_HIP;
+    if (phase_groups(c, 7, read) || read_counters(c, read)) return BT_ERR_HIP;
   }
   if (c.hc.err & kSortErr) return fail(c, BT_ERR_HIP, kSortErrMsg);
   if (c.hc.err & 2) return fail(c, BT_ERR_CAPACITY, kGroupCapacityMsg);
@@ -859,11 +862,13 @@ int bt_compute_forces(bt_ctx *h, int intcount, double stats[4]) {
   // the check's sum runs after this walk, from the tree-order particles
   if (join_check(c)) return BT_ERR_HIP;
   c.check_state = 0;
-  if (phase_forces(c, true) || launch_learned_check(c)) return BT_ERR_HIP;
+  // the walk is the last to change the counters
+  const bool read = walk_stats_in_one(c) && !check_active(c) && c.pending_kick == 0.0;
+  if (phase_forces(c, true, read) || launch_learned_check(c)) return BT_ERR_HIP;
   // a moveParticles before this evaluation owes its step's closing half kick
   if (c.pending_kick != 0.0) launch_kick(c, c.pending_kick, true);
   BT_LAUNCH_CK();
-  if (read_counters(c)) return BT_ERR_HIP;
+  if (read_counters(c, read)) return BT_ERR_HIP;
   if (c.hc.err_sticky & 4) return fail(c, BT_ERR_STACK, "walk stack overflow");
   c.pending_kick = 0.0;
   c.have_acc = true;
@@ -958,7 +963,7 @@ int bt_step_f64(bt_ctx *h, double dt, int nleaf, int level_split, int ncrit) {
   launch_clear_sticky(c);
   launch_kick_drift(c, 0.5 * dt, dt);
   c.have_tree = c.have_mp = c.have_groups = c.have_acc = false;
-  int rc = step_second_half(c, dt);
+  int rc = step_second_half(c, dt, true);
   if (!rc) rc = finish_step(c, dt);
   if (rc) return rc;
   c.have_tree = c.have_mp = c.have_groups = c.have_acc = true;
@@ -1670,7 +1675,7 @@ int bt_step_graph(bt_ctx *h, float dt, int nleaf, int level_split, int ncrit, in
         break;
       }
       launch_kick_drift(c, 0.5 * (double)dt, dt);
-      rc = step_second_half(c, dt);   // the build swaps the buffers on the host side
+      rc = step_second_half(c, dt, false);   // the build swaps the buffers on the host side
       if (hipStreamEndCapture(c.stream, &c.graph[g]) != hipSuccess) rc = BT_ERR_HIP;
       c.check_state = 0;   // captured work is not queued: nothing of it to join
       if (!rc && hipGraphInstantiate(&c.graph_exec[g], c.graph[g], nullptr, nullptr, 0) !=

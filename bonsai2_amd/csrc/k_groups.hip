@@ -106,6 +106,7 @@ struct GroupArgs {
   int2 *groups;
   int *group_sys;
   DevCounters *dc;
+  DevCounters *host;   // pinned, or null
 };
 
 // Whether particle i starts a run; the ones past the last do.
@@ -264,6 +265,8 @@ __global__ __launch_bounds__(kScanThreads) void k_group_scan(GroupArgs a) {
 template <bool FOREST>
 __global__ __launch_bounds__(kBlock) void k_group_write(GroupArgs a) {
   BT_BUILD_PRIO();
+  // (no more groups than particles: nothing below changes them)
+  if (blockIdx.x == 0) write_counters(a.dc, a.host);
   __shared__ GroupTile tile;
   const int t0 = blockIdx.x * kGroupTile;
   const int lane = lane_id(), w = threadIdx.x >> 6;
@@ -417,7 +420,7 @@ void launch_leaf_groups(Ctx &c) {
                      c.stream, c.n, c.cap_groups, c.groups, c.dc);
 }
 
-void launch_groups(Ctx &c) {
+void launch_groups(Ctx &c, bool read) {
   const int ls = c.level_split < 1 ? 1 : c.level_split;
   GroupArgs a;
   a.n = c.n;
@@ -441,6 +444,7 @@ void launch_groups(Ctx &c) {
   a.groups = c.groups;
   a.group_sys = c.group_sys;
   a.dc = c.dc;
+  a.host = read ? c.pinned_dc : nullptr;
   const dim3 tiles(a.ntiles);
   const bool forest = c.nsys > 1;
   if (c.fp64) {

@@ -33,9 +33,18 @@ template <typename R>
 __global__ __launch_bounds__(kBlock) void k_kick(int n, const int *__restrict__ perm,
                                                  const V4<R> *__restrict__ acc,
                                                  V4<R> *__restrict__ vel, R dth,
-                                                 DevCounters *dc, int closing) {
-  if (dc->err_sticky) return;
-  if (closing && blockIdx.x == 0 && threadIdx.x == 0) dc->steps_done++;
+                                                 DevCounters *dc, int closing,
+                                                 DevCounters *host) {
+  const bool failed = dc->err_sticky != 0;
+  if (blockIdx.x == 0) {
+    if (closing && !failed && threadIdx.x == 0) {
+      dc->steps_done++;
+      __threadfence();
+    }
+    __syncthreads();
+    write_counters(dc, host);
+  }
+  if (failed) return;
   for (int k = blockIdx.x * kBlock + threadIdx.x; k < n; k += gridDim.x * kBlock) {
     const int t = perm[k];
     const V4<R> a = acc[k];
@@ -231,14 +240,15 @@ __global__ __launch_bounds__(kBlock) void k_direct_reduce(int ns, int nslices,
 
 }  // namespace
 
-void launch_kick(Ctx &c, double dth, bool closing) {
+void launch_kick(Ctx &c, double dth, bool closing, bool read) {
+  DevCounters *host = read ? c.pinned_dc : nullptr;
   const dim3 g(grid_for(c.n, kBlock, 8192));
   if (c.fp64)
     hipLaunchKernelGGL(k_kick<double>, g, dim3(kBlock), 0, c.stream, c.n, c.perm,
-                       as4<double>(c.acc), as4<double>(c.vel), dth, c.dc, closing ? 1 : 0);
+                       as4<double>(c.acc), as4<double>(c.vel), dth, c.dc, closing ? 1 : 0, host);
   else
     hipLaunchKernelGGL(k_kick<float>, g, dim3(kBlock), 0, c.stream, c.n, c.perm, c.acc, c.vel,
-                       (float)dth, c.dc, closing ? 1 : 0);
+                       (float)dth, c.dc, closing ? 1 : 0, host);
 }
 
 void launch_kick_drift(Ctx &c, double dth, double dt) {

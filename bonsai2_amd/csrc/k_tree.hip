@@ -267,6 +267,7 @@ struct LevelArgs {
   int2 *root_cells;
   int2 *level_beg;
   DevCounters *dc;
+  DevCounters *host;   // pinned, or null
 };
 
 // Octant digits two 63-bit keys share.
@@ -561,6 +562,7 @@ __global__ __launch_bounds__(kBlock) void k_cells_place(LevelArgs a) {
 
 __global__ __launch_bounds__(kBlock) void k_cells_finish(LevelArgs a) {
   BT_BUILD_PRIO();
+  if (blockIdx.x == 0) write_counters(a.dc, a.host);
   const int nc_all = a.dc->ncells;
   for (int s = blockIdx.x * kBlock + threadIdx.x; s < nc_all; s += gridDim.x * kBlock) {
     uint4 r = a.raw[s];
@@ -872,7 +874,7 @@ int cell_tiles(int n) {   // particle n, past the last, included
 // the most tiles that any number of particles up to n takes
 int max_cell_tiles(int n) { return std::max(cell_tiles(n), cell_tiles(std::min(n, kCellSmall))); }
 
-void launch_levels(Ctx &c) {
+void launch_levels(Ctx &c, bool read) {
   LevelArgs a;
   a.nsys = c.nsys;
   a.nleaf = c.nleaf;
@@ -890,6 +892,7 @@ void launch_levels(Ctx &c) {
   a.root_cells = c.root_cells;
   a.level_beg = c.level_beg;
   a.dc = c.dc;
+  a.host = read ? c.pinned_dc : nullptr;
   const dim3 tiles(a.ntiles), cells(grid_for(std::max(c.cap_cells, c.nsys), kBlock, 4096));
   const bool forest = c.nsys > 1;
   const bool small = c.n <= kCellSmall;

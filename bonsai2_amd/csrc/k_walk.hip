@@ -1130,11 +1130,17 @@ __device__ __forceinline__ void put_stats(DevCounters *dc, const WStat &v) {
 __global__ __launch_bounds__(kStatThreads) void k_walk_stats(const int2 *__restrict__ groups,
                                                              const int2 *__restrict__ gcounts,
                                                              const double *__restrict__ gpot,
-                                                             DevCounters *dc, const int *run_if) {
-  if (run_if && *run_if == 0) return;
+                                                             DevCounters *dc, const int *run_if,
+                                                             DevCounters *host) {
+  if (run_if && *run_if == 0) return;   // (host is null then)
   __shared__ WStat sh[kStatThreads / kWave];
   const WStat v = block_stats(group_stats(groups, gcounts, gpot, 0, dc->ngroups), sh);
-  if (threadIdx.x == 0) put_stats(dc, v);
+  if (threadIdx.x == 0) {
+    put_stats(dc, v);
+    __threadfence();
+  }
+  __syncthreads();
+  write_counters(dc, host);
 }
 
 __global__ __launch_bounds__(kBlock) void k_walk_stats_part(const int2 *__restrict__ groups,
@@ -1263,7 +1269,9 @@ auto double_kernel(bool team) {
 
 }  // namespace
 
-void launch_walk(Ctx &c, const int *run_if, bool clear) {
+bool walk_stats_in_one(const Ctx &c) { return c.n <= kStatSmall; }
+
+void launch_walk(Ctx &c, const int *run_if, bool clear, bool read) {
   c.wstats_valid = false;   // they change with this walk
   const bool team = walk_as_team(c);
   const dim3 blocks(c.walk_blocks), threads(kBlock);
@@ -1277,9 +1285,9 @@ void launch_walk(Ctx &c, const int *run_if, bool clear) {
     auto kern = c.kahan ? float_kernel_of<true>(c, team) : float_kernel_of<false>(c, team);
     hipLaunchKernelGGL(kern, blocks, threads, 0, c.stream, walk_args<float>(c, run_if));
   }
-  if (c.n <= kStatSmall) {
+  if (walk_stats_in_one(c)) {
     hipLaunchKernelGGL(k_walk_stats, dim3(1), dim3(kStatThreads), 0, c.stream, c.groups, c.gcounts,
-                       c.gpot, c.dc, run_if);
+                       c.gpot, c.dc, run_if, read ? c.pinned_dc : nullptr);
     return;
   }
   WStat *part = reinterpret_cast<WStat *>(c.d_wpart);
