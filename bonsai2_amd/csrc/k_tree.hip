@@ -925,9 +925,10 @@ void multipoles_t(Ctx &c) {
   a.arrived = c.cell_arrived;
   a.dc = c.dc;
   const int grid = grid_for(c.cap_cells, kBlock, 2048);
-  // computeMultipoles, one launch per level / one in all: 2^10 87 / 26 us, 2^16 88 /
-  // 46, 2^18 106 / 58, 2^20 118 / 159 (records past the L2 cost more than launches)
-  if (c.n <= 1 << 18) {
+  // computeMultipoles, one launch per level / one in all: 2^16 88 / 43 us, 4*10^5 140 /
+  // 86, 7*10^5 150 / 120, 10^6 159 / 148, 2*10^6 175 / 243 (records past the L2 cost more
+  // than launches); FP64 4*10^5 175 / 138
+  if (c.n <= 1 << 20) {
     hipLaunchKernelGGL(k_multipole_climb<T>, dim3(grid), dim3(kBlock), 0, c.stream, a);
     return;
   }
