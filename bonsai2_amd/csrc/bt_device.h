@@ -184,8 +184,11 @@ __device__ __forceinline__ int system_of(int i, int nsys, const int *__restrict_
 // The place of pair i among pairs sorted by all but the low `low` bits of their keys
 // (stably, and within systems): pairs that agree in the sorted bits form short runs,
 // in which a pair's place is the number of smaller keys, ties in their order.  A run
-// of more than kRunMax pairs is not looked through: `ok` is cleared.
-constexpr int kRunMax = 64;
+// of more than kRunMax pairs is not looked through: `ok` is cleared.  256: an evolving
+// halo and disk of 2^24, whose box grows with the particles that leave it, had a run of
+// more than 64 in its 24th step, and 8 digits instead of 5 from then on (sorts 1.53 ->
+// 2.47 ms a step); looking through longer runs costs its gathers 0.09 ms.
+constexpr int kRunMax = 256;
 template <bool FOREST>
 __device__ __forceinline__ int place_in_run(int i, int n, int low, const uint64_t *keys,
                                             const int *vals, int nsys, const int *off,
