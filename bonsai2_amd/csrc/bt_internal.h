@@ -229,7 +229,10 @@ struct Ctx {
   hipStream_t stream3 = nullptr;
   hipEvent_t chk_fork_ev = nullptr, chk_join_ev = nullptr;
   int check_state = 0;
-  int check_slices = 768;
+  // Four blocks on every CU: a step of 2^24 (halo + disk, learned) takes 30.9 ms with
+  // 512 or 768 slices, whose sum runs into the walk, 29.8 with 1024, 30.3 with 1280 and
+  // more, which hold the build back; of 2^22 7.20, 7.02, 6.99 and 7.03 ms.
+  int check_slices = 1024;
 
   // energies / direct sum scratch
   double *d_energy = nullptr;  // 2 * nsys
