@@ -332,7 +332,7 @@ def plain_walk(bt):
 
 def hbm_phases(t, phase, n, sort_passes):
     """Algorithmic bytes of the build, sort and multipole phases over their
-    HIP-event times (bytes per kernel as listed in DESIGN.md)."""
+    HIP-event times."""
     tr = t.tree(multipoles=False)
     cells = tr["cells"].astype(np.int64)
     node = cells[:, 1] != 0xFFFFFFFF

@@ -21,8 +21,9 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libbonsai2_amd.so")
 
 ORDER_INPUT, ORDER_TREE, ORDER_PH = 0, 1, 2
-# radix passes per sort of the 63-bit keys (bytes per pass: 24 per key-value pair)
-SORT_PASSES = 8
+# radix passes per sort of more than 2^17 keys of one system (bytes per pass: 24 per
+# key-value pair): 40 of the 63 bits, the gather orders the rest
+SORT_PASSES = 5
 P = ctypes.c_void_p
 I = ctypes.c_int
 F = ctypes.c_float

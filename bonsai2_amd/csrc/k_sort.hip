@@ -9,15 +9,16 @@
 // (2) exclusive scan of each digit's row over the tiles, one block per digit, and the
 // digits' totals, which the scatter's blocks scan themselves (one launch; a scan of the
 // whole array took two, 9 us instead of 3 at 10^6 pairs, 12 instead of 6 at 2*10^7);
-// (3) stable ranks: each wave ranks its contiguous quarter of the tile with 8
+// (3) stable ranks: each wave ranks its contiguous eighth of the tile with 8
 // ballots per 64 pairs (lanes with equal digits form a peer mask) against its
 // own digit counters in LDS, keeping the pairs in registers; the waves' counts
 // are then chained per digit, each pair is placed at its sorted position
 // within the tile in LDS, and the tile is written out in that order, so
 // consecutive threads store consecutive addresses of one digit's run (whole
 // cache lines instead of one scattered store per pair).
-// A tile is 256 threads x 16 rounds = 4096 pairs; HBM traffic per pass is
-// ~8 B (histogram read) + 12 B read + 12 B written per pair.
+// A tile is 512 threads x 8 rounds = 4096 pairs; HBM traffic per pass is
+// ~8 B (histogram read) + 12 B read + 12 B written per pair.  Up to 2^17 pairs of one
+// system are sorted by tiles in LDS and merged instead (below).
 #include "bt_device.h"
 #include "bt_internal.h"
 

@@ -218,7 +218,9 @@ int bt_set_overlap(bt_ctx *ctx, int on);
 int bt_set_group_mode(bt_ctx *ctx, int mode);
 /* Deepest traversal stack of any group in the walks of the last call that
  * walked (entries, LDS and global parts together; all replays of a
- * bt_step_graph): the stack_ints a walk of this tree needs. */
+ * bt_step_graph): the stack_ints a walk of this tree needs.  Up to 2^19
+ * particles the four waves of a block share a group's stack, which then holds
+ * more than one wave's would. */
 int bt_get_walk_stack_max(bt_ctx *ctx, int *entries);
 /* code/Treecode.h:14-16 (#define QUADRUPOLE): 1 (default) = monopole +
  * quadrupole P2C (code/computeForces.cu:83-128, 64 flops); 0 = monopole-only
