@@ -90,6 +90,14 @@ __device__ __forceinline__ void write_counters(const DevCounters *dc, DevCounter
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// Before every walk: its queues, its stack's depth and its error.
+__device__ __forceinline__ void reset_walk(DevCounters *dc) {
+  dc->queue = 0;
+  dc->stack_max = 0;
+  for (int x = 0; x < 8; x++) dc->xq[x] = 0;
+  atomicAnd(&dc->err, ~4);
+}
+
 __device__ __forceinline__ void clear_sticky(DevCounters *dc) {
   dc->err_sticky = 0;
   dc->stack_hw = 0;
@@ -305,7 +313,8 @@ void launch_leaf_groups(Ctx &c);
 
 // run_if: device flag; the walk (reset, traversal, statistics) does nothing
 // unless it is nonzero (nullptr = always run)
-void launch_walk(Ctx &c, const int *run_if = nullptr, bool clear = false, bool read = false);
+void launch_walk(Ctx &c, const int *run_if = nullptr, bool clear = false, bool read = false,
+                 bool reset = true);
 bool walk_stats_in_one(const Ctx &c);   // the walks that can do so
 
 void launch_mlp_prepare(Ctx &c);
@@ -335,7 +344,7 @@ void launch_learn_check(Ctx &c, int ns, const int *d_idx, const double *d_direct
 // closing: the second half kick of a step (counted in steps_done)
 void launch_kick(Ctx &c, double dt_half, bool closing = false, bool read = false);
 // the opening half kick (dth) and the drift (dt) of a step, in one pass
-void launch_kick_drift(Ctx &c, double dth, double dt);
+void launch_kick_drift(Ctx &c, double dth, double dt, bool clear);   // resets the walk too
 void launch_clear_sticky(Ctx &c);
 void launch_iota(Ctx &c, int n, int *out);   // out[k] = k
 // n values of the context's 4-vector type: dst[idx[k]] = src[k] (scatter) or

@@ -258,9 +258,10 @@ int phase_tree_and_groups(Ctx &c) {
 }
 
 // clear: the sticky state is cleared with the walk's own (launch_clear_sticky).
-int phase_forces(Ctx &c, bool clear = false, bool read = false) {
+// reset: the walk's state has not been reset since the last one.
+int phase_forces(Ctx &c, bool clear = false, bool read = false, bool reset = true) {
   if (ensure_stack(c)) return BT_ERR_HIP;
-  launch_walk(c, nullptr, clear, read);
+  launch_walk(c, nullptr, clear, read, reset);
   record(c, 8);
   BT_LAUNCH_CK();
   return 0;
@@ -391,14 +392,14 @@ int build_checked(Ctx &c) {
 // The second half of a kick-drift-kick step, after the drift: the forces at
 // the new positions and the closing half kick.  Queued without host
 // synchronisation.
-int step_second_half(Ctx &c, double dt, bool read) {
+int step_second_half(Ctx &c, double dt, bool read, bool reset) {
   if (queue_check_direct(c, c.overlap)) return BT_ERR_HIP;
   if (c.overlap && c.group_mode == 0) {   // leaf groups read the cells: after the levels
     if (phase_tree_and_groups(c)) return BT_ERR_HIP;
   } else if (phase_build(c) || phase_multipoles(c) || phase_groups(c)) {
     return BT_ERR_HIP;
   }
-  if (phase_forces(c) || launch_learned_check(c)) return BT_ERR_HIP;
+  if (phase_forces(c, false, false, reset) || launch_learned_check(c)) return BT_ERR_HIP;
   launch_kick(c, 0.5 * dt, true, read);
   record(c, 9);
   BT_LAUNCH_CK();
@@ -418,7 +419,7 @@ int redo_second_half(Ctx &c, double dt) {
     if (rc) return rc;
   }
   launch_clear_sticky(c);
-  return step_second_half(c, dt, true);
+  return step_second_half(c, dt, true, true);
 }
 
 // After the queued second half of a step.  (Sorted by every digit, the tree may
@@ -900,8 +901,7 @@ int bt_move_particles_f64(bt_ctx *h, double dt) {
   if (!h) return BT_ERR_ARG;
   Ctx &c = h->c;
   if (!c.have_acc) return fail(c, BT_ERR_STATE, "computeForces first");
-  launch_clear_sticky(c);
-  launch_kick_drift(c, 0.5 * dt, dt);
+  launch_kick_drift(c, 0.5 * dt, dt, true);
   BT_LAUNCH_CK();
   BT_CK(hipStreamSynchronize(c.stream));
   // positions moved: the tree, moments, groups and forces are stale; the
@@ -960,10 +960,9 @@ int bt_step_f64(bt_ctx *h, double dt, int nleaf, int level_split, int ncrit) {
     if (!rc) rc = bt_compute_forces(h, 1, nullptr);
     if (rc) return rc;
   }
-  launch_clear_sticky(c);
-  launch_kick_drift(c, 0.5 * dt, dt);
+  launch_kick_drift(c, 0.5 * dt, dt, true);
   c.have_tree = c.have_mp = c.have_groups = c.have_acc = false;
-  int rc = step_second_half(c, dt, true);
+  int rc = step_second_half(c, dt, true, false);
   if (!rc) rc = finish_step(c, dt);
   if (rc) return rc;
   c.have_tree = c.have_mp = c.have_groups = c.have_acc = true;
@@ -1674,8 +1673,8 @@ int bt_step_graph(bt_ctx *h, float dt, int nleaf, int level_split, int ncrit, in
         rc = BT_ERR_HIP;
         break;
       }
-      launch_kick_drift(c, 0.5 * (double)dt, dt);
-      rc = step_second_half(c, dt, false);   // the build swaps the buffers on the host side
+      launch_kick_drift(c, 0.5 * (double)dt, dt, false);
+      rc = step_second_half(c, dt, false, false);   // the build swaps the buffers on the host side
       if (hipStreamEndCapture(c.stream, &c.graph[g]) != hipSuccess) rc = BT_ERR_HIP;
       c.check_state = 0;   // captured work is not queued: nothing of it to join
       if (!rc && hipGraphInstantiate(&c.graph_exec[g], c.graph[g], nullptr, nullptr, 0) !=

@@ -1174,10 +1174,7 @@ __global__ __launch_bounds__(kBlock) void k_walk_stats_final(const WStat *__rest
 // clear: the sticky state too, where the walk is the first launch of an API call.
 __global__ void k_walk_reset(DevCounters *dc, const int *run_if, bool clear) {
   if (threadIdx.x == 0 && !(run_if && *run_if == 0)) {
-    dc->queue = 0;
-    dc->stack_max = 0;
-    for (int x = 0; x < kXcd; x++) dc->xq[x] = 0;
-    atomicAnd(&dc->err, ~4);
+    reset_walk(dc);
     if (clear) clear_sticky(dc);
   }
 }
@@ -1271,11 +1268,12 @@ auto double_kernel(bool team) {
 
 bool walk_stats_in_one(const Ctx &c) { return c.n <= kStatSmall; }
 
-void launch_walk(Ctx &c, const int *run_if, bool clear, bool read) {
+void launch_walk(Ctx &c, const int *run_if, bool clear, bool read, bool reset) {
   c.wstats_valid = false;   // they change with this walk
   const bool team = walk_as_team(c);
   const dim3 blocks(c.walk_blocks), threads(kBlock);
-  hipLaunchKernelGGL(k_walk_reset, dim3(1), dim3(64), 0, c.stream, c.dc, run_if, clear);
+  if (reset)
+    hipLaunchKernelGGL(k_walk_reset, dim3(1), dim3(64), 0, c.stream, c.dc, run_if, clear);
   if (c.opening == 1 && !c.fp64) launch_sys_scale(c);   // the learned angle's scales
   if (c.fp64) {
     // Treecode<double>: one i-particle per lane, LDS j-data, FP64 sums
