@@ -559,6 +559,18 @@ int create_ctx(bt_ctx **out, double eps, double theta, int ncrit, bool fp64) {
   return 0;
 }
 
+// Appends to the systems' offsets what system_of reads behind them: the systems of
+// particles 0, kSystemStep, ..., the last of them past the last particle's stretch.
+void system_table(std::vector<int> &off, int n) {
+  const int entries = (n - 1) / kSystemStep + 2;
+  off.reserve(off.size() + entries);
+  for (int k = 0, sys = 0; k < entries; k++) {
+    const int i = (int)std::min<long long>((long long)k * kSystemStep, n - 1);
+    while (off[sys + 1] <= i) sys++;
+    off.push_back(sys);
+  }
+}
+
 // The real type of a data entry point must match the context's.
 template <typename T>
 int check_real(Ctx &c) {
@@ -745,7 +757,7 @@ int bt_alloc(bt_ctx *h, int n, int nsys, const int *offsets) {
     rc |= dev_alloc(c, &c.box, (size_t)nsys * w); rc |= dev_alloc(c, &c.root_cells, nsys);
     rc |= dev_alloc(c, &c.sys_scale, nsys);
     rc |= dev_alloc(c, &c.cell_cnt, (size_t)kCellCntRows * max_cell_tiles(n));
-    rc |= dev_alloc(c, &c.d_off, nsys + 1);
+    rc |= dev_alloc(c, &c.d_off, nsys + 1 + (size_t)(n - 1) / kSystemStep + 2);
     rc |= dev_alloc(c, &c.d_energy, 2 * (size_t)nsys * 65);
     if (rc) return BT_ERR_HIP;
     if (alloc_cells(c, n + 1024 * nsys + 64)) return BT_ERR_HIP;
@@ -755,7 +767,8 @@ int bt_alloc(bt_ctx *h, int n, int nsys, const int *offsets) {
   const int part_n = (long long)nsys * ((c.max_sys_n + 2047) / 2048) <= 65536 ? 2048 : 16384;
   c.bbox_blocks = std::max(1, std::min(1024, (c.max_sys_n + part_n - 1) / part_n));
   if (dev_alloc(c, &c.bbox_part, 2 * (size_t)nsys * c.bbox_blocks * rw(c))) return BT_ERR_HIP;
-  BT_CK(hipMemcpy(c.d_off, off.data(), sizeof(int) * (nsys + 1), hipMemcpyHostToDevice));
+  system_table(off, n);
+  BT_CK(hipMemcpy(c.d_off, off.data(), sizeof(int) * off.size(), hipMemcpyHostToDevice));
   c.have_particles = c.have_tree = c.have_mp = c.have_groups = c.have_acc = false;
   return 0;
 }
