@@ -59,9 +59,8 @@ struct DevCounters {
   int stack_max;  // deepest walk stack of the last walk (entries)
   int xq[8];      // walk group queues, one per XCD range
   // per-step check of the learned angle, decided on the device
-  int check_calls;  // checks drawn so far (seeds the sample indices)
   int fallback;     // 1: the last check failed and the fixed-angle walk ran
-  int checks, fallbacks;
+  int checks, fallbacks;   // judged so far; checks seeds the sample indices
   // Sticky state, cleared only by the host (launch_clear_sticky) at the start
   // of each API call that steps or walks: every error bit any phase raised
   // since (err is cleared by each phase for itself), the deepest walk stack of

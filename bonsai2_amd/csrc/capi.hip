@@ -6,6 +6,7 @@
 // code/cutil.h:772-780) all state is per context and errors are returned.
 #include <algorithm>
 #include <cmath>
+#include <cstddef>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -1594,9 +1595,11 @@ int bt_set_opening_check(bt_ctx *h, int nsamples, float p99_max, uint64_t seed) 
   c.check_ns = nsamples;
   c.check_p99 = p99_max;
   c.check_seed = seed;
-  // restart the device's check count (the sample draws) and statistics
-  const int zero[4] = {0, 0, 0, 0};
-  BT_CK(hipMemcpyAsync(&c.dc->check_calls, zero, sizeof(zero), hipMemcpyHostToDevice, c.stream));
+  // restart the device's last decision, check count (the sample draws) and fallbacks
+  const int zero[3] = {0, 0, 0};
+  static_assert(offsetof(DevCounters, fallbacks) == offsetof(DevCounters, fallback) + 2 * sizeof(int),
+                "fallback, checks, fallbacks");
+  BT_CK(hipMemcpyAsync(&c.dc->fallback, zero, sizeof(zero), hipMemcpyHostToDevice, c.stream));
   if (nsamples > 0) {
     const double z3[3] = {0.0, 0.0, 0.0};
     BT_CK(hipMemcpyAsync(check_result(c), z3, sizeof(z3), hipMemcpyHostToDevice, c.stream));

@@ -508,21 +508,24 @@ __global__ __launch_bounds__(64) void k_mlp_reduce(const float *__restrict__ par
 // ---- per-step check of the learned walk -------------------------------------------
 
 // Targets of a check (one block of 1024 threads, ns <= 1024): draw k is
-// idx[k] = mix64(seed ^ (calls << 32) ^ k) mod n, an index into the particle
-// arrays as they are when the draw runs (calls = the checks drawn before).
+// idx[k] = mix64(seed ^ (checks << 32) ^ k) mod n, an index into the particle
+// arrays as they are when the draw runs (checks = the checks judged before: a step
+// that fails and is run again draws with the same number, and so do the replays of a
+// graph after a failed one, so a captured step's checks are those of eager steps).
 // Their input ids, sorted with the draw slot as tie-break, go to
 // idx[ns + j] and the slots to idx[2 ns + j], for k_check_map.
 __global__ __launch_bounds__(1024) void k_check_idx(int ns, int n, unsigned long long seed,
-                                                    DevCounters *dc, const int *__restrict__ id,
+                                                    const DevCounters *dc,
+                                                    const int *__restrict__ id,
                                                     int *__restrict__ idx) {
   __shared__ int s_id[1024];
   __shared__ int s_slot[1024];
-  const unsigned long long calls = (unsigned long long)(unsigned)dc->check_calls;
+  const unsigned long long checks = (unsigned long long)(unsigned)dc->checks;
   const int t = threadIdx.x;
   int key = 0x7FFFFFFF;
   if (t < ns) {
     const int k =
-        (int)(mix64(seed ^ (calls << 32) ^ (unsigned long long)t) % (unsigned long long)n);
+        (int)(mix64(seed ^ (checks << 32) ^ (unsigned long long)t) % (unsigned long long)n);
     idx[t] = k;
     key = id[k];
   }
@@ -548,7 +551,6 @@ __global__ __launch_bounds__(1024) void k_check_idx(int ns, int n, unsigned long
     idx[ns + t] = s_id[t];
     idx[2 * ns + t] = s_slot[t];
   }
-  if (t == 0) dc->check_calls = (int)(calls + 1);
 }
 
 // PH index of each check target: particle p (PH order) looks its input id up
