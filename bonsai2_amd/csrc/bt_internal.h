@@ -109,6 +109,7 @@ struct GraphKey {
   double dt, eps, theta;
   int nleaf, level_split, ncrit;
   int opening, kahan, quadrupole, walk_variant, stack_ints, blocks_per_cu, lds_stack, group_mode;
+  int wave_walk;
   int overlap, full_sort;
   float learn_shift, learn_theta_lo, learn_theta_hi;
   int check_ns;
@@ -203,6 +204,7 @@ struct Ctx {
   int group_mode = 0;   // 0: PH-key groups (makeGroups); 1: leaves; 2: tree cells <= ncrit
   int walk_blocks = 0;         // persistent grid (blocks of 256)
   int blocks_per_cu = 0;
+  bool wave_walk = false;      // blocks_per_cu set by the caller: one wave per group
   int kahan = 1;
   int walk_variant = 0;        // 0: LDS j-data, 1: scalar loads, 2: two i-particles per lane
   int quadrupole = 1;          // 0: monopole-only P2C (the reference without QUADRUPOLE)
@@ -315,6 +317,12 @@ void launch_leaf_groups(Ctx &c);
 void launch_walk(Ctx &c, const int *run_if = nullptr, bool clear = false, bool read = false,
                  bool reset = true);
 bool walk_stats_in_one(const Ctx &c);   // the walks that can do so
+bool walk_as_team(const Ctx &c);        // the four waves of a block walk a group together
+// Stack entries no walk can exceed: a step pops 64 cells and pushes at most 512,
+// so at most 448 more than it takes stay behind on each of the 21 levels.  A
+// context whose stack may be too small keeps to one wave per group, so that the
+// same calls report BT_ERR_STACK.
+constexpr int kSafeStack = 8 + 21 * 448;
 
 void launch_mlp_prepare(Ctx &c);
 void launch_mlp_forward(Ctx &c, int n, const float *x, float *y);

@@ -40,6 +40,7 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kWavesPerBlock = kBlock / kWave;
 constexpr int kMaxWalkSteps = 1 << 20;
+static_assert(kSafeStack == 8 + kMaxLevel * 448, "entries left behind on every level");
 
 // Unroll of the full-batch j-loops and the occupancy target of the walk.
 #ifndef BT_UNROLL_LDS
@@ -1217,11 +1218,7 @@ WalkArgs<R> walk_args(Ctx &c, const int *run_if) {
   return a;
 }
 
-// Stack entries no walk can exceed: a step pops 64 cells and pushes at most 512,
-// so at most 448 more than it takes stay behind on each of the 21 levels.  A
-// context whose stack may be too small keeps to one wave per group, so that the
-// same calls report BT_ERR_STACK.
-constexpr int kSafeStack = 8 + kMaxLevel * 448;
+}  // namespace
 
 // Whether the blocks walk groups as teams: below the sizes at which one wave per
 // group fills the chip evenly.  Walk times on Plummer spheres (theta 0.5), one wave
@@ -1230,9 +1227,11 @@ constexpr int kSafeStack = 8 + kMaxLevel * 448;
 // 2072; FP64 2^18 1816 / 1659, 2^19 3426 / 3150.  (Teams of 2 and 8 waves were
 // slower than of 4; with the groups cut into one range per XCD 2^16 took 407 us.)
 bool walk_as_team(const Ctx &c) {
-  return c.n <= 1 << 19 && c.walk_variant == 0 && c.blocks_per_cu == 0 &&
-         c.lds_stack == kLdsStack && c.stack_ints >= kSafeStack;
+  return c.n <= 1 << 19 && c.walk_variant == 0 && !c.wave_walk && c.lds_stack == kLdsStack &&
+         c.stack_ints >= kSafeStack;
 }
+
+namespace {
 
 // variant 0: LDS j-data, one i-particle per lane; 1: scalar-load j-data, one
 // i-particle per lane; 2: two i-particles per lane, batches split between the

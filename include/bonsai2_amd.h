@@ -179,7 +179,12 @@ int bt_get_timings(bt_ctx *ctx, float ms[10]);
 /* Walk options: kahan = compensated accumulators (default 1);
  * stack_ints = per-wave traversal stack capacity (default 16384, at least 64;
  *   a walk that needs more returns BT_ERR_STACK);
- * blocks_per_cu = persistent grid size (default 0 = automatic). */
+ * blocks_per_cu = persistent grid size (default 0 = automatic).
+ * Systems of up to 2^19 particles are walked by the four waves of a block per
+ * group, several times faster below 2^17, unless blocks_per_cu is set here,
+ * stack_ints is less than 9416, bt_set_walk_variant is not 0 or
+ * bt_set_walk_lds_stack not 1024: then by one wave per group (the same
+ * interaction lists, forces equal to the rounding of their sums). */
 int bt_set_walk_options(bt_ctx *ctx, int kahan, int stack_ints, int blocks_per_cu);
 /* How the walk feeds interaction data to the lanes: 0 (default) = one
  * i-particle per lane, the wave stages each batch of 64 cells / particles in
@@ -193,7 +198,8 @@ int bt_set_walk_variant(bt_ctx *ctx, int variant);
 /* Treecode<float> walks (no reference counterpart): entries of each wave's
  * traversal stack kept in LDS, 512..1024 (default 1024); deeper entries spill
  * to the global stack of bt_set_walk_options and come back in LIFO order, so
- * the traversal and the forces do not depend on it.  A walk whose stack
+ * the traversal does not depend on it, nor do the forces unless the system is
+ * walked by four waves per group at 1024 (bt_set_walk_options).  A walk whose stack
  * needs more than these entries plus stack_ints returns BT_ERR_STACK. */
 int bt_set_walk_lds_stack(bt_ctx *ctx, int entries);
 /* Steps of bt_step and bt_step_graph (no reference counterpart: the
@@ -245,7 +251,9 @@ int bt_set_quadrupole(bt_ctx *ctx, int on);
 int bt_step_graph(bt_ctx *ctx, float dt, int nleaf, int level_split, int ncrit, int nsteps);
 /* Picks NLEAF, NCRIT (3 x 3 candidates, timed zero-dt steps), the persistent
  * walk grid (4, 8, 12, 16 blocks per CU) and the traversal stack depth
- * (4x the deepest stack seen) for the current particles, and leaves them set.
+ * (4x the deepest stack seen, at least 9416 entries where four waves walk a
+ * group, see bt_set_walk_options) for the current particles, and leaves them
+ * set; a grid set before by bt_set_walk_options is dropped.
  * table (may be NULL) gets 6 doubles per timed candidate: nleaf, ncrit,
  * blocks_per_cu, step ms, walk ms, deepest stack; *ntable their count (<= 13).
  * best = {nleaf, ncrit, blocks_per_cu, stack entries}.  flags: reserved, 0. */
