@@ -1220,6 +1220,23 @@ WalkArgs<R> walk_args(Ctx &c, const int *run_if) {
 
 }  // namespace
 
+// Whether a forest's groups are many and each has little to do.  A team takes its
+// barriers and, with the learned angle, four network evaluations for cells that fill
+// one; and the wave walk has enough groups to fill the chip.  Fixed angle / learned /
+// FP64, teams then waves (us): 256 systems of 1024 1186 1491 / 1768 1510 / 1737 1539, 512
+// of 1024 2280 2476 / 3382 2465 / 3330 2498, 32 of 16384 1684 1370 / 1823 1311 / 2758
+// 2286, 200 of 1000 927 1272 / 1386 1284 / 1359 1313; 140 of 1000 (-) / 1005 1062 / 984
+// 1095, 100 of 2000 654 979 / 923 983 / 1008 1024, 4 of 65536 953 1017 / 841 955 / 1784
+// 1693, 128 of 1024 654 1016 / 947 1018 / 922 1049.  At 8 digits a group is a particle or
+// two, fixed angle: 512 of 1024 10712 9409, 32 of 16384 6849 4864, but 2048 of 128, whose
+// groups are as small at 5 digits, 4645 5566.
+static bool many_small_walks(const Ctx &c) {
+  if (c.nsys == 1 || c.n <= 1 << 17) return false;
+  const bool learned = c.opening == 1 && c.have_mlp;
+  if (learned || c.fp64) return c.nsys > 160 || c.n > 1 << 18;
+  return c.group_mode == 0 && c.level_split > 6 && c.n / c.nsys >= 512;
+}
+
 // Whether the blocks walk groups as teams: below the sizes at which one wave per
 // group fills the chip evenly.  Walk times on Plummer spheres (theta 0.5), one wave
 // per group / teams: 2^10 509 / 44 us, 2^16 753 / 267, 2^18 1060 / 881, 2^19 1789 /
@@ -1227,8 +1244,8 @@ WalkArgs<R> walk_args(Ctx &c, const int *run_if) {
 // 2072; FP64 2^18 1816 / 1659, 2^19 3426 / 3150.  (Teams of 2 and 8 waves were
 // slower than of 4; with the groups cut into one range per XCD 2^16 took 407 us.)
 bool walk_as_team(const Ctx &c) {
-  return c.n <= 1 << 19 && c.walk_variant == 0 && !c.wave_walk && c.lds_stack == kLdsStack &&
-         c.stack_ints >= kSafeStack;
+  return c.n <= 1 << 19 && !many_small_walks(c) && c.walk_variant == 0 && !c.wave_walk &&
+         c.lds_stack == kLdsStack && c.stack_ints >= kSafeStack;
 }
 
 namespace {

@@ -181,7 +181,8 @@ int bt_get_timings(bt_ctx *ctx, float ms[10]);
  *   a walk that needs more returns BT_ERR_STACK);
  * blocks_per_cu = persistent grid size (default 0 = automatic).
  * Systems of up to 2^19 particles are walked by the four waves of a block per
- * group, several times faster below 2^17, unless blocks_per_cu is set here,
+ * group, several times faster below 2^17 (not forests of more than 2^17 in many
+ * small groups, where that is slower), unless blocks_per_cu is set here,
  * stack_ints is less than 9416, bt_set_walk_variant is not 0 or
  * bt_set_walk_lds_stack not 1024: then by one wave per group (the same
  * interaction lists, forces equal to the rounding of their sums). */
