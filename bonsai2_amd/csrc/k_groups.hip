@@ -196,7 +196,9 @@ __global__ __launch_bounds__(kBlock) void k_gather_count(GroupArgs a, const T *_
       if (a.low > 0) {
         const uint64_t key = a.keys[i];
         bool ok = true;
-        dst = place_in_run<FOREST>(i, a.n, a.low, a.keys, a.perm, a.nsys, a.off, key, ok);
+        const int sys = FOREST ? system_of(i, a.nsys, a.off) : 0;
+        dst = place_in_run(i, FOREST ? a.off[sys] : 0, FOREST ? a.off[sys + 1] : a.n, a.low, a.keys,
+                           key, ok);
         if (!ok) {
           atomicOr(&a.dc->err, kShortPh);
           atomicOr(&a.dc->err_sticky, kShortPh);

@@ -205,7 +205,8 @@ __global__ __launch_bounds__(kBlock) void k_gather3(int n, const int *__restrict
     if (SHORT) {
       const uint64_t key = keys[i];
       bool ok = true;
-      dst = place_in_run<FOREST>(i, n, low, keys, perm, nsys, off, key, ok);
+      const int sys = FOREST ? system_of(i, nsys, off) : 0;
+      dst = place_in_run(i, FOREST ? off[sys] : 0, FOREST ? off[sys + 1] : n, low, keys, key, ok);
       if (!ok) {
         atomicOr(&dc->err, kShortTree);
         atomicOr(&dc->err_sticky, kShortTree);
