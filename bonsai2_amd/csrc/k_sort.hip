@@ -652,11 +652,12 @@ constexpr int kTileRounds = kSortTile / kTileThreads;
 constexpr int kSmallTiles = 32;
 constexpr int kTileRun = 16;   // the longest run of a tile that is put in order by itself
 
+// keys_out and vals_out may be keys and vals (a single tile is sorted in place): a block
+// has its whole tile in LDS before its first store, and reads nothing after that.
 template <int ROUNDS>
-__global__ __launch_bounds__(kTileThreads) void k_tile_sort(const uint64_t *__restrict__ keys,
-                                                            const int *__restrict__ vals, int n,
-                                                            int key_bits, uint64_t *keys_out,
-                                                            int *vals_out) {
+__global__ __launch_bounds__(kTileThreads) void k_tile_sort(const uint64_t *keys, const int *vals,
+                                                            int n, int key_bits,
+                                                            uint64_t *keys_out, int *vals_out) {
   BT_BUILD_PRIO();
   static_assert(ROUNDS <= kTileRounds && kSortTile == 4096, "places of 12 bits");
   constexpr int kPairs = ROUNDS * kTileThreads;
