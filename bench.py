@@ -330,29 +330,46 @@ def plain_walk(bt):
 
 # ---- HBM fractions of the non-walk phases ------------------------------------------------
 
-def hbm_phases(t, phase, n, sort_passes):
-    """Algorithmic bytes of the build, sort and multipole phases over their
-    HIP-event times."""
-    tr = t.tree(multipoles=False)
-    cells = tr["cells"].astype(np.int64)
-    node = cells[:, 1] != 0xFFFFFFFF
-    nsplit = int((cells[node, 3] - cells[node, 2]).sum())
-    ncells = len(cells)
-    ngroups = t.counts()["ngroups"]
-    b = {"bbox_keys": 44.0 * n,
-         "sort": 24.0 * n * sort_passes,
-         "levels": 32.0 * nsplit + 16.0 * ncells,
-         "multipoles": 16.0 * n + 112.0 * ncells,
+def sort_passes_of(bt, t, n):
+    """Radix passes of one sort of n keys of one system, or None up to 2^17, where keys are
+    sorted in tiles and merged.  A run of more than 256 equal leading digits (looked for in
+    the groups' keys) has made the context sort by all 8 digits."""
+    if n <= 1 << 17:
+        return None
+    lead = t.ph()[0] >> np.uint64(63 - 8 * bt.SORT_PASSES)
+    ends = np.flatnonzero(np.diff(lead, append=~lead[-1]))
+    return 8 if int(np.diff(ends, prepend=-1).max()) > 256 else bt.SORT_PASSES
+
+
+def hbm_phases(bt, t, phase, n):
+    """Bytes that the kernels of the build, sort and multipole phases read and write
+    (FP32, one system; caches taken as perfect within a kernel), over the phases'
+    HIP-event times.  No fraction for sorts in tiles, which HBM does not bound."""
+    c = t.counts()
+    passes = sort_passes_of(bt, t, n)
+    short = passes == bt.SORT_PASSES   # the gathers put runs in order: keys in, keys and places out
+    # a pass: keys for the histogram, pairs in, pairs out
+    sort = None if passes is None else 32.0 * n * passes
+    b = {"bbox_keys": 16.0 * n + 16.0 * n + 12.0 * n,
+         "sort": sort,
+         # the tree gather (pos, vel, id through the order), then the keys twice; per cell the
+         # octant-order record written, read twice, its slot, the cell; per node its child
+         # count and its arrivals
+         "levels": (4.0 + 72.0 + (16.0 if short else 0.0)) * n + 16.0 * n +
+                   76.0 * c["ncells"] + 12.0 * c["nnodes"],
+         # leaf particles; per cell its links, 192 B of moments written, 80 of them read again
+         "multipoles": 16.0 * n + (16.0 + 192.0 + 80.0) * c["ncells"],
          "ph_keys": 28.0 * n,
-         "ph_sort": 24.0 * n * sort_passes,
-         "groups": 36.0 * n + 8.0 * n + 8.0 * ngroups}
+         "ph_sort": sort,
+         # the PH gather (pos, id through the order), the keys for counting and for writing
+         "groups": (4.0 + 40.0 + (20.0 if short else 0.0)) * n + 16.0 * n + 12.0 * c["ngroups"]}
     out = {}
     for k, v in b.items():
         ms = phase.get(k, 0.0)
-        gbs = v / (ms * 1e-3) / 1e9 if ms > 0 else None
+        gbs = v / (ms * 1e-3) / 1e9 if ms > 0 and v else None
         out[k] = {"bytes": v, "ms": ms, "GB_s": gbs,
                   "frac": gbs / HBM_PEAK_GBS if gbs else None}
-    out["sort_passes"] = sort_passes
+    out["sort_passes"] = passes
     return out
 
 
@@ -506,7 +523,7 @@ def main():
     phase_ms = {k: float(np.mean([p[k] for p in phase])) for k in phase[0]}
     phase_ms_serial = ({k: float(np.mean([p[k] for p in phase_serial])) for k in phase_serial[0]}
                        if phase_serial else None)
-    hbm = hbm_phases(t, phase_ms_serial or phase_ms, n, sort_passes=bt.SORT_PASSES)
+    hbm = hbm_phases(bt, t, phase_ms_serial or phase_ms, n)
     compare = None
     if learned:
         # the metric's comparison on the same particles and tree: the fixed
