@@ -353,10 +353,10 @@ void launch_kick(Ctx &c, double dt_half, bool closing = false, bool read = false
 // the opening half kick (dth) and the drift (dt) of a step, in one pass
 void launch_kick_drift(Ctx &c, double dth, double dt, bool clear);   // resets the walk too
 void launch_clear_sticky(Ctx &c);
-void launch_iota(Ctx &c, int n, int *out);   // out[k] = k
+hipError_t launch_iota(Ctx &c, int n, int *out);   // out[k] = k
 // n values of the context's 4-vector type: dst[idx[k]] = src[k] (scatter) or
 // dst[k] = src[idx[k]]
-void launch_permute(Ctx &c, bool scatter, const int *idx, const void *src, void *dst);
+hipError_t launch_permute(Ctx &c, bool scatter, const int *idx, const void *src, void *dst);
 void launch_energies(Ctx &c);
 int direct_slices(int ns);   // d_out of launch_direct: ns * (slices + 1) double4
 void launch_direct(Ctx &c, int ns, const int *d_idx, double *d_out, bool check = false);

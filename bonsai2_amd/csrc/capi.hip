@@ -786,8 +786,7 @@ int put_particles(Ctx &c, const void *pos4, const void *vel4, hipMemcpyKind kind
   const size_t bytes = sizeof(float4) * rw(c) * (size_t)c.n;
   BT_CK(hipMemcpyAsync(c.pos, pos4, bytes, kind, c.stream));
   BT_CK(hipMemcpyAsync(c.vel, vel4, bytes, kind, c.stream));
-  launch_iota(c, c.n, c.id);
-  BT_CK(hipGetLastError());   // (the text of an earlier call's error is no failure here)
+  BT_CK(launch_iota(c, c.n, c.id));
   c.ids_in_order = true;
   BT_CK(hipStreamSynchronize(c.stream));
   c.have_particles = true;
@@ -999,8 +998,7 @@ int read_in_order(Ctx &c, void *host, const void *src, void *tmp, bool as_is, co
   const size_t bytes = sizeof(float4) * rw(c) * (size_t)c.n;
   if (!as_is) {
     if (join_check(c)) return BT_ERR_HIP;   // a check sum may still read the old particles
-    launch_permute(c, scatter, idx, src, tmp);
-    BT_CK(hipGetLastError());
+    BT_CK(launch_permute(c, scatter, idx, src, tmp));
     src = tmp;
   }
   BT_CK(d2h(c, host, src, bytes));

@@ -14,6 +14,7 @@
 #include <cfloat>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "bt_device.h"
 #include "bt_internal.h"
@@ -269,21 +270,33 @@ void launch_kick_drift(Ctx &c, double dth, double dt, bool clear) {
                        c.vel, c.pos, (float)dth, (float)dt, c.dc, clear ? 1 : 0);
 }
 
-void launch_iota(Ctx &c, int n, int *out) {
-  hipLaunchKernelGGL(k_iota, dim3(grid_for(n, kBlock, 8192)), dim3(kBlock), 0, c.stream, n, out);
+namespace {
+
+// A launch whose own error is returned, whatever error other code left behind.
+template <typename... P, typename... A>
+hipError_t launch_checked(Ctx &c, void (*kern)(P...), dim3 grid, A... args) {
+  static_assert(sizeof...(P) == sizeof...(A) && (std::is_same<P, A>::value && ...),
+                "passed as they are");
+  void *p[] = {&args...};
+  return hipLaunchKernel(reinterpret_cast<const void *>(kern), grid, dim3(kBlock), p, 0, c.stream);
 }
 
-void launch_permute(Ctx &c, bool scatter, const int *idx, const void *src, void *dst) {
-  const dim3 g(grid_for(c.n, kBlock, 8192));
-  if (c.fp64) {
-    auto kern = scatter ? k_permute<true, double4> : k_permute<false, double4>;
-    hipLaunchKernelGGL(kern, g, dim3(kBlock), 0, c.stream, c.n, idx,
-                       static_cast<const double4 *>(src), static_cast<double4 *>(dst));
-  } else {
-    auto kern = scatter ? k_permute<true, float4> : k_permute<false, float4>;
-    hipLaunchKernelGGL(kern, g, dim3(kBlock), 0, c.stream, c.n, idx,
-                       static_cast<const float4 *>(src), static_cast<float4 *>(dst));
-  }
+template <typename T>
+hipError_t permute_t(Ctx &c, bool scatter, const int *idx, const void *src, void *dst) {
+  return launch_checked(c, scatter ? k_permute<true, T> : k_permute<false, T>,
+                        dim3(grid_for(c.n, kBlock, 8192)), c.n, idx, static_cast<const T *>(src),
+                        static_cast<T *>(dst));
+}
+
+}  // namespace
+
+hipError_t launch_iota(Ctx &c, int n, int *out) {
+  return launch_checked(c, k_iota, dim3(grid_for(n, kBlock, 8192)), n, out);
+}
+
+hipError_t launch_permute(Ctx &c, bool scatter, const int *idx, const void *src, void *dst) {
+  return c.fp64 ? permute_t<double4>(c, scatter, idx, src, dst)
+                : permute_t<float4>(c, scatter, idx, src, dst);
 }
 
 void launch_clear_sticky(Ctx &c) {
