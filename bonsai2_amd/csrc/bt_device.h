@@ -194,29 +194,39 @@ __device__ __forceinline__ int system_of(int i, int nsys, const int *__restrict_
 // is cleared, in all of its pairs.  256: an evolving halo and disk of 2^24, whose box
 // grows with the particles that leave it, had a run of more than 64 in its 24th step, and
 // 8 digits instead of 5 from then on (sorts 1.53 -> 2.47 ms a step); looking through
-// longer runs costs its gathers 0.09 ms.  Most pairs have no neighbour in their run, so
-// the first kSingly keys on either side are read one by one; those past them eight at a
-// time, as the reads' latency is what a long run costs (2^22 particles in clumps of 120:
-// build 1.12 -> 0.92 ms, groups 0.93 -> 0.72; 2^20 in clumps of 250 0.51 -> 0.41 and 0.57
-// -> 0.36; ordinary systems: the tree's gather as before, the groups' 3% more).
+// longer runs costs its gathers 0.09 ms.  Most pairs have no neighbour in their run: the
+// nearest two are read together (2*10^7 ordinary particles: the tree's gather 364 -> 367 us,
+// the groups' 400 -> 390), up to kSingly on either side one by one, and those past them
+// eight at a time, as the reads' latency is what a long run costs (2^22 particles in clumps
+// of 120: build 1.11 -> 0.92 ms, groups 0.93 -> 0.72; 2^20 in clumps of 250 0.50 -> 0.41 and
+// 0.57 -> 0.37).
 constexpr int kRunMax = 256;
 __device__ __forceinline__ int place_in_run(int i, int lo, int hi, int low,
                                             const uint64_t *__restrict__ keys, uint64_t key,
                                             bool &ok) {
   constexpr int kSingly = 8, kAhead = 8;
   auto in_run = [&](uint64_t x) { return ((x ^ key) >> low) == 0; };
-  int place = i, before = 0, after = 0;
-  for (int k = i - 1; k >= lo; k--) {
-    const uint64_t x = keys[k];
-    if (!in_run(x)) break;
-    place -= x > key ? 1 : 0;
-    if (++before >= kSingly) break;
+  // the nearest two together; most pairs are done with that
+  const uint64_t prev = keys[max(i - 1, lo)], next = keys[min(i + 1, hi - 1)];
+  int before = i > lo && in_run(prev) ? 1 : 0, after = i + 1 < hi && in_run(next) ? 1 : 0;
+  int place = i;
+  if (before + after == 0) return place;
+  place += (after && next < key ? 1 : 0) - (before && prev > key ? 1 : 0);
+  if (before) {
+    for (int k = i - 2; k >= lo; k--) {
+      const uint64_t x = keys[k];
+      if (!in_run(x)) break;
+      place -= x > key ? 1 : 0;
+      if (++before >= kSingly) break;
+    }
   }
-  for (int k = i + 1; k < hi; k++) {
-    const uint64_t x = keys[k];
-    if (!in_run(x)) break;
-    place += x < key ? 1 : 0;
-    if (++after >= kSingly) break;
+  if (after) {
+    for (int k = i + 2; k < hi; k++) {
+      const uint64_t x = keys[k];
+      if (!in_run(x)) break;
+      place += x < key ? 1 : 0;
+      if (++after >= kSingly) break;
+    }
   }
   if (max(before, after) < kSingly) return place;
   if (before >= kSingly) {
